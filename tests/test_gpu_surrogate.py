@@ -151,6 +151,48 @@ def test_layers_and_gradients_match_bf16_oracle(vc, small):
     net.release()
 
 
+@pytest.mark.parametrize("shape", [(8, 8, 8), (16, 24, 40), (23, 9, 66), (96, 88, 8)])
+def test_weight_gradients_on_partial_and_chunked_bricks(vc, shape):
+    """The weight gradient's bricks are 4 x 4 x 32 voxels: levels with fewer
+    voxels than a brick along every axis, a second partly filled brick along z,
+    ragged axes, and more bricks than chunks (a workgroup walks several).
+    Against the BF16 variant of the oracle with the bounds of
+    test_layers_and_gradients_match_bf16_oracle; a dropped brick or a wrong
+    edge leaves its layer far outside them."""
+    from voxel_ma_amd import synth
+    rng = np.random.default_rng(sum(shape))
+    L = max(shape)
+    occ = np.zeros(shape, np.uint8)
+    while occ.sum() < 40:
+        o = synth.solids_host(L, synth.training_specs(L, rng)) if L <= 48 else \
+            (rng.random((L,) * 3) < 0.6).astype(np.uint8)
+        a = [(L - n) // 2 for n in shape]
+        occ = np.ascontiguousarray(o[a[0]:a[0] + shape[0], a[1]:a[1] + shape[1],
+                                     a[2]:a[2] + shape[2]])
+    occ[0, 0, 0] = 0
+    vol = vc.upload(occ)
+    vol.edt().measure()
+    th = _theta(5)
+    net = V.Surrogate(vc, seed=5)
+    net.set_params(th)
+    say("partial bricks", shape)
+    _, g = net.gradients(vol)
+    grow = [(0, (-n) % 8) for n in shape]
+    _, g_ref = U.gradients(th.astype(np.float64), np.pad(occ, grow),
+                           np.pad(vol.get(V.BUF_EDT), grow),
+                           np.pad(vol.get(V.BUF_LAM2), grow), bf16=True)
+    o = 0
+    for name, ci, co in U.LAYERS + [("head", 16, 2)]:
+        nw = (1 if name == "head" else 27) * ci * co
+        rw = _rel(g[o:o + nw].astype(np.float64), g_ref[o:o + nw])
+        rb = _rel(g[o + nw:o + nw + co].astype(np.float64), g_ref[o + nw:o + nw + co])
+        say("partial bricks", shape, name, round(rw, 5), round(rb, 5))
+        assert rw < 0.04 and rb < 0.04, (name, rw, rb)
+        o += nw + co
+    net.release()
+    vol.release()
+
+
 def test_training_lowers_loss(vc):
     """Adam on two volumes: the loss is noisy from step to step (it climbs
     for a while before it falls), so the mean of the last 10 of 60 steps is

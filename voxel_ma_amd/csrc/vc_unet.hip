@@ -601,191 +601,225 @@ __global__ void __launch_bounds__(kBlock)
         conv_store<NT, MT, BY, NZT, kRelu>(acc, out, bias, x0, y0, z0, X, Y, Z, box, off32);
 }
 
-// Weight gradient partials.  Block (chunk, tg): taps (dx, dy) = (tg/3 - 1,
-// tg%3 - 1), dz = -1, 0, 1; voxels [chunk * vbpc * 64, ...) in 64-voxel
-// blocks.  part[chunk][tap][ci][co] = sum_v x[v + off(tap)][ci] dzt[v][co].
-// MFMA rows = output channels (A = dzt^T), columns = (dz, 16 input
-// channels) (B = shifted x), K = 32 voxels.
-template <int RT, int CT>
-__global__ void __launch_bounds__(kBlock)
-    conv_wgrad(const bf16* __restrict__ x, int cinp,
-               const bf16* __restrict__ dzt, float* __restrict__ part, int X,
-               int Y, int Z, int64_t V, int vbpc)
+// Weight (and bias) gradient partials of one (output, input) pair of
+// 16-channel groups.  A workgroup walks its chunk of output bricks of 4 x 4
+// rows (x, y) by 32 voxels (z); wavefront w holds the 27 taps' 16 x 16
+// accumulators of the brick's rows x = w.  MFMA rows = output channels (A =
+// dz^T), columns = input channels (B = the shifted input), K = the 32 voxels
+// of a row, so an input row's three z shifts (3 B operands) feed the up to 9
+// (dy, dz) products of the output rows around it, and the wavefront's four
+// output rows (4 A operands) stay in registers for the whole brick: 0.54
+// operand reads per MFMA.
+//
+// The operands are channels-last in LDS and K runs over voxels, so they are
+// read with the transposing LDS load (16 lanes read 4 voxels x 16 channels
+// and lane i gets channel i of the 4); K slot 8 g + e is voxel 4 g + e (e < 4)
+// or 16 + 4 g + e - 4, which makes each load 512 contiguous bytes.  The next
+// brick's global loads are in flight during a brick's MFMAs.
+//
+// Bound: staging (2.4 x the brick's own input voxels with the halo, mostly L2
+// hits) and the MFMA chain are about even at two workgroups per CU.  The
+// earlier kernel (one workgroup per (dx, dy), 8 two-byte LDS reads per
+// operand) took 5.3 ms for the 14 layers of a 128^3 volume; this one takes
+// 0.66 ms, its reduction 0.09 ms (0.94 ms with one thread per sum).  The
+// bias gradient is one more product per output row (A times ones), which
+// replaces column-sum kernels (2.3 ms and their serial reduction 0.5 ms).
+// The partials of a chunk are summed over the four wavefronts in a fixed order.
+constexpr int kWgB = 4, kWgZ = 32;                  // brick rows (x and y), voxels
+constexpr int kWgR = kWgB + 2, kWgV = kWgZ + 2;     // region rows, voxels
+constexpr int kWgXU = kWgR * kWgR * kWgV * 2;       // 16-byte units of the region
+constexpr int kWgDU = kWgB * kWgB * kWgZ * 2;       // and of the brick's dz
+constexpr int kWgXN = (kWgXU + kBlock - 1) / kBlock, kWgDN = kWgDU / kBlock;
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+// the layer input of a weight gradient: channels below c1 from the coarse
+// level (nearest up-sampling of `up`, c1 channels), the rest from `sk` (c - c1
+// channels); c1 = 0 for a plain tensor of c channels
+struct WgIn
 {
-    constexpr int Cout = RT * 16, CP = CT * 16;
-    constexpr int SD = Cout + 2, SX = CP + 2; // LDS row strides (elements)
-    constexpr int NCOL = 3 * CT, CPW = (NCOL + 3) / 4;
-    __shared__ bf16 sdz[64 * SD];
-    __shared__ bf16 sx[66 * SX];
-    __shared__ int szc[64];
-    __shared__ int sok[64];
+    const bf16 *up, *sk;
+    int c1, c;
+};
+
+// 8 K slots of channel i of a row: two transposing reads at LDS element
+// offsets p and p + 16 voxels
+__device__ __forceinline__ bf16x8 wg_frag(const bf16* p)
+{
+    typedef __attribute__((address_space(3))) s16x4* lp;
+    union
+    {
+        s16x4 h[2];
+        bf16x8 v;
+    } u;
+    u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)p);
+    u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(p + 16 * 16));
+    return u.v;
+}
+
+__global__ void __launch_bounds__(kBlock, 2)
+    conv_wgrad(WgIn in, const bf16* __restrict__ dz, int cout, float* __restrict__ part,
+               float* __restrict__ part_b, int X, int Y, int Z, int nby, int nbz, int nb,
+               int bpc)
+{
+    __shared__ __attribute__((aligned(16))) bf16 sx[kWgXU * 8];
+    __shared__ __attribute__((aligned(16))) bf16 sd[kWgDU * 8];
+    static_assert(sizeof(float) * 27 * 256 <= sizeof(bf16) * kWgXU * 8, "the sums fit sx");
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int i = lane & 15, g = lane >> 4;
-    const int tg = blockIdx.y;
-    const int dx = tg / 3 - 1, dy = tg % 3 - 1;
-    const int64_t off = ((int64_t)dx * Y + dy) * Z;
-    f32x4 acc[RT][CPW];
+    const int ct = blockIdx.y % ((in.c + 15) / 16), rt = blockIdx.y / ((in.c + 15) / 16);
+    const bool coarse = ct * 16 < in.c1;
+    const bf16* src = coarse ? in.up + ct * 16 : in.sk + (ct * 16 - in.c1);
+    const int sc = coarse ? in.c1 : in.c - in.c1; // channels of a source voxel
+    const int nh = min(2, (in.c - ct * 16) / 8);  // 8-channel halves that exist
+    const bf16* dsrc = dz + rt * 16;
+    const bf16x8 zero8 = {};
+    bf16x8 xr[kWgXN], dr[kWgDN];
+    auto load = [&](int b) {
+        const int bz = b % nbz, r = b / nbz, by = r % nby, bx = r / nby;
+        const int x0 = bx * kWgB, y0 = by * kWgB, z0 = bz * kWgZ;
 #pragma unroll
-    for (int r = 0; r < RT; ++r)
+        for (int k = 0; k < kWgXN; ++k)
+        {
+            const int u = tid + k * kBlock;
+            const int row = u / (2 * kWgV), q = (u % (2 * kWgV)) >> 1, h = u & 1;
+            const int x = x0 - 1 + row / kWgR, y = y0 - 1 + row % kWgR, z = z0 - 1 + q;
+            const bool ok = u < kWgXU && h < nh && (unsigned)x < (unsigned)X &&
+                            (unsigned)y < (unsigned)Y && (unsigned)z < (unsigned)Z;
+            const int64_t v = coarse ? ((int64_t)(x >> 1) * (Y >> 1) + (y >> 1)) * (Z >> 1) +
+                                           (z >> 1)
+                                     : ((int64_t)x * Y + y) * Z + z;
+            xr[k] = zero8;
+            if (ok)
+                xr[k] = *reinterpret_cast<const bf16x8*>(src + v * sc + 8 * h);
+        }
 #pragma unroll
-        for (int c = 0; c < CPW; ++c)
-            acc[r][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const int64_t nvb = (V + 63) / 64;
-    const int64_t vb0 = (int64_t)blockIdx.x * vbpc;
-    for (int64_t vb = vb0; vb < vb0 + vbpc && vb < nvb; ++vb)
+        for (int k = 0; k < kWgDN; ++k)
+        {
+            const int u = tid + k * kBlock;
+            const int row = u / (2 * kWgZ), q = (u % (2 * kWgZ)) >> 1, h = u & 1;
+            const int x = x0 + row / kWgB, y = y0 + row % kWgB, z = z0 + q;
+            dr[k] = zero8;
+            if (x < X && y < Y && z < Z)
+                dr[k] = *reinterpret_cast<const bf16x8*>(
+                    dsrc + (((int64_t)x * Y + y) * Z + z) * cout + 8 * h);
+        }
+    };
+    f32x4 acc[27], accb = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int t = 0; t < 27; ++t)
+        acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    bf16x8 one8;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+        one8[e] = (bf16)1.0f;
+    const int b0 = (int)blockIdx.x * bpc, b1 = min(b0 + bpc, nb);
+    // this lane's place in a transposing read: voxel 4 g + i / 4, channels
+    // 4 (i % 4) .. + 3
+    const int lo = (4 * g + (i >> 2)) * 16 + 4 * (i & 3);
+    load(b0);
+    for (int b = b0; b < b1; ++b)
     {
-        const int64_t v0 = vb * 64;
-        // output gradient rows v0 .. v0+63, two channels per step
-        for (int idx = tid; idx < 64 * (Cout / 2); idx += kBlock)
-        {
-            const int row = idx / (Cout / 2), cp = idx % (Cout / 2);
-            uint32_t w = 0;
-            if (v0 + row < V)
-                w = *reinterpret_cast<const uint32_t*>(dzt + (v0 + row) * Cout +
-                                                       2 * cp);
-            *reinterpret_cast<uint32_t*>(sdz + row * SD + 2 * cp) = w;
-        }
-        // input rows s = v0 - 1 + r + off, r in [0, 66)
-        for (int idx = tid; idx < 66 * (CP / 2); idx += kBlock)
-        {
-            const int r = idx / (CP / 2), cp = idx % (CP / 2);
-            const int64_t s = v0 - 1 + r + off;
-            uint32_t w = 0;
-            if (s >= 0 && s < V && 2 * cp < cinp)
-                w = *reinterpret_cast<const uint32_t*>(x + s * cinp + 2 * cp);
-            *reinterpret_cast<uint32_t*>(sx + r * SX + 2 * cp) = w;
-        }
-        if (tid < 64)
-        {
-            const int64_t v = v0 + tid;
-            int ok = 0, zc = 0;
-            if (v < V)
-            {
-                zc = (int)(v % Z);
-                const int64_t t = v / Z;
-                const int yc = (int)(t % Y), xc = (int)(t / Y);
-                ok = (unsigned)(xc + dx) < (unsigned)X &&
-                     (unsigned)(yc + dy) < (unsigned)Y;
-            }
-            szc[tid] = zc;
-            sok[tid] = ok;
-        }
+        __syncthreads(); // the previous brick's reads are done
+#pragma unroll
+        for (int k = 0; k < kWgXN; ++k)
+            if (tid + k * kBlock < kWgXU)
+                *reinterpret_cast<bf16x8*>(sx + 8 * (tid + k * kBlock)) = xr[k];
+#pragma unroll
+        for (int k = 0; k < kWgDN; ++k)
+            *reinterpret_cast<bf16x8*>(sd + 8 * (tid + k * kBlock)) = dr[k];
         __syncthreads();
+        if (b + 1 < b1)
+            load(b + 1);
+        bf16x8 A[kWgB];
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-        {
-            const int k0 = kb * 32 + 8 * g;
-            bf16x8 A[RT];
+        for (int y = 0; y < kWgB; ++y)
+            A[y] = wg_frag(sd + (wv * kWgB + y) * kWgZ * 16 + lo);
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
+        for (int dx = 0; dx < 3; ++dx)
 #pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    A[rt][e] = sdz[(k0 + e) * SD + rt * 16 + i];
-            // validity of (voxel k0 + e, dz) as three 8-bit masks
-            uint32_t okm[3] = {0u, 0u, 0u};
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
+            for (int yy = 0; yy < kWgR; ++yy)
             {
-                const int zc = szc[k0 + e];
-                const bool ok = sok[k0 + e] != 0;
+                const bf16* row = sx + ((wv + dx) * kWgR + yy) * kWgV * 16 + lo;
 #pragma unroll
                 for (int d = 0; d < 3; ++d)
-                    okm[d] |= (uint32_t)(ok && (unsigned)(zc + d - 1) <
-                                                   (unsigned)Z)
-                              << e;
-            }
-#pragma unroll
-            for (int cw = 0; cw < CPW; ++cw)
-            {
-                const int col = wv + 4 * cw;
-                if (col < NCOL)
                 {
-                    const int d = col / CT, ct = col % CT;
-                    bf16x8 B;
+                    const bf16x8 B = wg_frag(row + d * 16);
 #pragma unroll
-                    for (int e = 0; e < 8; ++e)
+                    for (int dy = 0; dy < 3; ++dy)
                     {
-                        const bf16 val =
-                            sx[(k0 + e + d) * SX + ct * 16 + i];
-                        B[e] = ((okm[d] >> e) & 1u) ? val : (bf16)0.0f;
+                        const int y = yy - dy;
+                        if (y >= 0 && y < kWgB)
+                            acc[(dx * 3 + dy) * 3 + d] =
+                                __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                    A[y], B, acc[(dx * 3 + dy) * 3 + d], 0, 0, 0);
                     }
-#pragma unroll
-                    for (int rt = 0; rt < RT; ++rt)
-                        acc[rt][cw] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                            A[rt], B, acc[rt][cw], 0, 0, 0);
                 }
             }
-        }
+        if (ct == 0)
+#pragma unroll
+            for (int y = 0; y < kWgB; ++y)
+                accb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[y], one8, accb, 0, 0, 0);
+    }
+    // sum over the wavefronts, in order; lane holds output channels rt*16 +
+    // 4g + r of input channel ct*16 + i
+    f32x4* sum = reinterpret_cast<f32x4*>(sx);
+    f32x4* sumb = reinterpret_cast<f32x4*>(sd);
+    for (int w = 0; w < 4; ++w)
+    {
         __syncthreads();
-    }
-    // lane holds D[4g + r][i]: output channel rt*16 + 4g + r, input channel
-    // ct*16 + i
-#pragma unroll
-    for (int cw = 0; cw < CPW; ++cw)
-    {
-        const int col = wv + 4 * cw;
-        if (col >= NCOL)
-            continue;
-        const int d = col / CT, ct = col % CT;
-        const int tap = tg * 3 + d;
-        const int ci = ct * 16 + i;
-        if (ci >= cinp)
+        if (wv != w)
             continue;
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-            {
-                const int co = rt * 16 + 4 * g + r;
-                part[(((int64_t)blockIdx.x * 27 + tap) * cinp + ci) * Cout + co] =
-                    acc[rt][cw][r];
-            }
+        for (int t = 0; t < 27; ++t)
+        {
+            if (w > 0)
+                acc[t] = sum[t * 64 + lane] + acc[t];
+            if (w < 3)
+                sum[t * 64 + lane] = acc[t];
+            else if (ct * 16 + i < in.c)
+                *reinterpret_cast<f32x4*>(
+                    part + (((int64_t)blockIdx.x * 27 + t) * in.c + ct * 16 + i) * cout +
+                    rt * 16 + 4 * g) = acc[t];
+        }
+        if (ct == 0)
+        {
+            if (w > 0)
+                accb = sumb[lane] + accb;
+            if (w < 3)
+                sumb[lane] = accb;
+            else if (i == 0)
+                *reinterpret_cast<f32x4*>(part_b + (int64_t)blockIdx.x * cout + rt * 16 +
+                                          4 * g) = accb;
+        }
     }
 }
 
-// grad[(tap * cin + ci) * cout + co] += sum over chunks of the partials
+// grad += sum over chunks of the partials: 64 outputs per workgroup, the
+// chunks split over its four wavefronts (a fixed order).  Outputs are the
+// weights [tap][cin][cout] (of cinp input channels in the partials), then the
+// biases, from part_b.
 __global__ void __launch_bounds__(kBlock)
-    wgrad_reduce(const float* __restrict__ part, int nchunks, int cin,
-                 int cinp, int cout, float* __restrict__ grad)
+    wgrad_reduce(const float* __restrict__ part, const float* __restrict__ part_b, int nchunks,
+                 int cin, int cinp, int cout, float* __restrict__ grad)
 {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t n = 27LL * cin * cout;
-    if (t >= n)
-        return;
-    const int co = (int)(t % cout);
-    const int64_t r = t / cout;
-    const int ci = (int)(r % cin), tap = (int)(r / cin);
+    __shared__ float red[4][64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int t = blockIdx.x * 64 + lane, nw = 27 * cin * cout, n = nw + cout;
     float s = 0.0f;
-    for (int c = 0; c < nchunks; ++c)
-        s += part[(((int64_t)c * 27 + tap) * cinp + ci) * cout + co];
-    grad[t] += s;
-}
-
-// per-block column sums of a [V][C] BF16 tensor: part[block][c]
-__global__ void __launch_bounds__(kBlock)
-    colsum_part(const bf16* __restrict__ a, int C, int64_t V, int64_t vpb,
-                float* __restrict__ part)
-{
-    __shared__ float red[kBlock];
-    const int c = threadIdx.x % C;
-    const int lanes = kBlock / C; // threads per channel
-    const int j = threadIdx.x / C;
-    float s = 0.0f;
-    if (j < lanes)
+    if (t < n)
     {
-        const int64_t v0 = (int64_t)blockIdx.x * vpb;
-        for (int64_t v = v0 + j; v < v0 + vpb && v < V; v += lanes)
-            s += (float)a[v * C + c];
+        const int co = t % cout, r = t / cout, ci = r % cin, tap = r / cin;
+        const float* p = t < nw ? part + ((int64_t)tap * cinp + ci) * cout + co
+                                : part_b + (t - nw);
+        const int64_t step = t < nw ? 27LL * cinp * cout : cout;
+#pragma unroll 8
+        for (int c = wv; c < nchunks; c += 4)
+            s += p[c * step];
     }
-    red[threadIdx.x] = s;
+    red[wv][lane] = s;
     __syncthreads();
-    if (threadIdx.x < C)
-    {
-        float t = 0.0f;
-        for (int q = 0; q < lanes; ++q)
-            t += red[q * C + threadIdx.x];
-        part[(int64_t)blockIdx.x * C + threadIdx.x] = t;
-    }
+    if (wv == 0 && t < n)
+        grad[t] += (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
 }
 
 // dst[c] += sum_b part[b][c]
@@ -1619,6 +1653,27 @@ Box level_box(const vc_surrogate* s, int lv)
     return b;
 }
 
+// bricks of layer l's weight gradient and the chunks they are split into:
+// about two workgroups per CU over all channel-group pairs (the kernel's
+// occupancy), so that the partials stay small (at most 512 sums of 27 x 256)
+struct WgPlan
+{
+    int nby, nbz, nb, bpc, nchunks, pairs;
+};
+WgPlan wgrad_plan(const vc_surrogate* s, int l)
+{
+    const LayerSpec& L = kLayers[l];
+    WgPlan p;
+    p.nby = ((s->Y >> L.level) + kWgB - 1) / kWgB;
+    p.nbz = ((s->Z >> L.level) + kWgZ - 1) / kWgZ;
+    p.nb = ((s->X >> L.level) + kWgB - 1) / kWgB * p.nby * p.nbz;
+    p.pairs = (cinp_of(L.cin) + 15) / 16 * (L.cout / 16);
+    const int want = std::max(1, std::min(p.nb, 512 / p.pairs));
+    p.bpc = (p.nb + want - 1) / want;
+    p.nchunks = (p.nb + p.bpc - 1) / p.bpc;
+    return p;
+}
+
 int ensure_ws(vc_ctx* ctx, vc_surrogate* s, int X, int Y, int Z, bool bw)
 {
     if (s->X != X || s->Y != Y || s->Z != Z)
@@ -1666,13 +1721,12 @@ int ensure_ws(vc_ctx* ctx, vc_surrogate* s, int X, int Y, int Z, bool bw)
         if ((rc = ws_alloc(ctx, s, (void**)&s->dout,
                            8 * (size_t)level_voxels(s, 0))) != VC_OK)
             return rc;
-        // partials: weight gradients (chunks x 27 x cinp x cout, at most 256
-        // chunks) and column / loss sums
+        // partials: weight and bias gradients, and loss / head sums
         size_t pf = 0;
         for (int l = 0; l < 14; ++l)
         {
-            const size_t f = 256ull * 27 * cinp_of(kLayers[l].cin) *
-                             kLayers[l].cout;
+            const size_t f = (size_t)wgrad_plan(s, l).nchunks *
+                             (27ull * cinp_of(kLayers[l].cin) + 1) * kLayers[l].cout;
             pf = f > pf ? f : pf;
         }
         const size_t cs = (size_t)(level_voxels(s, 0) / kBlock + 1) * 64;
@@ -1775,49 +1829,21 @@ int launch_conv(vc_ctx* ctx, const bf16* in, int cinp, bf16* out, int cout,
     return VC_OK;
 }
 
-template <int RT, int CT>
-void launch_wgrad_t(hipStream_t S, const bf16* x, int cinp, const bf16* dz,
-                    float* part, int X, int Y, int Z, int nchunks, int vbpc)
-{
-    const int64_t V = (int64_t)X * Y * Z;
-    conv_wgrad<RT, CT><<<dim3((unsigned)nchunks, 9), kBlock, 0, S>>>(
-        x, cinp, dz, part, X, Y, Z, V, vbpc);
-}
-
-// layer l: gradient of W (and b) from its input x and pre-activation
-// gradient dz, accumulated into s->grad
-int layer_wgrad(vc_ctx* ctx, vc_surrogate* s, int l, const bf16* x,
-                const bf16* dz)
+// layer l: gradient of W and b from its input and pre-activation gradient
+// dz, accumulated into s->grad
+int layer_wgrad(vc_ctx* ctx, vc_surrogate* s, int l, const WgIn& in, const bf16* dz)
 {
     const LayerSpec& L = kLayers[l];
-    const int X = s->X >> L.level, Y = s->Y >> L.level, Z = s->Z >> L.level;
-    const int64_t V = (int64_t)X * Y * Z;
-    const int cinp = cinp_of(L.cin);
-    const int64_t nvb = (V + 63) / 64;
-    const int nchunks = (int)(nvb < 256 ? nvb : 256);
-    const int vbpc = (int)((nvb + nchunks - 1) / nchunks);
+    const WgPlan p = wgrad_plan(s, l);
     hipStream_t S = ctx->stream;
-    const int RT = L.cout / 16, CT = (cinp + 15) / 16;
-#define VC_WG(r, c)                                                            \
-    if (RT == r && CT == c)                                                    \
-        launch_wgrad_t<r, c>(S, x, cinp, dz, s->part, X, Y, Z, nchunks, vbpc); \
-    else
-    VC_WG(1, 1) VC_WG(2, 1) VC_WG(2, 2) VC_WG(3, 2) VC_WG(3, 3) VC_WG(4, 3)
-    VC_WG(4, 4) VC_WG(3, 7) VC_WG(2, 5) VC_WG(1, 3)
-    return vc_fail(ctx, VC_ERR_INVALID, "wgrad: no kernel for %d x %d", RT, CT);
-#undef VC_WG
+    float* part_b = s->part + (int64_t)p.nchunks * 27 * in.c * L.cout;
+    conv_wgrad<<<dim3((unsigned)p.nchunks, (unsigned)p.pairs), kBlock, 0, S>>>(
+        in, dz, L.cout, s->part, part_b, s->X >> L.level, s->Y >> L.level, s->Z >> L.level,
+        p.nby, p.nbz, p.nb, p.bpc);
     VC_CHECK_LAUNCH(ctx);
-    float* gW = s->grad + param_offset(l);
-    const int64_t nw = 27LL * L.cin * L.cout;
-    wgrad_reduce<<<blocks_for(nw), kBlock, 0, S>>>(s->part, nchunks, L.cin,
-                                                    cinp, L.cout, gW);
-    VC_CHECK_LAUNCH(ctx);
-    // bias: column sums of dz
-    const int64_t vpb = 4096;
-    const int nb = (int)((V + vpb - 1) / vpb);
-    colsum_part<<<nb, kBlock, 0, S>>>(dz, L.cout, V, vpb, s->part);
-    VC_CHECK_LAUNCH(ctx);
-    colsum_reduce<<<1, 64, 0, S>>>(s->part, nb, L.cout, gW + nw);
+    const int n = 27 * L.cin * L.cout + L.cout;
+    wgrad_reduce<<<(n + 63) / 64, kBlock, 0, S>>>(s->part, part_b, p.nchunks, L.cin, in.c,
+                                                   L.cout, s->grad + param_offset(l));
     VC_CHECK_LAUNCH(ctx);
     return VC_OK;
 }
@@ -1960,7 +1986,7 @@ int layer_back(vc_ctx* ctx, vc_surrogate* s, int l, bf16* gy, const bf16* x,
     relu_mask<<<grid_for(V * L.cout), kBlock, 0, S>>>(gy, s->act[l],
                                                          V * L.cout);
     VC_CHECK_LAUNCH(ctx);
-    int rc = layer_wgrad(ctx, s, l, x, gy);
+    int rc = layer_wgrad(ctx, s, l, WgIn{nullptr, x, 0, cinp_of(L.cin)}, gy);
     if (rc != VC_OK || !gx)
         return rc;
     return launch_conv(ctx, gy, L.cout, gx, cinp_of(L.cin), s->Wd[l], nullptr,
