@@ -822,17 +822,46 @@ __global__ void __launch_bounds__(kBlock)
         grad[t] += (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
 }
 
-// dst[c] += sum_b part[b][c]
-__global__ void colsum_reduce(const float* __restrict__ part, int nb, int C,
-                              float* __restrict__ dst)
+// dst[c] += sum of part[c][0 .. nb), in order (one workgroup per column c).
+// The order fixes the gradient's bits, so one thread adds; what it waited on
+// when it also loaded (0.2 us a value: 1.76 ms for the 8192 partials of a
+// 128^3 volume) was memory, so the workgroup stages the values in LDS first
+// and the chain runs at the adder's latency (52 us).
+constexpr int kSumStage = 4096;
+__global__ void __launch_bounds__(kBlock)
+    colsum_reduce(const float* __restrict__ part, int nb, float* __restrict__ dst)
 {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= C)
-        return;
+    __shared__ __attribute__((aligned(16))) float st[kSumStage];
+    const float* p = part + (int64_t)blockIdx.x * nb;
     float s = 0.0f;
-    for (int b = 0; b < nb; ++b)
-        s += part[(int64_t)b * C + c];
-    dst[c] += s;
+    for (int b0 = 0; b0 < nb; b0 += kSumStage)
+    {
+        const int n = min(kSumStage, nb - b0);
+        __syncthreads();
+        for (int b = threadIdx.x; b < n; b += kBlock)
+            st[b] = p[b0 + b];
+        __syncthreads();
+        if (threadIdx.x == 0)
+        {
+            int b = 0;
+            for (; b + 16 <= n; b += 16)
+            {
+                f32x4 v[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    v[q] = reinterpret_cast<const f32x4*>(st + b)[q];
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        s += v[q][e];
+            }
+            for (; b < n; ++b)
+                s += st[b];
+        }
+    }
+    if (threadIdx.x == 0)
+        dst[blockIdx.x] += s;
 }
 
 // ------------------------------------------------------------ elementwise
@@ -1080,8 +1109,38 @@ __global__ void __launch_bounds__(kBlock)
         part[blockIdx.x] = red[0];
 }
 
+// Sums of N values over the wavefront, each the butterfly's tree (x + x of
+// lane ^ 32, then ^ 16, ...), but with the values dealt out as the lanes
+// halve: at each step a lane passes on the half of its values that the other
+// lane keeps, so 34 values take 37 exchanges instead of 6 x 34.  The sum a
+// lane ends with is in val[0]; returns its index, or -1 for a lane left with
+// none.
+template <int N, int D, int M>
+__device__ __forceinline__ int wave_sums(float (&val)[M], int lane)
+{
+    if constexpr (D == 0)
+        return 0;
+    else
+    {
+        constexpr int H = (N + 1) / 2;
+        const bool up = (lane & D) != 0;
+#pragma unroll
+        for (int p = 0; p < H; ++p)
+        {
+            const float a = val[p], b = p + H < N ? val[p + H] : 0.0f;
+            val[p] = (up ? b : a) + __shfl_xor(up ? a : b, D);
+        }
+        const int r = wave_sums<H, D / 2>(val, lane);
+        if (r < 0)
+            return -1;
+        return up ? (r + H < N ? r + H : -1) : r;
+    }
+}
+
 // head backward: gd0[v][c] = sum_o dout[v][o] Wh[c][o]; per-block partials
-// of dWh[c][o] (32 values) and dbh[o] (2) in part[block][34]
+// of dWh[c][o] (32 values) and dbh[o] (2) in part[34][block].  112 us for a
+// 128^3 volume with a butterfly per value, 27 us with wave_sums
+// and 16-byte loads and stores of the two tensors.
 __global__ void __launch_bounds__(kBlock)
     head_bwd(const bf16* __restrict__ d0, const float* __restrict__ dout,
              const float* __restrict__ Wh, bf16* __restrict__ gd0, int64_t V,
@@ -1092,38 +1151,40 @@ __global__ void __launch_bounds__(kBlock)
     const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     float g0 = 0.0f, g1 = 0.0f;
     float h[kHeadIn];
+    bf16x8 hv[2] = {};
     if (v < V)
     {
-        g0 = dout[2 * v];
-        g1 = dout[2 * v + 1];
+        const float2 d = reinterpret_cast<const float2*>(dout)[v];
+        g0 = d.x;
+        g1 = d.y;
+        hv[0] = reinterpret_cast<const bf16x8*>(d0)[2 * v];
+        hv[1] = reinterpret_cast<const bf16x8*>(d0)[2 * v + 1];
+        bf16x8 o[2];
+#pragma unroll
+        for (int c = 0; c < kHeadIn; ++c)
+            o[c >> 3][c & 7] = (bf16)(g0 * Wh[c * 2] + g1 * Wh[c * 2 + 1]);
+        reinterpret_cast<bf16x8*>(gd0)[2 * v] = o[0];
+        reinterpret_cast<bf16x8*>(gd0)[2 * v + 1] = o[1];
     }
 #pragma unroll
     for (int c = 0; c < kHeadIn; ++c)
-    {
-        h[c] = v < V ? (float)d0[v * kHeadIn + c] : 0.0f;
-        if (v < V)
-            gd0[v * kHeadIn + c] = (bf16)(g0 * Wh[c * 2] + g1 * Wh[c * 2 + 1]);
-    }
+        h[c] = (float)hv[c >> 3][c & 7];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    float val[NP];
 #pragma unroll
     for (int p = 0; p < NP; ++p)
-    {
-        float val = p < kHeadIn * kHeadOut
-                        ? h[p >> 1] * ((p & 1) ? g1 : g0)
-                        : ((p - kHeadIn * kHeadOut) ? g1 : g0);
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1)
-            val += __shfl_xor(val, d);
-        if (lane == 0)
-            red[p][wv] = val;
-    }
+        val[p] = p < kHeadIn * kHeadOut ? h[p >> 1] * ((p & 1) ? g1 : g0)
+                                        : ((p - kHeadIn * kHeadOut) ? g1 : g0);
+    const int p = wave_sums<NP, 32>(val, lane);
+    if (p >= 0)
+        red[p][wv] = val[0];
     __syncthreads();
     if (threadIdx.x < NP)
     {
         float s = 0.0f;
         for (int w = 0; w < kBlock / 64; ++w)
             s += red[threadIdx.x][w];
-        part[(int64_t)blockIdx.x * NP + threadIdx.x] = s;
+        part[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = s;
     }
 }
 
@@ -1993,16 +2054,30 @@ int layer_back(vc_ctx* ctx, vc_surrogate* s, int l, bf16* gy, const bf16* x,
                        X, Y, Z, s->kcd[l], 0, level_box(s, L.level));
 }
 
-// inside voxels, one add per workgroup (a capped grid strides over them)
+// inside voxels: 16 per load, one add per workgroup of a grid of at most one
+// workgroup per CU (an add per 256 voxels had made the adds on one address
+// the kernel's time: 38 us for a 128^3 volume, below 9 us now)
 __global__ void __launch_bounds__(kBlock)
     count_occ(const uint8_t* __restrict__ occ, int64_t N,
               unsigned long long* __restrict__ cnt)
 {
     __shared__ unsigned long long sh[kBlock / 64];
     unsigned long long c = 0;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < N;
-         i += (int64_t)gridDim.x * blockDim.x)
-        c += occ[i] != 0;
+    const int64_t n16 = N / 16;
+    VC_GRID_STRIDE(t, n16)
+    {
+        const uint4 v = reinterpret_cast<const uint4*>(occ)[t];
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+        {
+            // bit 7 of each byte that is not zero
+            const uint32_t m = ((w[k] & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | w[k];
+            c += __popc(m & 0x80808080u);
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x < (N & 15))
+        c += occ[n16 * 16 + threadIdx.x] != 0;
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1)
         c += __shfl_xor(c, d);
@@ -2053,7 +2128,8 @@ int backward(vc_ctx* ctx, vc_surrogate* s, const vc_vol* v, float* loss_dev,
     const int64_t V0 = level_voxels(s, 0);
     const unsigned nb = blocks_for(V0);
     VC_HIP(ctx, hipMemsetAsync(cnt, 0, 8, S));
-    count_occ<<<(unsigned)std::min<int64_t>(blocks_for(v->N), 4096), kBlock, 0, S>>>(
+    count_occ<<<(unsigned)std::min<int64_t>(blocks_for(v->N / 16 + 1), ctx->cu_count), kBlock, 0,
+                S>>>(
         v->occ, v->N, cnt);
     VC_CHECK_LAUNCH(ctx);
     loss_bwd<<<nb, kBlock, 0, S>>>(s->out, v->occ, v->lam2, v->nx, v->ny,
@@ -2067,8 +2143,7 @@ int backward(vc_ctx* ctx, vc_surrogate* s, const vc_vol* v, float* loss_dev,
                                     s->theta + param_offset(14), s->gact[13],
                                     V0, s->part);
     VC_CHECK_LAUNCH(ctx);
-    colsum_reduce<<<1, 64, 0, S>>>(s->part, (int)nb, NP,
-                                    s->grad + param_offset(14));
+    colsum_reduce<<<NP, kBlock, 0, S>>>(s->part, (int)nb, s->grad + param_offset(14));
     VC_CHECK_LAUNCH(ctx);
     int rc;
     auto dims = [&](int lv, int& X, int& Y, int& Z) {
