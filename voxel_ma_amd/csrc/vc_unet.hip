@@ -310,14 +310,17 @@ __device__ __forceinline__ void conv_slice_coarse(const bf16x8* __restrict__ reg
 
 // Bias, ReLU and the zeroing outside the padded volume for one wavefront's
 // MT tiles: lane (i, g) holds channels n 16 + 4 g .. + 3 of voxel i.  With
-// off32 the output offsets from the brick's first voxel fit 31 bits.
+// off32 the output offsets from the brick's first voxel fit 31 bits.  An
+// input gradient (kRelu false) is stored already masked by the ReLU of the
+// layer it belongs to: `mask` (when given) holds that layer's activations,
+// and where they are not positive the gradient is 0.
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 template <int NT, int MT, int BY, int NZT, bool kRelu>
 __device__ __forceinline__ void conv_store(const f32x4 (&acc)[MT][NT], bf16* __restrict__ out,
                                            const float* __restrict__ bias, int x0, int y0,
                                            int z0, int X, int Y, int Z, const Box& box,
-                                           int off32)
+                                           int off32, const bf16* __restrict__ mask = nullptr)
 {
     constexpr int Cout = NT * 16;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -328,7 +331,9 @@ __device__ __forceinline__ void conv_store(const f32x4 (&acc)[MT][NT], bf16* __r
 #pragma unroll
         for (int r = 0; r < 4; ++r)
             bv[n][r] = bias ? bias[n * 16 + 4 * g + r] : 0.0f;
-    bf16* ob = out + (((int64_t)x0 * Y + y0) * Z + z0) * Cout + 4 * g;
+    const int64_t o0 = (((int64_t)x0 * Y + y0) * Z + z0) * Cout + 4 * g;
+    bf16* ob = out + o0;
+    const bf16* mb = mask ? mask + o0 : nullptr;
 #pragma unroll
     for (int m = 0; m < MT; ++m)
     {
@@ -341,10 +346,18 @@ __device__ __forceinline__ void conv_store(const f32x4 (&acc)[MT][NT], bf16* __r
                            (unsigned)(box.oz + z) < (unsigned)box.pz;
         const int lo = ((row / BY) * Y + row % BY) * Z + 16 * seg + i;
         bf16* o = off32 ? ob + lo * Cout : ob + (int64_t)lo * Cout;
+        const bf16* k = off32 ? mb + lo * Cout : mb + (int64_t)lo * Cout;
 #pragma unroll
         for (int n = 0; n < NT; ++n)
         {
             f32x4 val = acc[m][n] + bv[n];
+            if (!kRelu && mask)
+            {
+                const bf16x4 y = *reinterpret_cast<const bf16x4*>(k + n * 16);
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    val[r] = (float)y[r] > 0.0f ? val[r] : 0.0f;
+            }
             if (kRelu)
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
@@ -537,7 +550,7 @@ __global__ void __launch_bounds__(kBlock)
                  int cinp, bf16* __restrict__ out, const bf16x8* __restrict__ W,
                  const float* __restrict__ bias, int X, int Y, int Z, Box box, int off32,
                  const float* __restrict__ Wh = nullptr, float* __restrict__ hout = nullptr,
-                 CoreOut core = CoreOut{})
+                 CoreOut core = CoreOut{}, const bf16* __restrict__ mask = nullptr)
 {
     constexpr int Cout = NT * 16;
     constexpr int MT = BX * BY * NZT / 4;
@@ -598,7 +611,8 @@ __global__ void __launch_bounds__(kBlock)
     if constexpr (kHead)
         conv_store_head<MT, BY, NZT>(acc, bias, Wh, hout, x0, y0, z0, X, Y, Z, box, core);
     else
-        conv_store<NT, MT, BY, NZT, kRelu>(acc, out, bias, x0, y0, z0, X, Y, Z, box, off32);
+        conv_store<NT, MT, BY, NZT, kRelu>(acc, out, bias, x0, y0, z0, X, Y, Z, box, off32,
+                                           mask);
 }
 
 // Weight (and bias) gradient partials of one (output, input) pair of
@@ -872,23 +886,6 @@ __global__ void __launch_bounds__(kBlock)
 #define VC_GRID_STRIDE(t, n)                                                  \
     for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < (n); \
          t += (int64_t)gridDim.x * blockDim.x)
-__global__ void __launch_bounds__(kBlock)
-    relu_mask(bf16* __restrict__ g, const bf16* __restrict__ y, int64_t n)
-{
-    VC_GRID_STRIDE(t, n)
-    if (!((float)y[t] > 0.0f))
-        g[t] = (bf16)0.0f;
-}
-
-// child voxel (x, y, z) of level dims (X, Y, Z) -> parent at (X/2, Y/2, Z/2)
-__device__ __forceinline__ int64_t parent_of(int64_t v, int X, int Y, int Z)
-{
-    const int z = (int)(v % Z);
-    const int64_t r = v / Z;
-    const int y = (int)(r % Y), x = (int)(r / Y);
-    return (((int64_t)(x >> 1) * (Y >> 1)) + (y >> 1)) * (Z >> 1) + (z >> 1);
-}
-
 // p[parent][c] = mean of the 8 children (dims of the child level X, Y, Z)
 __global__ void __launch_bounds__(kBlock)
     pool_fwd(const bf16* __restrict__ a, bf16* __restrict__ p, int C, int X,
@@ -929,75 +926,79 @@ __global__ void __launch_bounds__(kBlock)
     }
 }
 
-// g_child += g_parent / 8
-__global__ void __launch_bounds__(kBlock)
-    pool_bwd_acc(bf16* __restrict__ ga, const bf16* __restrict__ gp, int C,
-                 int X, int Y, int Z)
+// 0 where the layer's activation is not positive (its ReLU)
+__device__ __forceinline__ bf16x8 relu_masked(const bf16x8& g, const bf16x8& y)
 {
-    const int64_t n = (int64_t)X * Y * Z * C;
-    VC_GRID_STRIDE(t, n)
+    bf16x8 o;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        o[k] = (float)y[k] > 0.0f ? g[k] : (bf16)0.0f;
+    return o;
+}
+
+// Gradient of a level's skip tensor (the second encoder convolution's output
+// y): g[v][c] = mask(g_cat[v][C1 + c] + g_pool[parent(v)][c] / 8), the
+// decoder concatenation's part plus the pooling's.  One thread per 8
+// channels (C2 is a multiple of 8) with 16-byte accesses: split, pooling and
+// mask as three kernels of one channel per thread took 0.37 ms for a 128^3
+// volume, 0.08 ms together.
+__global__ void __launch_bounds__(kBlock)
+    skip_grad(const bf16* __restrict__ gcat, int C, int C1, const bf16* __restrict__ gp,
+              const bf16* __restrict__ y, bf16* __restrict__ g, int X, int Y, int Z)
+{
+    const int C2 = C - C1, C8 = C2 >> 3;
+    VC_GRID_STRIDE(t, (int64_t)X * Y * Z * C8)
     {
-        const int c = (int)(t % C);
-        const int64_t v = t / C;
-        const int64_t pv = parent_of(v, X, Y, Z);
-        ga[t] = (bf16)((float)ga[t] + 0.125f * (float)gp[pv * C + c]);
+        const int c = 8 * (int)(t % C8);
+        const int64_t v = t / C8;
+        const int vz = (int)(v % Z);
+        const int64_t r = v / Z;
+        const int vy = (int)(r % Y), vx = (int)(r / Y);
+        const int64_t pv = ((int64_t)(vx >> 1) * (Y >> 1) + (vy >> 1)) * (Z >> 1) + (vz >> 1);
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(gcat + v * C + C1 + c);
+        const bf16x8 b = *reinterpret_cast<const bf16x8*>(gp + pv * C2 + c);
+        const bf16x8 yv = *reinterpret_cast<const bf16x8*>(y + v * C2 + c);
+        bf16x8 o;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            o[k] = (bf16)((float)a[k] + 0.125f * (float)b[k]);
+        *reinterpret_cast<bf16x8*>(g + v * C2 + c) = relu_masked(o, yv);
     }
 }
 
-// cat[v] = [up[parent(v)] (C1 channels), skip[v] (C2)] at child dims
+// Gradient of a decoder level's up-sampled input (the coarse level's output
+// y): g_up[parent][c] = mask(sum over the 8 children of g_cat[child][c]), c <
+// C1, the children in the cell order.  8 channels per thread.
 __global__ void __launch_bounds__(kBlock)
-    concat_fwd(const bf16* __restrict__ up, int C1, const bf16* __restrict__ sk,
-               int C2, bf16* __restrict__ cat, int X, int Y, int Z)
-{
-    const int C = C1 + C2;
-    const int64_t n = (int64_t)X * Y * Z * C;
-    VC_GRID_STRIDE(t, n)
-    {
-        const int c = (int)(t % C);
-        const int64_t v = t / C;
-        cat[t] = c < C1 ? up[parent_of(v, X, Y, Z) * C1 + c]
-                        : sk[v * C2 + (c - C1)];
-    }
-}
-
-// g_up[parent][c] = sum over the 8 children of g_cat[child][c] (c < C1)
-__global__ void __launch_bounds__(kBlock)
-    split_up(const bf16* __restrict__ gcat, int C, int C1,
+    split_up(const bf16* __restrict__ gcat, int C, int C1, const bf16* __restrict__ yup,
              bf16* __restrict__ gup, int X, int Y, int Z)
 {
-    const int Xp = X >> 1, Yp = Y >> 1, Zp = Z >> 1;
-    const int64_t n = (int64_t)Xp * Yp * Zp * C1;
-    VC_GRID_STRIDE(t, n)
+    const int Xp = X >> 1, Yp = Y >> 1, Zp = Z >> 1, C8 = C1 >> 3;
+    VC_GRID_STRIDE(t, (int64_t)Xp * Yp * Zp * C8)
     {
-        const int c = (int)(t % C1);
-        const int64_t v = t / C1;
+        const int c = 8 * (int)(t % C8);
+        const int64_t v = t / C8;
         const int z = (int)(v % Zp);
         const int64_t r = v / Zp;
         const int y = (int)(r % Yp), x = (int)(r / Yp);
-        float s = 0.0f;
+        float s[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int q = 0; q < 8; ++q)
         {
             const int64_t cv =
                 (((int64_t)(2 * x + (q >> 2)) * Y) + (2 * y + ((q >> 1) & 1))) * Z +
                 (2 * z + (q & 1));
-            s += (float)gcat[cv * C + c];
+            const bf16x8 w = *reinterpret_cast<const bf16x8*>(gcat + cv * C + c);
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                s[k] += (float)w[k];
         }
-        gup[t] = (bf16)s;
-    }
-}
-
-// g_skip[v][c] = g_cat[v][C1 + c]
-__global__ void __launch_bounds__(kBlock)
-    split_skip(const bf16* __restrict__ gcat, int C, int C1,
-               bf16* __restrict__ gsk, int64_t V)
-{
-    const int C2 = C - C1;
-    VC_GRID_STRIDE(t, V * C2)
-    {
-        const int c = (int)(t % C2);
-        const int64_t v = t / C2;
-        gsk[t] = gcat[v * C + C1 + c];
+        bf16x8 o;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            o[k] = (bf16)s[k];
+        *reinterpret_cast<bf16x8*>(gup + v * C1 + c) =
+            relu_masked(o, *reinterpret_cast<const bf16x8*>(yup + v * C1 + c));
     }
 }
 
@@ -1137,7 +1138,8 @@ __device__ __forceinline__ int wave_sums(float (&val)[M], int lane)
     }
 }
 
-// head backward: gd0[v][c] = sum_o dout[v][o] Wh[c][o]; per-block partials
+// head backward: gd0[v][c] = sum_o dout[v][o] Wh[c][o] masked by the ReLU of
+// d0 (the last layer's activations); per-block partials
 // of dWh[c][o] (32 values) and dbh[o] (2) in part[34][block].  112 us for a
 // 128^3 volume with a butterfly per value, 27 us with wave_sums
 // and 16-byte loads and stores of the two tensors.
@@ -1163,8 +1165,8 @@ __global__ void __launch_bounds__(kBlock)
 #pragma unroll
         for (int c = 0; c < kHeadIn; ++c)
             o[c >> 3][c & 7] = (bf16)(g0 * Wh[c * 2] + g1 * Wh[c * 2 + 1]);
-        reinterpret_cast<bf16x8*>(gd0)[2 * v] = o[0];
-        reinterpret_cast<bf16x8*>(gd0)[2 * v + 1] = o[1];
+        reinterpret_cast<bf16x8*>(gd0)[2 * v] = relu_masked(o[0], hv[0]);
+        reinterpret_cast<bf16x8*>(gd0)[2 * v + 1] = relu_masked(o[1], hv[1]);
     }
 #pragma unroll
     for (int c = 0; c < kHeadIn; ++c)
@@ -1645,7 +1647,6 @@ struct vc_surrogate
     int inf_n[3] = {0, 0, 0};
     // and where its head writes the core voxels' lam / rel (no copy_core)
     CoreOut inf_core{};
-    bf16 *cat2 = nullptr, *cat1 = nullptr, *cat0 = nullptr;
     float* out = nullptr;
     // backward workspace (allocated on first use)
     bool bw = false;
@@ -1679,7 +1680,7 @@ void free_ws(vc_surrogate* s)
         s->act[l] = nullptr;
         s->gact[l] = nullptr;
     }
-    s->x0 = s->x8 = s->p1 = s->p2 = s->p3 = s->cat2 = s->cat1 = s->cat0 = nullptr;
+    s->x0 = s->x8 = s->p1 = s->p2 = s->p3 = nullptr;
     s->gcat2 = s->gcat1 = s->gcat0 = s->gp1 = s->gp2 = s->gp3 = nullptr;
     s->out = s->dout = s->part = nullptr;
     s->part_floats = 0;
@@ -1756,8 +1757,7 @@ int ensure_ws(vc_ctx* ctx, vc_surrogate* s, int X, int Y, int Z, bool bw)
                 VC_OK)
                 return rc;
         if ((rc = A(&s->p1, 1, 16)) != VC_OK || (rc = A(&s->p2, 2, 32)) != VC_OK ||
-            (rc = A(&s->p3, 3, 48)) != VC_OK || (rc = A(&s->cat2, 2, 112)) != VC_OK ||
-            (rc = A(&s->cat1, 1, 80)) != VC_OK || (rc = A(&s->cat0, 0, 48)) != VC_OK)
+            (rc = A(&s->p3, 3, 48)) != VC_OK)
             return rc;
         if ((rc = ws_alloc(ctx, s, (void**)&s->out,
                            8 * (size_t)level_voxels(s, 0))) != VC_OK)
@@ -1840,21 +1840,23 @@ int conv_off32(int Y, int Z, int cmax)
 template <int NT, bool kCat, bool kRelu>
 void launch_conv_t(hipStream_t S, const bf16* in, const bf16* in2, int c1, int cinp,
                    bf16* out, const bf16* W, const float* bias, int X, int Y, int Z,
-                   const Box& box)
+                   const Box& box, const bf16* mask)
 {
     const int64_t nb = (int64_t)((X + kCBX - 1) / kCBX) * ((Y + kCBY - 1) / kCBY) *
                        ((Z + 16 * kCNZT - 1) / (16 * kCNZT));
     conv_fwd_lds<NT, kCBX, kCBY, kCNZT, kCSC, kCat, kRelu><<<conv_grid(nb), kBlock, 0, S>>>(
         in, in2, c1, cinp, out, reinterpret_cast<const bf16x8*>(W), bias, X, Y, Z, box,
-        conv_off32(Y, Z, std::max(cinp, NT * 16)));
+        conv_off32(Y, Z, std::max(cinp, NT * 16)), nullptr, nullptr, CoreOut{}, mask);
 }
 
 // box: the region's origin and the padded-volume extent at this level.  With
 // in2 the input is the concatenation [in (coarse level, c1 channels,
-// upsampled) | in2 (cinp - c1 channels)].
+// upsampled) | in2 (cinp - c1 channels)].  mask: conv_store's, for an input
+// gradient.
 int launch_conv(vc_ctx* ctx, const bf16* in, int cinp, bf16* out, int cout,
                 const bf16* W, const float* bias, int X, int Y, int Z, int kc,
-                int relu, const Box& b, const bf16* in2 = nullptr, int c1 = 0)
+                int relu, const Box& b, const bf16* in2 = nullptr, int c1 = 0,
+                const bf16* mask = nullptr)
 {
     hipStream_t S = ctx->stream;
     (void)kc;
@@ -1866,13 +1868,14 @@ int launch_conv(vc_ctx* ctx, const bf16* in, int cinp, bf16* out, int cout,
 #define VC_CONV_CASE(nt)                                                              \
     case nt:                                                                          \
         if (in2)                                                                      \
-            launch_conv_t<nt, true, true>(S, in, in2, c1, cinp, out, W, bias, X, Y, Z, b); \
+            launch_conv_t<nt, true, true>(S, in, in2, c1, cinp, out, W, bias, X, Y, Z, b, \
+                                          nullptr);                                   \
         else if (relu)                                                                \
             launch_conv_t<nt, false, true>(S, in, nullptr, 0, cinp, out, W, bias, X, Y, Z, \
-                                           b);                                        \
+                                           b, nullptr);                               \
         else                                                                          \
             launch_conv_t<nt, false, false>(S, in, nullptr, 0, cinp, out, W, bias, X, Y, \
-                                            Z, b);                                    \
+                                            Z, b, mask);                              \
         break;
     switch (cout / 16)
     {
@@ -1909,16 +1912,16 @@ int layer_wgrad(vc_ctx* ctx, vc_surrogate* s, int l, const WgIn& in, const bf16*
     return VC_OK;
 }
 
-// forward over the current workspace region (input x0 filled); keep_cat
-// materializes the decoder's concatenated inputs (the weight gradients read
-// them), otherwise the first decoder convolution of a level reads the coarse
-// level and the skip tensor directly
-int forward(vc_ctx* ctx, vc_surrogate* s, bool keep_cat)
+// forward over the current workspace region (input x0 filled); train keeps
+// every layer's activations (the backward pass reads them), inference fuses
+// layers 0 and 1 and the head.  The first decoder convolution of a level
+// reads the coarse level and the skip tensor directly.
+int forward(vc_ctx* ctx, vc_surrogate* s, bool train)
 {
     hipStream_t S = ctx->stream;
     const bf16* in = s->x0;
     int rc;
-    s->full_acts = keep_cat;
+    s->full_acts = train;
     auto conv = [&](int l, const bf16* x) {
         const LayerSpec& L = kLayers[l];
         if (l == 0)
@@ -1944,7 +1947,7 @@ int forward(vc_ctx* ctx, vc_surrogate* s, bool keep_cat)
         Z = s->Z >> lv;
     };
     int X, Y, Z;
-    if (keep_cat || !VC_CONV_FUSE01)
+    if (train || !VC_CONV_FUSE01)
     {
         if ((rc = conv(0, in)) != VC_OK || (rc = conv(1, s->act[0])) != VC_OK)
             return rc;
@@ -1981,33 +1984,21 @@ int forward(vc_ctx* ctx, vc_surrogate* s, bool keep_cat)
             return rc;
     }
     // decoder: level 2, 1, 0
-    bf16* cats[3] = {s->cat2, s->cat1, s->cat0};
-    const int c1s[3] = {64, 48, 32}, c2s[3] = {48, 32, 16};
+    const int c1s[3] = {64, 48, 32};
     const bf16* ups[3] = {s->act[7], s->act[9], s->act[11]};
     const bf16* skips[3] = {s->act[5], s->act[3], s->act[1]};
     for (int d = 0; d < 3; ++d)
     {
         const int lv = 2 - d;
         dims(lv, X, Y, Z);
-        if (keep_cat)
-        {
-            const int64_t n = level_voxels(s, lv) * (c1s[d] + c2s[d]);
-            concat_fwd<<<grid_for(n), kBlock, 0, S>>>(ups[d], c1s[d], skips[d],
-                                                         c2s[d], cats[d], X, Y, Z);
-            VC_CHECK_LAUNCH(ctx);
-            rc = conv(8 + 2 * d, cats[d]);
-        }
-        else
-        {
-            const int l = 8 + 2 * d;
-            const LayerSpec& L = kLayers[l];
-            rc = launch_conv(ctx, ups[d], L.cin, s->act[l], L.cout, s->Wf[l],
-                             s->theta + param_offset(l) + 27LL * L.cin * L.cout, X, Y,
-                             Z, s->kc[l], 1, level_box(s, L.level), skips[d], c1s[d]);
-        }
+        const int l = 8 + 2 * d;
+        const LayerSpec& L = kLayers[l];
+        rc = launch_conv(ctx, ups[d], L.cin, s->act[l], L.cout, s->Wf[l],
+                         s->theta + param_offset(l) + 27LL * L.cin * L.cout, X, Y, Z, s->kc[l],
+                         1, level_box(s, L.level), skips[d], c1s[d]);
         if (rc != VC_OK)
             return rc;
-        if (d == 2 && !keep_cat)
+        if (d == 2 && !train)
         {
             // inference: the last layer with the head fused (its activations
             // are not kept)
@@ -2035,23 +2026,19 @@ int forward(vc_ctx* ctx, vc_surrogate* s, bool keep_cat)
     return VC_OK;
 }
 
-// layer l backward: gy (gradient of its ReLU output, in place) -> masked,
-// weight gradient, and (unless gx is null) the input gradient into gx
-int layer_back(vc_ctx* ctx, vc_surrogate* s, int l, bf16* gy, const bf16* x,
-               bf16* gx)
+// layer l backward: gy (gradient of its output, already masked by its ReLU)
+// -> weight gradient from its input and (unless gx is null) the input gradient
+// into gx, masked by the ReLU of the layer whose activations `mask` holds
+int layer_back(vc_ctx* ctx, vc_surrogate* s, int l, const bf16* gy, const WgIn& in, bf16* gx,
+               const bf16* mask)
 {
     const LayerSpec& L = kLayers[l];
     const int X = s->X >> L.level, Y = s->Y >> L.level, Z = s->Z >> L.level;
-    const int64_t V = (int64_t)X * Y * Z;
-    hipStream_t S = ctx->stream;
-    relu_mask<<<grid_for(V * L.cout), kBlock, 0, S>>>(gy, s->act[l],
-                                                         V * L.cout);
-    VC_CHECK_LAUNCH(ctx);
-    int rc = layer_wgrad(ctx, s, l, WgIn{nullptr, x, 0, cinp_of(L.cin)}, gy);
+    int rc = layer_wgrad(ctx, s, l, in, gy);
     if (rc != VC_OK || !gx)
         return rc;
-    return launch_conv(ctx, gy, L.cout, gx, cinp_of(L.cin), s->Wd[l], nullptr,
-                       X, Y, Z, s->kcd[l], 0, level_box(s, L.level));
+    return launch_conv(ctx, gy, L.cout, gx, cinp_of(L.cin), s->Wd[l], nullptr, X, Y, Z,
+                       s->kcd[l], 0, level_box(s, L.level), nullptr, 0, mask);
 }
 
 // inside voxels: 16 per load, one add per workgroup of a grid of at most one
@@ -2152,59 +2139,62 @@ int backward(vc_ctx* ctx, vc_surrogate* s, const vc_vol* v, float* loss_dev,
         Z = s->Z >> lv;
     };
     int X, Y, Z;
-    // decoder levels 0, 1, 2: (second conv, first conv, concat input, its
-    // gradient, up channels, coarse gradient target, skip gradient target)
+    auto plain = [&](const bf16* x, int l) {
+        return WgIn{nullptr, x, 0, cinp_of(kLayers[l].cin)};
+    };
+    // decoder levels 0, 1, 2: second and first convolution; the latter's
+    // input is the concatenation of the coarse level's output (layer lu, C1
+    // channels) and the skip tensor (layer ls), and gcat its gradient.  The
+    // skip's part waits there for the pooling's (below).
     struct Dec
     {
-        int lb, la, lv, C, C1;
-        bf16 *cat, *gcat, *gup, *gskip;
+        int lb, la, lv, C1, lu, ls;
+        bf16* gcat;
     };
-    const Dec dec[3] = {
-        {13, 12, 0, 48, 32, s->cat0, s->gcat0, s->gact[11], s->gact[1]},
-        {11, 10, 1, 80, 48, s->cat1, s->gcat1, s->gact[9], s->gact[3]},
-        {9, 8, 2, 112, 64, s->cat2, s->gcat2, s->gact[7], s->gact[5]}};
+    const Dec dec[3] = {{13, 12, 0, 32, 11, 1, s->gcat0},
+                        {11, 10, 1, 48, 9, 3, s->gcat1},
+                        {9, 8, 2, 64, 7, 5, s->gcat2}};
     for (const Dec& d : dec)
     {
-        if ((rc = layer_back(ctx, s, d.lb, s->gact[d.lb], s->act[d.la],
-                             s->gact[d.la])) != VC_OK)
+        if ((rc = layer_back(ctx, s, d.lb, s->gact[d.lb], plain(s->act[d.la], d.lb),
+                             s->gact[d.la], s->act[d.la])) != VC_OK)
             return rc;
-        if ((rc = layer_back(ctx, s, d.la, s->gact[d.la], d.cat, d.gcat)) !=
+        const int C = kLayers[d.la].cin;
+        if ((rc = layer_back(ctx, s, d.la, s->gact[d.la],
+                             WgIn{s->act[d.lu], s->act[d.ls], d.C1, C}, d.gcat, nullptr)) !=
             VC_OK)
             return rc;
         dims(d.lv, X, Y, Z);
-        const int64_t nu = level_voxels(s, d.lv + 1) * d.C1;
-        split_up<<<grid_for(nu), kBlock, 0, S>>>(d.gcat, d.C, d.C1, d.gup, X,
-                                                    Y, Z);
-        VC_CHECK_LAUNCH(ctx);
-        const int64_t Vl = level_voxels(s, d.lv);
-        split_skip<<<grid_for(Vl * (d.C - d.C1)), kBlock, 0, S>>>(
-            d.gcat, d.C, d.C1, d.gskip, Vl);
+        const int64_t nu = level_voxels(s, d.lv + 1) * d.C1 / 8;
+        split_up<<<grid_for(nu), kBlock, 0, S>>>(d.gcat, C, d.C1, s->act[d.lu], s->gact[d.lu],
+                                                  X, Y, Z);
         VC_CHECK_LAUNCH(ctx);
     }
-    // encoder levels 3, 2, 1: the pooled input's gradient adds into the
-    // gradient of the level above's second conv output
+    // encoder levels 3, 2, 1: the pooled input's gradient joins the skip's in
+    // the gradient of the level above's second convolution output
     bf16* pools[3] = {s->p1, s->p2, s->p3};
     bf16* gpools[3] = {s->gp1, s->gp2, s->gp3};
-    const int pc[3] = {16, 32, 48};
     for (int lv = 3; lv >= 1; --lv)
     {
-        const int lb = 2 * lv + 1, la = 2 * lv;
-        if ((rc = layer_back(ctx, s, lb, s->gact[lb], s->act[la],
-                             s->gact[la])) != VC_OK)
+        const int lb = 2 * lv + 1, la = 2 * lv, ls = 2 * lv - 1;
+        if ((rc = layer_back(ctx, s, lb, s->gact[lb], plain(s->act[la], lb), s->gact[la],
+                             s->act[la])) != VC_OK)
             return rc;
-        if ((rc = layer_back(ctx, s, la, s->gact[la], pools[lv - 1],
-                             gpools[lv - 1])) != VC_OK)
+        if ((rc = layer_back(ctx, s, la, s->gact[la], plain(pools[lv - 1], la),
+                             gpools[lv - 1], nullptr)) != VC_OK)
             return rc;
         dims(lv - 1, X, Y, Z);
-        const int64_t n = level_voxels(s, lv - 1) * pc[lv - 1];
-        pool_bwd_acc<<<grid_for(n), kBlock, 0, S>>>(
-            s->gact[2 * lv - 1], gpools[lv - 1], pc[lv - 1], X, Y, Z);
+        const Dec& d = dec[lv - 1]; // the decoder level of the same voxels
+        const int64_t n = level_voxels(s, lv - 1) * kLayers[ls].cout / 8;
+        skip_grad<<<grid_for(n), kBlock, 0, S>>>(d.gcat, kLayers[d.la].cin, d.C1,
+                                                  gpools[lv - 1], s->act[ls], s->gact[ls], X,
+                                                  Y, Z);
         VC_CHECK_LAUNCH(ctx);
     }
-    if ((rc = layer_back(ctx, s, 1, s->gact[1], s->act[0], s->gact[0])) !=
+    if ((rc = layer_back(ctx, s, 1, s->gact[1], plain(s->act[0], 1), s->gact[0], s->act[0])) !=
         VC_OK)
         return rc;
-    return layer_back(ctx, s, 0, s->gact[0], s->x8, nullptr);
+    return layer_back(ctx, s, 0, s->gact[0], plain(s->x8, 0), nullptr, nullptr);
 }
 
 int round8(int n) { return (n + 7) / 8 * 8; }
