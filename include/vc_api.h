@@ -134,7 +134,8 @@ typedef struct vc_thin_stats {
  * (lambda < level  <=>  lam2 < ceil(level^2) for the exact measure).
  * Result (vc_get_labels): 0 background, 1 kept at every level, 2+k removed at
  * level k.  The skeleton at level k is {label == 1 or label > 2+k}.
- * stats may be NULL; when given, the call waits for the result. */
+ * stats may be NULL; when given, the call waits for the result (otherwise the
+ * result is ordered on the context stream, as with the other entry points). */
 int vc_thin_levels(vc_ctx* ctx, vc_vol* vol, const float* levels,
                    int n_levels, vc_thin_stats* stats);
 

@@ -98,3 +98,33 @@ def test_thin_empty_and_full(vc, oracle):
                       "full": np.ones((9, 9, 9), np.uint8),
                       "one": np.pad(np.ones((1, 1, 1), np.uint8), 2)}.items():
         _compare(vc, oracle, occ, [2.0, 5.0], name)
+
+
+@pytest.mark.parametrize("case", ["ring", "levels", "unwaited"])
+def test_thin_watched_levels(vc, oracle, case):
+    """The host follows a level through one word that each sweep writes for the
+    sweep before it: more sweeps in a level than the device's ring of flags has
+    entries (64), many levels in a row of which most converge in their first
+    sweep, and calls that follow each other without a wait."""
+    if case == "ring":  # a bar loses two voxels per end and sweep
+        occ = np.zeros((5, 6, 410), np.uint8)
+        occ[2, 3, 3:-3] = 1
+        _compare(vc, oracle, occ, [1e6], case)
+        occ[1:3, 2:4, 3:-3] = 1
+        _compare(vc, oracle, occ, [1.5, 1e6], case)
+    elif case == "levels":
+        rng = np.random.default_rng(17)
+        occ = (rng.random((33, 20, 70)) < 0.9).astype(np.uint8)
+        _compare(vc, oracle, occ, [0.25 * q for q in range(64)], case)
+    else:
+        rng = np.random.default_rng(18)
+        occ = (rng.random((40, 37, 50)) < 0.85).astype(np.uint8)
+        sets = [[1.5], [0.5, 2.5, 4.0], [1e6]]
+        vol = vc.upload(occ)
+        vol.edt().measure()
+        for levels in sets + sets[::-1]:
+            say("thin", case, levels)
+            vol.thin_levels(levels, stats=False)
+            vol.thin_levels(levels, stats=False)
+            assert np.array_equal(vol.get(4), _oracle_thin(oracle, occ, levels)[0])
+        vol.release()

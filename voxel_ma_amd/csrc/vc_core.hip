@@ -141,8 +141,18 @@ int vc_ctx_create(int device, vc_ctx** out)
          hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming) != hipSuccess ||
          hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming) != hipSuccess))
         rc = VC_ERR_HIP;
+    if (rc == VC_OK && hipHostMalloc((void**)&ctx->h_prog, sizeof(*ctx->h_prog),
+                                     hipHostMallocMapped | hipHostMallocCoherent) !=
+                           hipSuccess)
+    {
+        (void)hipGetLastError();
+        rc = VC_ERR_NOMEM;
+    }
     if (rc == VC_OK)
+    {
+        *ctx->h_prog = 0;
         rc = vc_lut_build(ctx);
+    }
     if (rc == VC_OK)
         rc = vc_noalloc_setup(ctx);
     if (rc == VC_OK && hipStreamSynchronize(ctx->stream) != hipSuccess)
@@ -167,6 +177,8 @@ int vc_ctx_destroy(vc_ctx* ctx)
     for (int k = 0; k < VC_WS_SLOTS; ++k)
         vc_free(ctx->ws[k]);
     vc_noalloc_teardown(ctx);
+    if (ctx->h_prog)
+        (void)hipHostFree(ctx->h_prog);
     for (hipEvent_t e : ctx->ev_free)
         (void)hipEventDestroy(e);
     for (auto& pr : ctx->ev_open)

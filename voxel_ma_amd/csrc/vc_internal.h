@@ -55,6 +55,10 @@ struct vc_ctx
     std::vector<hipEvent_t> ev_free;                         // reusable
     std::vector<std::pair<hipEvent_t, hipEvent_t>> ev_open;  // not yet read
     std::vector<int> ev_open_n;                              // launches per pair
+    // the word (pinned, coherent host memory) in which a tile sweep reports
+    // the sweep before it, and the level it belongs to (vc_thin.hip)
+    unsigned long long* h_prog = nullptr;
+    uint32_t prog_epoch = 0;
     // vc_skeleton_noalloc: this device's scratch array (device address) and
     // the host records of the call, built at context creation
     uint8_t* na_scratch = nullptr;
@@ -202,7 +206,9 @@ struct vc_work
                   // no dependent load before the first data access)
 };
 
-// sweeps per segment when vc_schedule.sweeps_per_sync is 0 (adaptive)
+// sweeps per segment when vc_schedule.sweeps_per_sync is 0 or -1 (adaptive)
+// and the convergence is checked by copying the ring (dense passes, graphs,
+// timed sweeps)
 constexpr int VC_SEG_MIN = 4, VC_SEG_MAX = 16;
 // ring of per-sweep "removed anything" flags
 constexpr int VC_RING = 64;

@@ -281,5 +281,9 @@ extern "C" int vc_skeleton_noalloc(vc_ctx* ctx, const uint8_t* d_occ, int nx,
         rc = vc_measure_sched(ctx, s);
     if (rc == VC_OK)
         rc = vc_thin_sched(ctx, s, levels, n_levels, stats);
+    // the caller's label array is complete for every stream and the host, and
+    // the scratch array idle, when the call returns
+    if (rc == VC_OK)
+        VC_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return rc;
 }

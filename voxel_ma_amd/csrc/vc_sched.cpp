@@ -66,9 +66,14 @@ void drop_graphs(vc_sched* s);
 // captured launches hold the views by value: every change re-captures
 int upload_desc(vc_ctx* ctx, vc_sched* s)
 {
+    // a single volume's kernels take its view as an argument (vc_work::one)
+    if (s->n == 1 && s->graphs.empty())
+        return VC_OK;
     // the staging buffer may still feed an earlier copy
     VC_HIP(ctx, hipStreamSynchronize(ctx->stream));
     drop_graphs(s);
+    if (s->n == 1)
+        return VC_OK;
     std::memcpy(s->h_stage, s->h_desc.data(), sizeof(vc_vdesc) * s->n);
     VC_HIP(ctx, hipMemcpyAsync(s->d_desc, s->h_stage,
                                sizeof(vc_vdesc) * s->n,
