@@ -128,3 +128,34 @@ def test_thin_watched_levels(vc, oracle, case):
             vol.thin_levels(levels, stats=False)
             assert np.array_equal(vol.get(4), _oracle_thin(oracle, occ, levels)[0])
         vol.release()
+
+
+@pytest.mark.parametrize("nz", [1, 2, 7, 8, 9, 15, 63, 64, 65, 71, 128, 131, 255, 257, 519])
+def test_row_lengths(vc, oracle, nz):
+    """Rows of every alignment: the row pass of the EDT and the level set-ups
+    read 8 voxels per access, a chunk that the row's end cuts as the row's last
+    8 (rows shorter than 8 voxel by voxel), and share a wavefront between short
+    rows; the last voxels of a row, inside and outside, and the exact and the
+    float measure, against the oracle."""
+    import voxel_ma_amd as V
+    rng = np.random.default_rng(nz)
+    occ = (rng.random((7, 9, nz)) < 0.8).astype(np.uint8)
+    occ[3, :, -3:] = 1
+    occ[4, :, -3:] = 0
+    levels = [0.5, 1.5, 3.0]
+    _compare(vc, oracle, occ, levels, "nz %d" % nz)
+    vol = vc.upload(occ)
+    vol.edt()
+    d, f = oracle.edt_ft(occ)
+    assert np.array_equal(vol.get(V.BUF_EDT), d) and np.array_equal(vol.get(V.BUF_FT), f)
+    meas = rng.uniform(0, 4, size=occ.shape).astype(np.float32)
+    dm = V.DeviceBuffer.from_array(meas)
+    vol.set_measure_f32(dm.ptr)
+    vol.thin_levels(levels)
+    lvlo = np.full(occ.shape, 255, np.uint8)
+    for k in reversed(range(len(levels))):
+        lvlo[(occ > 0) & (meas < np.float32(levels[k]))] = k
+    assert np.array_equal(vol.get(V.BUF_LEVEL), lvlo)
+    assert np.array_equal(vol.get(V.BUF_LABEL), oracle.thin(occ, lvlo, len(levels))[0])
+    vol.release()
+    dm.free()

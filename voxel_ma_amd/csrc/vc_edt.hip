@@ -26,7 +26,6 @@ namespace
 {
 
 constexpr int kBlock = 256;
-constexpr int kRowsZ = 4; // pass z: one wavefront per row, 4 rows per item
 constexpr uint32_t kOob = 0xFFFFFFFEu; // neighbour outside the grid
 // every candidate cost fits in int32: the volume constructor rejects shapes
 // whose squared diagonal exceeds INT32_MAX
@@ -47,17 +46,18 @@ constexpr int kInf = 0x7FFFFFFF;
 // radius 250 most are (EDT 10.2 -> 4.1 ms).
 constexpr int kDeepY = 128, kDeepX = 48;
 
-// rows along z: wavefront = row; the row's background bitmask sits in the
-// wavefront's LDS slice of `stride` words (rows whose length is a multiple
-// of 8: 8 voxels per lane and access; others: one ballot per 64 voxels)
+// rows along z: vc_ez_lanes(nz) lanes per row and 8 voxels per lane and
+// access, whatever nz is (one load, a background byte by SWAR zero-byte
+// detection, one nearest-background search per side of the lane's block, one
+// store); the row's background bitmask sits in its LDS words.  A wavefront per
+// row with one byte per lane for the lengths that are no multiple of 8 took 67
+// us for 301 x 222 x 437 voxels and 228 us for 64 volumes of edge 32-192 (84 M
+// voxels); with this 49 and 124 us (512^3: 141 -> 138 us).
 template <bool kB>
 __global__ void __launch_bounds__(kBlock)
-    edt_pass_z(vc_work W, int stride)
+    edt_pass_z(vc_work W)
 {
     extern __shared__ uint64_t lds_z[];
-    const int lane = threadIdx.x & 63;
-    const int wv = threadIdx.x >> 6;
-    uint64_t* bgmask = lds_z + (size_t)wv * stride;
     for (uint32_t b = blockIdx.x; b < W.total; b += gridDim.x)
     {
         int vi;
@@ -65,159 +65,119 @@ __global__ void __launch_bounds__(kBlock)
         vc_item<kB>(W, b, vi, lt);
         const vc_vdesc d = vc_desc<kB>(W, vi);
         const int nz = d.nz;
-        const int64_t row = (int64_t)lt * kRowsZ + wv;
-        const bool active = row < (int64_t)d.nx * d.ny;
-        const uint8_t* r = d.occ + row * nz;
-        const int nw = (nz + 63) >> 6;
-        if ((nz & 7) == 0)
+        const int lpr = vc_ez_lanes(nz), lsh = __ffs(lpr) - 1;
+        const int lane = threadIdx.x & (lpr - 1), ri = threadIdx.x >> lsh;
+        const uint32_t rows = (uint32_t)d.nx * (uint32_t)d.ny;
+        const int nw = (nz + 63) >> 6, nr = vc_ez_rows(nz);
+        const int rpi = kBlock >> lsh; // rows in flight together, nr times
+        // row q of this lane and its mask words
+        const uint32_t row0 = lt * (uint32_t)(nr * rpi) + (uint32_t)ri;
+        uint64_t* bgmask = lds_z + (size_t)ri * nw;
+        // the bytes of the last word past the row end hold no background
+        for (int q = 0; q < nr; ++q)
+            for (int c = ((nz + 7) >> 3) + lane; c < nw * 8; c += lpr)
+                reinterpret_cast<uint8_t*>(bgmask + (size_t)q * rpi * nw)[c] = 0;
+        for (int z0 = lane * 8; z0 < nz; z0 += 8 * lpr)
         {
-            // 8 voxels per lane: one 8-byte load, a background byte by SWAR
-            // zero-byte detection, one nearest-background search per side of
-            // the lane's block, one 16-byte store
-            uint8_t* bgb = reinterpret_cast<uint8_t*>(bgmask);
-            if (active)
-            {
-                // the bytes of the last word past the row end hold no
-                // background
-                for (int q = (nz >> 3) + lane; q < nw * 8; q += 64)
-                    bgb[q] = 0;
-                for (int z0 = lane * 8; z0 < nz; z0 += 512)
-                {
-                    const uint64_t v =
-                        *reinterpret_cast<const uint64_t*>(r + z0);
-                    constexpr uint64_t k7f = 0x7F7F7F7F7F7F7F7Full;
-                    const uint64_t zb = ~(((v & k7f) + k7f) | v | k7f);
-                    bgb[z0 >> 3] = (uint8_t)(((zb >> 7) * 0x0102040810204080ull) >> 56);
-                }
-            }
-            __syncthreads();
-            if (active)
-            {
-                int16_t* out = reinterpret_cast<int16_t*>(d.edt) + row * nz;
-                for (int z0 = lane * 8; z0 < nz; z0 += 512)
-                {
-                    const int w = z0 >> 6, k = (z0 >> 3) & 7;
-                    const uint64_t m = bgmask[w];
-                    const uint32_t b = (uint32_t)(m >> (8 * k)) & 0xFFu;
-                    int Lb = -1, Rb = -1;
-                    const uint64_t lm = k ? m & ((1ull << (8 * k)) - 1ull) : 0ull;
-                    if (lm)
-                        Lb = (w << 6) + 63 - __clzll(lm);
-                    else
-                        for (int ww = w - 1; ww >= 0; --ww)
-                        {
-                            const uint64_t q = bgmask[ww];
-                            if (q)
-                            {
-                                Lb = (ww << 6) + 63 - __clzll(q);
-                                break;
-                            }
-                        }
-                    const uint64_t rm = k < 7 ? m & ~((1ull << (8 * k + 8)) - 1ull) : 0ull;
-                    if (rm)
-                        Rb = (w << 6) + __ffsll((unsigned long long)rm) - 1;
-                    else
-                        for (int ww = w + 1; ww < nw; ++ww)
-                        {
-                            const uint64_t q = bgmask[ww];
-                            if (q)
-                            {
-                                Rb = (ww << 6) + __ffsll((unsigned long long)q) - 1;
-                                break;
-                            }
-                        }
-                    uint32_t packed[4];
+            uint64_t v[kEzRep];
 #pragma unroll
-                    for (int j = 0; j < 8; ++j)
-                    {
-                        const int z = z0 + j;
-                        int res;
-                        if ((b >> j) & 1u)
-                            res = z;
-                        else
-                        {
-                            const uint32_t below = b & ((1u << j) - 1u);
-                            const uint32_t above = b & ~((2u << j) - 1u);
-                            const int L = below ? z0 + 31 - __clz(below) : Lb;
-                            const int R = above ? z0 + __ffs(above) - 1 : Rb;
-                            res = L < 0 ? R : (R < 0 ? L : (z - L <= R - z ? L : R));
-                            if (res < 0 || abs(z - res) > kDeepY)
-                                d.fy[(row / d.ny) * ((nz + d.tzy - 1) / d.tzy) + z / d.tzy] = 1;
-                        }
-                        if (j & 1)
-                            packed[j >> 1] |= (uint32_t)(uint16_t)res << 16;
-                        else
-                            packed[j >> 1] = (uint32_t)(uint16_t)res;
-                    }
-                    *reinterpret_cast<uint4*>(out + z0) =
-                        make_uint4(packed[0], packed[1], packed[2], packed[3]);
-                }
-            }
-            __syncthreads(); // the slice is rewritten by the next item
-            continue;
-        }
-        if (active)
-            for (int w = 0; w < nw; ++w)
+            for (int q = 0; q < kEzRep; ++q)
             {
-                const int z = (w << 6) + lane;
-                const bool bg = (z < nz) && r[z] == 0;
-                const uint64_t m = __ballot(bg);
-                if (lane == 0)
-                    bgmask[w] = m;
+                const uint32_t row = row0 + (uint32_t)(q * rpi);
+                v[q] = q < nr && row < rows ? vc_row8(d.occ + (int64_t)row * nz, z0, nz) : 0;
             }
+            // past the row's end: no background
+            const uint32_t in = nz - z0 < 8 ? (1u << (nz - z0)) - 1u : 0xFFu;
+#pragma unroll
+            for (int q = 0; q < kEzRep; ++q)
+            {
+                constexpr uint64_t k7f = 0x7F7F7F7F7F7F7F7Full;
+                const uint64_t zb = ~(((v[q] & k7f) + k7f) | v[q] | k7f);
+                const uint32_t bg = (uint32_t)(((zb >> 7) * 0x0102040810204080ull) >> 56);
+                if (q < nr)
+                    reinterpret_cast<uint8_t*>(bgmask + (size_t)q * rpi * nw)[z0 >> 3] =
+                        (uint8_t)(bg & in);
+            }
+        }
         __syncthreads();
-        if (active)
+        for (int q = 0; q < nr; ++q)
         {
-            int16_t* out = reinterpret_cast<int16_t*>(d.edt) + row * nz;
-            for (int z = lane; z < nz; z += 64)
+            const uint32_t row = row0 + (uint32_t)(q * rpi);
+            if (row >= rows)
+                break;
+            const uint64_t* bgm = bgmask + (size_t)q * rpi * nw;
+            int16_t* out = reinterpret_cast<int16_t*>(d.edt) + (int64_t)row * nz;
+            for (int z0 = lane * 8; z0 < nz; z0 += 8 * lpr)
             {
-                const int w = z >> 6, bb = z & 63;
-                const uint64_t m = bgmask[w];
-                int res;
-                if ((m >> bb) & 1ull)
-                    res = z;
+                const int w = z0 >> 6, k = (z0 >> 3) & 7;
+                const uint64_t m = bgm[w];
+                const uint32_t b = (uint32_t)(m >> (8 * k)) & 0xFFu;
+                int Lb = -1, Rb = -1;
+                const uint64_t lm = k ? m & ((1ull << (8 * k)) - 1ull) : 0ull;
+                if (lm)
+                    Lb = (w << 6) + 63 - __clzll(lm);
                 else
+                    for (int ww = w - 1; ww >= 0; --ww)
+                    {
+                        const uint64_t bw = bgm[ww];
+                        if (bw)
+                        {
+                            Lb = (ww << 6) + 63 - __clzll(bw);
+                            break;
+                        }
+                    }
+                const uint64_t rm = k < 7 ? m & ~((1ull << (8 * k + 8)) - 1ull) : 0ull;
+                if (rm)
+                    Rb = (w << 6) + __ffsll((unsigned long long)rm) - 1;
+                else
+                    for (int ww = w + 1; ww < nw; ++ww)
+                    {
+                        const uint64_t bw = bgm[ww];
+                        if (bw)
+                        {
+                            Rb = (ww << 6) + __ffsll((unsigned long long)bw) - 1;
+                            break;
+                        }
+                    }
+                uint32_t packed[4];
+                bool deep = false;
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
                 {
-                    int L = -1, R = -1;
-                    const uint64_t lm = m & ((1ull << bb) - 1ull); // below bb
-                    if (lm)
-                        L = (w << 6) + 63 - __clzll(lm);
+                    const int z = z0 + j;
+                    int res;
+                    if ((b >> j) & 1u)
+                        res = z;
                     else
-                        for (int ww = w - 1; ww >= 0; --ww)
-                        {
-                            const uint64_t q = bgmask[ww];
-                            if (q)
-                            {
-                                L = (ww << 6) + 63 - __clzll(q);
-                                break;
-                            }
-                        }
-                    const uint64_t rm = m & ~((2ull << bb) - 1ull); // above bb
-                    if (rm)
-                        R = (w << 6) + __ffsll((unsigned long long)rm) - 1;
+                    {
+                        const uint32_t below = b & ((1u << j) - 1u);
+                        const uint32_t above = b & ~((2u << j) - 1u);
+                        const int L = below ? z0 + 31 - __clz(below) : Lb;
+                        const int R = above ? z0 + __ffs(above) - 1 : Rb;
+                        res = L < 0 ? R : (R < 0 ? L : (z - L <= R - z ? L : R));
+                        deep = deep || res < 0 || abs(z - res) > kDeepY;
+                    }
+                    if (j & 1)
+                        packed[j >> 1] |= (uint32_t)(uint16_t)res << 16;
                     else
-                        for (int ww = w + 1; ww < nw; ++ww)
-                        {
-                            const uint64_t q = bgmask[ww];
-                            if (q)
-                            {
-                                R = (ww << 6) + __ffsll((unsigned long long)q) - 1;
-                                break;
-                            }
-                        }
-                    if (L < 0)
-                        res = R;
-                    else if (R < 0)
-                        res = L;
-                    else
-                        res = (z - L <= R - z) ? L : R;
-                    if (res < 0 || abs(z - res) > kDeepY)
-                        d.fy[(row / d.ny) * ((nz + d.tzy - 1) / d.tzy) + z / d.tzy] = 1;
+                        packed[j >> 1] = (uint32_t)(uint16_t)res;
                 }
-                out[z] = (int16_t)res;
+                // (a flag too many, past the row's end or in a narrower tile,
+                // costs time only)
+                if (deep)
+                    for (int z = z0; z < min(z0 + 8, nz); z += d.tzy)
+                        d.fy[(int64_t)(row / (uint32_t)d.ny) * ((nz + d.tzy - 1) / d.tzy) +
+                             z / d.tzy] = 1;
+                if (nz - z0 >= 8)
+                    vc_stu(out + z0, make_uint4(packed[0], packed[1], packed[2], packed[3]));
+                else
+#pragma unroll
+                    for (int j = 0; j < 7; ++j)
+                        if (j < nz - z0)
+                            out[z0 + j] = (int16_t)(packed[j >> 1] >> (16 * (j & 1)));
             }
         }
-        __syncthreads(); // the slice is rewritten by the next item
+        __syncthreads(); // the rows' words are rewritten by the next item
     }
 }
 
@@ -904,10 +864,10 @@ int vc_edt_sched(vc_ctx* ctx, vc_sched* s)
     {
         if (s->n > 1)
             edt_pass_z<true><<<g, kBlock, s->lds[VK_EZ], ctx->stream>>>(
-                vc_sched_work(s, VK_EZ), s->ez_stride);
+                vc_sched_work(s, VK_EZ));
         else
             edt_pass_z<false><<<g, kBlock, s->lds[VK_EZ], ctx->stream>>>(
-                vc_sched_work(s, VK_EZ), s->ez_stride);
+                vc_sched_work(s, VK_EZ));
         VC_CHECK_LAUNCH(ctx);
     }
     g = vc_sched_grid(ctx, s, VK_EY, pc);

@@ -185,11 +185,11 @@ struct vc_vdesc
 // kernels with a work table
 enum vc_kind
 {
-    VK_EZ = 0, // EDT pass z: 4 rows per item
+    VK_EZ = 0, // EDT pass z: vc_ez_rows * 256 / vc_ez_lanes rows per item
     VK_EY,     // EDT pass y: one (x, z-tile) column tile per item
     VK_EX,     // EDT pass x: one (y, z-tile) column tile per item
     VK_MS,     // measure: one kMeasZ x kMeasY x kMeasXC wavefront strip per item
-    VK_LI,     // level set-up: 4 wavefronts (512 z each) per item
+    VK_LI,     // level set-up: 32 plane words per item
     VK_TP,     // subfield pass, (x, y) parity 0..3: 256 words per item
     VK_TT = VK_TP + 4, // tile sweep: one 32 x 32 x 64 (x, y, z) tile per item
     VK_LN,             // level set-up for k > 0: 256 plane words per item
@@ -226,7 +226,6 @@ struct vc_sched
     uint64_t* d_items[VK_COUNT] = {};
     uint32_t total[VK_COUNT] = {};
     size_t lds[VK_COUNT] = {};
-    int ez_stride = 0; // LDS words per wavefront in pass z
     int64_t voxels = 0, words = 0;
     vc_schedule sc{};
     // per-volume level thresholds, n x VC_MAX_LEVELS each
@@ -305,6 +304,48 @@ __host__ __device__ inline void vc_unpack_xyz(const vc_pack& p, uint32_t v,
     y = (int)((v >> p.bz) & p.my);
     x = (int)(v >> (p.by + p.bz));
 }
+
+// ---------------------------------------------------------------- rows
+// Rows of nz voxels start at any byte when nz is not a multiple of 8: the
+// hardware takes such vector accesses, so a chunk of 8 voxels is one access
+// whatever nz is.  T at p, no alignment assumed.
+template <typename T> __device__ __forceinline__ T vc_ldu(const void* p)
+{
+    T v;
+    __builtin_memcpy(&v, p, sizeof(T));
+    return v;
+}
+template <typename T> __device__ __forceinline__ void vc_stu(void* p, const T& v)
+{
+    __builtin_memcpy(p, &v, sizeof(T));
+}
+// 8 bytes of a row of nz bytes from z0 < nz on, 0 past its end; a chunk that
+// the row's end cuts is read as the row's last 8 bytes
+__device__ __forceinline__ uint64_t vc_row8(const uint8_t* row, int z0, int nz)
+{
+    const int rem = nz - z0;
+    if (rem >= 8)
+        return vc_ldu<uint64_t>(row + z0);
+    if (nz >= 8)
+        return vc_ldu<uint64_t>(row + nz - 8) >> (8 * (8 - rem));
+    uint64_t v = 0;
+    for (int j = 0; j < rem; ++j)
+        v |= (uint64_t)row[z0 + j] << (8 * j);
+    return v;
+}
+// EDT pass z: lanes of a row (8 voxels each), so that short rows share a
+// wavefront
+__host__ __device__ inline int vc_ez_lanes(int nz)
+{
+    int l = 1;
+    while (l < 64 && 8 * l < nz)
+        l <<= 1;
+    return l;
+}
+// and rows per lane: kEzRep rows in flight together (their bit masks fit
+// 16 KB of LDS up to 2048 voxels a row), one for longer rows
+constexpr int kEzRep = 4;
+__host__ __device__ inline int vc_ez_rows(int nz) { return nz <= 2048 ? kEzRep : 1; }
 
 // ---------------------------------------------------------------- work items
 // Kernels are instantiated twice: kB = false for one volume (the view is the

@@ -13,8 +13,7 @@
 namespace
 {
 
-constexpr int kRowsZ = 4;       // EDT pass z: rows (wavefronts) per item
-constexpr int kLiWaves = 4;     // level set-up: wavefronts per item
+constexpr int kLiWords = 32;    // level set-up: plane words per item
 constexpr int kTpWords = 256;   // subfield pass: words per item
 constexpr int kTileXY = 32;     // tile sweep: rows per tile along x and y
 
@@ -36,13 +35,14 @@ int64_t items_of(const vc_vdesc& d, int kind)
 {
     switch (kind)
     {
-    case VK_EZ: return cdiv((int64_t)d.nx * d.ny, kRowsZ);
+    case VK_EZ:
+        return cdiv((int64_t)d.nx * d.ny, vc_ez_rows(d.nz) * (256 / vc_ez_lanes(d.nz)));
     case VK_EY: return (int64_t)d.nx * cdiv(d.nz, d.tzy);
     case VK_EX: return (int64_t)d.ny * cdiv(d.nz, d.tzx);
     case VK_MS:
         return cdiv(d.nz, kMeasZ) * cdiv(d.ny, kMeasY) * cdiv(d.nx, kMeasXC);
     case VK_LI:
-        return cdiv((int64_t)d.nx * d.ny * cdiv(d.nz, 512), kLiWaves);
+        return cdiv((int64_t)d.nx * d.ny * d.nwz, kLiWords);
     case VK_TT:
         return (int64_t)d.ntx * d.nty * d.nwz;
     case VK_LN:
@@ -206,15 +206,15 @@ int vc_sched_apply(vc_ctx* ctx, vc_sched* s, const vc_schedule& sc)
         d.tzx = pick_tile(d.nx, 4, std::min(2 * budget, (size_t)65536), d.nz);
     }
     std::memset(s->lds, 0, sizeof(s->lds));
-    s->ez_stride = 0;
     for (const auto& d : s->h_desc)
     {
-        s->ez_stride = std::max(s->ez_stride, d.nwz);
+        s->lds[VK_EZ] =
+            std::max(s->lds[VK_EZ], (size_t)vc_ez_rows(d.nz) * (256 / vc_ez_lanes(d.nz)) *
+                                        d.nwz * 8);
         s->lds[VK_EY] = std::max(s->lds[VK_EY],
                                  (size_t)vc_edt_ystride(d.tzy) * d.ny * 2);
         s->lds[VK_EX] = std::max(s->lds[VK_EX], (size_t)d.tzx * d.nx * 4);
     }
-    s->lds[VK_EZ] = (size_t)kRowsZ * s->ez_stride * 8;
     for (int k = 0; k < VK_COUNT; ++k)
     {
         vc_free(s->d_items[k]);

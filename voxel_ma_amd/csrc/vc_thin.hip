@@ -133,33 +133,34 @@ __device__ __forceinline__ int64_t widx(const Plane& P, int x, int y, int w)
     return ((int64_t)x * P.ny + y) * P.nwz + w;
 }
 
-// Level set-up.  An item is 4 wavefronts; a wavefront covers 512 consecutive
-// z of one row (8 words): lane l handles z = z0 + 8l .. z0 + 8l + 7 and lanes
-// 8j .. 8j+7 assemble word j.  Words holding an alive voxel that becomes
-// eligible at level k are flagged for both z parities (every other eligible
-// voxel was found non-simple when the previous level converged and its
-// neighbourhood has not changed since).  Level 0 derives each voxel's first
-// eligible level from its volume's thresholds (exact: lam2 < T[q]; float
-// measure: m < L[q]); later levels read it back.  The launch also resets the
-// level's sweep control (sweep counter, level, "removed anything" rings).
-constexpr int kLiWaves = 4;
-
+// Level 0 set-up: 8 lanes per plane word, 8 voxels per lane, 32 words per
+// item.  Derives each voxel's first eligible level from its volume's
+// thresholds (exact: lam2 < T[q]; float measure: m < L[q]), the label (inside
+// or not) and the planes; flags words holding a voxel eligible at level 0 for
+// both z parities; resets the level's sweep control (sweep counter, level,
+// "removed anything" rings).
+//
+// A chunk that the row's end cuts is taken as the row's last 8 voxels (its
+// lower part is the chunk before it, whose values it writes again) and its
+// mask bits shifted down, so every row length runs on vector accesses: byte
+// accesses for the lengths that are no multiple of 8, and a wavefront per row,
+// took 131 us for 301 x 222 x 437 voxels and 831 us for 64 volumes of edge
+// 32-192 (84 M voxels), 58 and 169 us now (512^3: 240 us either way).  Bound: memory (occupancy, the measure of inside
+// voxels, levels and labels).
 template <bool kB>
 __global__ void __launch_bounds__(kBlock)
     thin_level_init(vc_work W, const uint64_t* __restrict__ Tq,
-                    const float* __restrict__ Lq, int nlev, int k, int nvol,
+                    const float* __restrict__ Lq, int nlev, int nvol,
                     uint32_t* __restrict__ ctl, uint32_t* __restrict__ gany,
                     uint32_t* __restrict__ vany)
 {
-    const int lane = threadIdx.x & 63;
-    const int wv = threadIdx.x >> 6;
     {
         const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
         const uint32_t gs = gridDim.x * blockDim.x;
         if (g == 0)
         {
             ctl[0] = 0;
-            ctl[1] = (uint32_t)k;
+            ctl[1] = 0;
         }
         for (uint32_t i = g; i < (uint32_t)VC_RING; i += gs)
             gany[i] = 0;
@@ -173,116 +174,58 @@ __global__ void __launch_bounds__(kBlock)
         vc_item<kB>(W, b, vi, lt);
         const vc_vdesc d = vc_desc<kB>(W, vi);
         const int nz = d.nz;
-        const int nchunk = (nz + 511) >> 9;
-        const int64_t wave = (int64_t)lt * kLiWaves + wv;
-        const int64_t rowi = wave / nchunk;
-        if (rowi >= (int64_t)d.nx * d.ny) // whole wavefront
+        const uint32_t o = lt * (kBlock / 8) + (threadIdx.x >> 3); // plane word
+        const uint32_t rowi = o / (uint32_t)d.nwz;
+        if (rowi >= (uint32_t)d.nx * (uint32_t)d.ny) // the word's 8 lanes
             continue;
-        const int z0 = (int)(wave % nchunk) * 512 + 8 * lane;
-        const int64_t base = rowi * nz;
-        const int mode = k > 0 ? 2 : (d.mkind == 2 ? 1 : 0);
-        // rows start 8-aligned when nz is a multiple of 8: one 8-byte access
-        // per lane instead of eight byte accesses (z0 + 8 <= nz then)
-        const bool vec = (nz & 7) == 0 && z0 < nz;
-        uint32_t am = 0, em = 0, nm = 0;
-        uint8_t lv8[8], lb8[8];
-        if (mode == 2)
+        const int z0 = (int)(o - rowi * (uint32_t)d.nwz) * 64 + 8 * (threadIdx.x & 7);
+        const int64_t base = (int64_t)rowi * nz;
+        uint32_t am = 0, em = 0;
+        if (z0 < nz)
         {
-            // alive voxels from the maintained plane; levels read back
-            if (z0 < nz)
-                am = (uint32_t)(d.alive[rowi * d.nwz + (z0 >> 6)] >> (z0 & 63)) &
-                     0xFFu;
-            if (vec)
+            const int zs = min(z0, max(nz - 8, 0)); // first voxel of the window
+            const int nv = min(8, nz);              // its voxels (nz < 8: the row)
+            const uint64_t ov = vc_row8(d.occ + base, zs, nz);
+            bool in[8];
+            uint8_t lv8[8];
+            uint32_t mi[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+            // 8 background voxels need no measure: skipping their loads
+            // leaves whole sectors of the measure unread inside the
+            // background (70 % of the 512^3 headline volume)
+            const void* m = d.mkind == 2 ? (const void*)(d.meas + base + zs)
+                                         : (const void*)(d.lam2 + base + zs);
+            if (ov && nv == 8)
             {
-                const uint64_t v =
-                    *reinterpret_cast<const uint64_t*>(d.lvl + base + z0);
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    lv8[j] = (uint8_t)(v >> (8 * j));
+                const uint4 u0 = vc_ldu<uint4>(m);
+                const uint4 u1 = vc_ldu<uint4>((const char*)m + 16);
+                mi[0] = u0.x; mi[1] = u0.y; mi[2] = u0.z; mi[3] = u0.w;
+                mi[4] = u1.x; mi[5] = u1.y; mi[6] = u1.z; mi[7] = u1.w;
             }
-            else
-            {
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    lv8[j] = z0 + j < nz ? d.lvl[base + z0 + j] : (uint8_t)255;
-            }
+            else if (ov)
+                for (int j = 0; j < 7; ++j)
+                    if (j < nv)
+                        mi[j] = static_cast<const uint32_t*>(m)[j];
 #pragma unroll
             for (int j = 0; j < 8; ++j)
-                lb8[j] = (uint8_t)((am >> j) & 1u);
-        }
-        else
-        {
-            // measure of the inside voxels, then the first level whose
-            // threshold exceeds it (thresholds ascending; q descending so the
-            // smallest such q is kept); thresholds are uniform scalar loads
-            uint64_t mi[8];
-            float mf[8];
-            if (vec)
             {
-                const uint64_t ov =
-                    *reinterpret_cast<const uint64_t*>(d.occ + base + z0);
-                uint32_t m32[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-                // 8 background voxels need no measure: skipping their loads
-                // leaves whole sectors of the measure unread inside the
-                // background (70 % of the 512^3 headline volume)
-                if (mode == 0 && ov)
-                {
-                    const uint4 u0 = *reinterpret_cast<const uint4*>(d.lam2 + base + z0);
-                    const uint4 u1 =
-                        *reinterpret_cast<const uint4*>(d.lam2 + base + z0 + 4);
-                    m32[0] = u0.x; m32[1] = u0.y; m32[2] = u0.z; m32[3] = u0.w;
-                    m32[4] = u1.x; m32[5] = u1.y; m32[6] = u1.z; m32[7] = u1.w;
-                }
-                else if (mode != 0 && ov)
-                {
-                    const float4 f0 = *reinterpret_cast<const float4*>(d.meas + base + z0);
-                    const float4 f1 =
-                        *reinterpret_cast<const float4*>(d.meas + base + z0 + 4);
-                    mf[0] = f0.x; mf[1] = f0.y; mf[2] = f0.z; mf[3] = f0.w;
-                    mf[4] = f1.x; mf[5] = f1.y; mf[6] = f1.z; mf[7] = f1.w;
-                }
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                {
-                    lb8[j] = ((ov >> (8 * j)) & 0xFFu) != 0;
-                    lv8[j] = 255;
-                    mi[j] = lb8[j] ? m32[j] : 0;
-                    if (mode == 0 || !lb8[j])
-                        mf[j] = 0.0f;
-                }
+                in[j] = ((ov >> (8 * j)) & 0xFFu) != 0;
+                lv8[j] = 255;
             }
-            else
-            {
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                {
-                    const int64_t i = base + z0 + j;
-                    const bool in = z0 + j < nz && d.occ[i] != 0;
-                    lb8[j] = in;
-                    lv8[j] = 255;
-                    mi[j] = 0;
-                    mf[j] = 0.0f;
-                    if (in)
-                    {
-                        if (mode == 0)
-                            mi[j] = d.lam2[i];
-                        else
-                            mf[j] = d.meas[i];
-                    }
-                }
-            }
+            // the first level whose threshold exceeds the measure (thresholds
+            // ascending; q descending so the smallest such q is kept);
+            // thresholds are uniform scalar loads
             typedef const __attribute__((address_space(4))) uint64_t* cu64;
             typedef const __attribute__((address_space(4))) float* cf32;
             const cu64 T = (cu64)(Tq + (size_t)vi * VC_MAX_LEVELS);
             const cf32 Lf = (cf32)(Lq + (size_t)vi * VC_MAX_LEVELS);
             for (int q = nlev - 1; q >= 0; --q)
             {
-                if (mode == 0)
+                if (d.mkind != 2)
                 {
                     const uint64_t t = T[q];
 #pragma unroll
                     for (int j = 0; j < 8; ++j)
-                        if (lb8[j] && mi[j] < t)
+                        if (in[j] && mi[j] < t)
                             lv8[j] = (uint8_t)q;
                 }
                 else
@@ -290,71 +233,68 @@ __global__ void __launch_bounds__(kBlock)
                     const float t = Lf[q];
 #pragma unroll
                     for (int j = 0; j < 8; ++j)
-                        if (lb8[j] && mf[j] < t)
+                        if (in[j] && __uint_as_float(mi[j]) < t)
                             lv8[j] = (uint8_t)q;
                 }
             }
-        }
+            uint64_t lvw = 0, lbw = 0;
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-        {
-            am |= (uint32_t)lb8[j] << j;
-            em |= (uint32_t)(lv8[j] <= k) << j;
-            nm |= (uint32_t)(lv8[j] == k) << j;
-        }
-        if (mode != 2)
-        {
-            if (vec)
+            for (int j = 0; j < 8; ++j)
             {
-                uint64_t lvw = 0, lbw = 0;
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                {
-                    lvw |= (uint64_t)lv8[j] << (8 * j);
-                    lbw |= (uint64_t)lb8[j] << (8 * j);
-                }
-                *reinterpret_cast<uint64_t*>(d.lvl + base + z0) = lvw;
-                *reinterpret_cast<uint64_t*>(d.label + base + z0) = lbw;
+                am |= (uint32_t)in[j] << j;
+                em |= (uint32_t)(lv8[j] == 0) << j;
+                lvw |= (uint64_t)lv8[j] << (8 * j);
+                lbw |= (uint64_t)in[j] << (8 * j);
+            }
+            if (nv == 8)
+            {
+                vc_stu(d.lvl + base + zs, lvw);
+                vc_stu(d.label + base + zs, lbw);
             }
             else
-            {
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    if (z0 + j < nz)
-                    {
-                        d.lvl[base + z0 + j] = lv8[j];
-                        d.label[base + z0 + j] = lb8[j];
-                    }
-            }
+                for (int j = 0; j < nv; ++j)
+                {
+                    d.lvl[base + j] = (uint8_t)(lvw >> (8 * j));
+                    d.label[base + j] = (uint8_t)(lbw >> (8 * j));
+                }
+            am >>= z0 - zs;
+            em >>= z0 - zs;
         }
-        const int sh = 8 * (lane & 7);
-        uint64_t a = (uint64_t)am << sh, e = (uint64_t)em << sh,
-                 nw = (uint64_t)nm << sh;
+        const int sh = 8 * (threadIdx.x & 7);
+        uint64_t a = (uint64_t)am << sh, e = (uint64_t)em << sh;
 #pragma unroll
         for (int dd = 1; dd <= 4; dd <<= 1)
         {
             a |= __shfl_xor(a, dd);
             e |= __shfl_xor(e, dd);
-            nw |= __shfl_xor(nw, dd);
         }
-        if ((lane & 7) == 0 && z0 < nz)
+        if ((threadIdx.x & 7) == 0)
         {
-            const int64_t o = rowi * d.nwz + (z0 >> 6);
             d.elig[o] = e;
-            const uint8_t f = (nw & a) ? 1 : 0;
+            const uint8_t f = (e & a) ? 1 : 0;
             d.d0[o] = f;
             d.d1[o] = f;
-            if (mode != 2)
-                d.alive[o] = a;
+            d.alive[o] = a;
         }
     }
 }
 
+// the bytes of v that are at most k < 64 (v: levels, 0..63 or 255), as 8 bits
+__device__ __forceinline__ uint64_t bytes_le(uint64_t v, int k)
+{
+    constexpr uint64_t kH = 0x8080808080808080ull, kL = 0x0101010101010101ull;
+    // high bit of a byte of t: its low 7 bits are at least k + 1
+    const uint64_t t = (v | kH) - (uint64_t)(k + 1) * kL;
+    return (((~t & kH) >> 7) * 0x0102040810204080ull) >> 56;
+}
+
 // Level set-up for k > 0, one thread per plane word: elig = (lvl <= k) of
 // its 64 voxels, and both revisit flags = an alive voxel becomes eligible
-// now (lvl == k).  The 64 level bytes are read as four 16-byte loads when the
-// rows are 16-byte aligned (nz a multiple of 16).  Also resets the level's
-// sweep control.
+// now (lvl == k; every other eligible voxel was found non-simple when the
+// previous level converged and its neighbourhood has not changed since).  The
+// level bytes are read 16 or 8 at a time whatever the row length (one byte at
+// a time, the lengths that are no multiple of 16 had taken 53 us for 301 x 222
+// x 437 voxels, 12 us now).  Also resets the level's sweep control.
 template <bool kB>
 __global__ void __launch_bounds__(kBlock)
     thin_level_next(vc_work W, int k, int nvol, uint32_t* __restrict__ ctl,
@@ -385,43 +325,35 @@ __global__ void __launch_bounds__(kBlock)
             continue;
         const int64_t rowi = o / d.nwz;
         const int z0 = (int)(o - rowi * d.nwz) * 64;
-        const uint8_t* lv = d.lvl + rowi * d.nz + z0;
         uint64_t e = 0, nw = 0;
         // eligibility only matters for alive voxels (every use ands it with
         // the alive plane): a word without one reads no levels, which at
         // later levels, after most voxels were removed, skips most of them
         const uint64_t al = d.alive[o];
-        if (!al)
+        if (al)
         {
-        }
-        else if ((d.nz & 15) == 0 && z0 + 64 <= d.nz)
-        {
+            const uint8_t* row = d.lvl + rowi * d.nz;
+            uint64_t c[8];
+            if (z0 + 64 <= d.nz)
 #pragma unroll
-            for (int c = 0; c < 4; ++c)
+                for (int q = 0; q < 4; ++q)
+                {
+                    const ulonglong2 v = vc_ldu<ulonglong2>(row + z0 + 16 * q);
+                    c[2 * q] = v.x;
+                    c[2 * q + 1] = v.y;
+                }
+            else
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+                    c[q] = z0 + 8 * q < d.nz ? vc_row8(row, z0 + 8 * q, d.nz) : 0ull;
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
             {
-                const uint4 q = reinterpret_cast<const uint4*>(lv)[c];
-                const uint32_t wd[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                    {
-                        const uint32_t l = (wd[u] >> (8 * j)) & 0xFFu;
-                        const int bit = 16 * c + 4 * u + j;
-                        e |= (uint64_t)(l <= (uint32_t)k) << bit;
-                        nw |= (uint64_t)(l == (uint32_t)k) << bit;
-                    }
+                const uint64_t le = bytes_le(c[q], k);
+                e |= le << (8 * q);
+                nw |= (le & ~bytes_le(c[q], k - 1)) << (8 * q);
             }
-        }
-        else
-        {
-            const int n = min(64, d.nz - z0);
-            for (int j = 0; j < n; ++j)
-            {
-                const uint32_t l = lv[j];
-                e |= (uint64_t)(l <= (uint32_t)k) << j;
-                nw |= (uint64_t)(l == (uint32_t)k) << j;
-            }
+            // (bytes past the row's end read as level 0; alive has no bit there)
         }
         d.elig[o] = e;
         const uint8_t f = (nw & al) ? 1 : 0;
@@ -1832,11 +1764,11 @@ int vc_thin_sched(vc_ctx* ctx, vc_sched* s, const float* levels, int nlev,
             }
             else if (s->n > 1)
                 thin_level_init<true><<<g, kBlock, 0, S>>>(
-                    W, s->d_T, s->d_L, nlev, k, s->n, s->d_ctl, s->d_gany,
+                    W, s->d_T, s->d_L, nlev, s->n, s->d_ctl, s->d_gany,
                     s->d_vany);
             else
                 thin_level_init<false><<<g, kBlock, 0, S>>>(
-                    W, s->d_T, s->d_L, nlev, k, s->n, s->d_ctl, s->d_gany,
+                    W, s->d_T, s->d_L, nlev, s->n, s->d_ctl, s->d_gany,
                     s->d_vany);
             VC_CHECK_LAUNCH(ctx);
             launches++;
