@@ -1,0 +1,72 @@
+"""GPU: the memory that a context frees and hands out again.  Volumes of sizes
+that share, split and miss each other's blocks, made and released without a
+wait between their work and the next volume's, in two threads with a context
+each: every result equals the oracle's; a context can be destroyed and
+another made in between."""
+import threading
+
+import numpy as np
+import pytest
+
+import voxel_ma_amd as V
+from conftest import say
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(20, 20, 20), (21, 20, 20), (40, 33, 70), (8, 8, 8), (64, 40, 24), (20, 20, 21)]
+
+
+@pytest.mark.parametrize("threads", [1, 2])
+def test_reused_blocks(oracle, threads):
+    rng = np.random.default_rng(41)
+    levels = [1.0, 2.5]
+    cases = []
+    for shape in SHAPES:
+        occ = (rng.random(shape) < 0.85).astype(np.uint8)
+        d, f = oracle.edt_ft(occ)
+        lvl = oracle.levels(occ, oracle.lambda2(occ, f), levels)
+        cases.append((occ, d, oracle.thin(occ, lvl, len(levels))[0]))
+    say("reused blocks", threads, "threads")
+    wrong = []
+
+    def work(seed):
+        order = np.random.default_rng(seed).integers(0, len(cases), 60)
+        ctx = V.Context(0)
+        held = []
+        for n, i in enumerate(order):
+            occ, d, lab = cases[i]
+            vol = ctx.upload(occ)
+            vol.edt().measure().thin_levels(levels, stats=False)
+            out = V.DeviceBuffer(occ.size)
+            vol.get_device(V.BUF_LABEL, out.ptr, out.nbytes)
+            if n % 3 == 0:  # some volumes outlive others
+                held.append((vol, d))
+            else:
+                vol.release()
+            if len(held) > 4:
+                v, dd = held.pop(0)
+                if not np.array_equal(v.get(V.BUF_EDT), dd):
+                    wrong.append(("edt", n))
+                v.release()
+            ctx.synchronize()
+            if not np.array_equal(out.download(np.uint8, occ.shape), lab):
+                wrong.append(("label", n))
+            out.free()
+            if n == 30:  # a second context's memory is its own
+                other = V.Context(0)
+                v2 = other.upload(occ)
+                v2.edt()
+                if not np.array_equal(v2.get(V.BUF_EDT), d):
+                    wrong.append(("other", n))
+                v2.release()
+                other.close()
+        for v, _ in held:
+            v.release()
+        ctx.close()
+
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(threads)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not wrong

@@ -5,6 +5,7 @@
 
 #include <cstdarg>
 #include <cstdint>
+#include <list>
 #include <map>
 #include <string>
 #include <utility>
@@ -31,6 +32,21 @@ enum vc_ws_slot
     VC_WS_BND_LAB,    // boundary: thin-layer labels
     VC_WS_SCAN,       // chunk totals of the scans
     VC_WS_SLOTS
+};
+
+// A context's freed memory, kept for its next allocations (vc_alloc,
+// vc_host_alloc): blocks in the order they were freed, oldest first, and by
+// size.  Guarded by one lock over all contexts.
+struct vc_cache
+{
+    struct block
+    {
+        void* p;
+        size_t bytes;
+    };
+    std::list<block> order;
+    std::multimap<size_t, std::list<block>::iterator> by_size;
+    size_t bytes = 0;
 };
 
 struct vc_ctx
@@ -64,6 +80,7 @@ struct vc_ctx
     uint8_t* na_scratch = nullptr;
     vc_vol* na_vol = nullptr;
     vc_sched* na_sched = nullptr;
+    vc_cache cache_dev, cache_host; // freed device / pinned host memory
     // reusable device scratch by slot (vc_ws_get): grown on demand, kept until
     // the context is destroyed, so repeated calls allocate nothing
     void* ws[VC_WS_SLOTS] = {};
@@ -142,8 +159,19 @@ int vc_fail(vc_ctx* ctx, int code, const char* fmt, ...);
 
 #define VC_CHECK_LAUNCH(ctx) VC_HIP(ctx, hipGetLastError())
 
+// Device memory of a context, from the blocks it freed before where one fits.
+// vc_free does not wait for the device: a block may be handed out again while
+// work queued on the context's stream still uses it, so every use of such
+// memory is queued on that stream, or on the second stream between a fork and
+// its join.  Contents are undefined.
 int vc_alloc(vc_ctx* ctx, void** p, size_t bytes);
 void vc_free(void* p);
+// the same for pinned host memory; the caller waits for the copies that use
+// it before it frees it
+int vc_host_alloc(vc_ctx* ctx, void** p, size_t bytes);
+void vc_host_free(void* p);
+// gives a context's kept memory back and forgets the context (its destruction)
+void vc_cache_release(vc_ctx* ctx);
 // device scratch of slot `slot` with at least `bytes` bytes, kept by the
 // context: contents are not preserved when it grows (the old buffer is freed
 // after the device finishes with it); calls on one context run one at a time

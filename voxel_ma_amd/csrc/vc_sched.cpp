@@ -160,14 +160,10 @@ void vc_sched_free(vc_sched* s)
     vc_free(s->d_gany);
     vc_free(s->d_vany);
     vc_free(s->d_ctr);
-    if (s->h_stage)
-        (void)hipHostFree(s->h_stage);
-    if (s->h_lv)
-        (void)hipHostFree(s->h_lv);
-    if (s->h_ring)
-        (void)hipHostFree(s->h_ring);
-    if (s->h_ctr)
-        (void)hipHostFree(s->h_ctr);
+    vc_host_free(s->h_stage);
+    vc_host_free(s->h_lv);
+    vc_host_free(s->h_ring);
+    vc_host_free(s->h_ctr);
     delete s;
 }
 
@@ -307,17 +303,14 @@ int vc_sched_build(vc_ctx* ctx, vc_vol* const* vols, int n,
     if (rc == VC_OK)
         rc = vc_alloc(ctx, (void**)&s->d_ctr,
                       8 * (size_t)VC_CTR_SLOTS * VC_CTR_WORDS);
-    if (rc == VC_OK &&
-        (hipHostMalloc((void**)&s->h_stage, sizeof(vc_vdesc) * n,
-                       hipHostMallocDefault) != hipSuccess ||
-         hipHostMalloc(&s->h_lv, 12 * (size_t)n * VC_MAX_LEVELS,
-                       hipHostMallocDefault) != hipSuccess ||
-         hipHostMalloc((void**)&s->h_ring, 4 * VC_RING,
-                       hipHostMallocDefault) != hipSuccess ||
-         hipHostMalloc((void**)&s->h_ctr,
-                       8 * (size_t)VC_CTR_SLOTS * VC_CTR_WORDS,
-                       hipHostMallocDefault) != hipSuccess))
-        rc = vc_fail(ctx, VC_ERR_NOMEM, "pinned host allocation failed");
+    if (rc == VC_OK)
+        rc = vc_host_alloc(ctx, (void**)&s->h_stage, sizeof(vc_vdesc) * n);
+    if (rc == VC_OK)
+        rc = vc_host_alloc(ctx, &s->h_lv, 12 * (size_t)n * VC_MAX_LEVELS);
+    if (rc == VC_OK)
+        rc = vc_host_alloc(ctx, (void**)&s->h_ring, 4 * VC_RING);
+    if (rc == VC_OK)
+        rc = vc_host_alloc(ctx, (void**)&s->h_ctr, 8 * (size_t)VC_CTR_SLOTS * VC_CTR_WORDS);
     if (rc == VC_OK)
         rc = vc_sched_apply(ctx, s, sc);
     if (rc != VC_OK)

@@ -2394,7 +2394,11 @@ int vc_surrogate_create(vc_ctx* ctx, uint64_t seed, vc_surrogate** out)
             }
             o += n + co;
         }
-        hipError_t e = hipMemcpy(s->theta, th.data(), pb, hipMemcpyHostToDevice);
+        // the copies below are not ordered with the context's stream, which
+        // may still use the memory's previous contents
+        hipError_t e = hipStreamSynchronize(ctx->stream);
+        if (e == hipSuccess)
+            e = hipMemcpy(s->theta, th.data(), pb, hipMemcpyHostToDevice);
         if (e == hipSuccess)
             e = hipMemset(s->m1, 0, pb);
         if (e == hipSuccess)
