@@ -70,6 +70,38 @@ def test_device_matches_host_on_large_grids(vc):
             _both(vc, nv, e, foff, fe, em, fm, f_t, l_t)
 
 
+@pytest.mark.parametrize("sides", [3, 6, 7, 14, 15, 30, 62, 63, 64, 65, 150])
+def test_device_matches_host_on_polygons(vc, sides):
+    """Lanes per pair follow the most sides of a face (8 up to 6 sides, 64 from
+    31 on, in rounds from 63 on): a band of polygons, neighbours sharing an edge,
+    with triangles, dangling edges and a second band over the first's edges."""
+    rng = np.random.default_rng(sides)
+    faces, nv = [], 0
+    for band in range(2):
+        a, b = 0, 1
+        nv = max(nv, 2)
+        for k in range(40):
+            n = sides if k % 3 else max(3, sides // 2)
+            ring = list(range(nv, nv + n - 2))
+            nv += n - 2
+            faces.append([a, b] + ring)
+            i = int(rng.integers(0, len(ring) - 1)) if len(ring) > 1 else 0
+            a, b = (ring[i], ring[i + 1]) if len(ring) > 1 else (b, ring[0])
+            faces.append([a, b, nv])
+            nv += 1
+    extra = [(int(rng.integers(0, nv)), nv + i) for i in range(10)]
+    nv += 10
+    e, foff, fe = V.cc_finalize(nv, extra, faces)
+    for q in (0, 3):
+        em = rng.random(len(e)).astype(np.float32)
+        fm = rng.random(len(faces)).astype(np.float32)
+        if q:
+            em, fm = np.floor(em * q) / q, np.floor(fm * q) / q
+        for f_t, l_t in ((1.1, 1.1), (0.6, 0.8), (1.1, 0.3)):
+            say("device collapse polygons", sides, q, f_t, l_t)
+            _both(vc, nv, e, foff, fe, em, fm, f_t, l_t)
+
+
 def test_device_matches_host_on_voxel_core(vc):
     """The inside part of the discrete Voronoi diagram of a ball and of a
     torus (triangulated, with the lambda measures of its faces and edges),

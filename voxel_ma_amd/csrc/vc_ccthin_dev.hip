@@ -21,9 +21,10 @@
 //     of the generation).  The pushed pair names the element's one cell left
 //     at that moment: the first in adjacency order not removed before the
 //     generation nor by an event with a smaller or equal key;
-//   * pushes are written to slots numbered by their keys (per pair |f| + 2
-//     slots for a face-edge pop, 1 for an edge-vertex pop), and compacting
-//     the slots gives the next generation in push order.
+//   * the next generation is the pushes in key order: pairs count their
+//     pushes, and a second evaluation writes each at the number of pushes
+//     before it.  An element pushes at most once in a generation, so a
+//     generation has at most (edges + vertices) pairs.
 // The reference exits with "logic err" when a pair it takes has a count
 // other than 1; those cases return VC_ERR_STATE here, as in vc_cc_prune.
 // An effective face-edge pair whose edge an edge-vertex pair of the same
@@ -121,12 +122,22 @@ __global__ void __launch_bounds__(kB)
 }
 
 // per face: side ids in range (else nothing is counted), sides listed
-// twice flagged; edge face counts
+// twice flagged; edge face counts; the most sides
 __global__ void __launch_bounds__(kB)
     deg_e(const int64_t* __restrict__ fo, const int32_t* __restrict__ fe,
           int32_t nf, int32_t ne, uint32_t* __restrict__ cnt, int* err)
 {
     const int64_t f = (int64_t)blockIdx.x * kB + threadIdx.x;
+    // the most sides of a face, where they are more than the 6 that 8 lanes a
+    // pair hold (pair_lanes_log2), in 64 words: one address would serialise the
+    // first wavefronts' updates
+    int* const most = err + 16 + (blockIdx.x & 63);
+    int sides = f < nf ? (int)(fo[f + 1] - fo[f]) : 0;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1)
+        sides = max(sides, __shfl_xor(sides, d));
+    if ((threadIdx.x & 63) == 0 && sides > 6 && sides > *most)
+        atomicMax(most, sides);
     if (f >= nf)
         return;
     for (int64_t i = fo[f]; i < fo[f + 1]; ++i)
@@ -314,102 +325,116 @@ struct Cx
     int* err;
 };
 
-__global__ void __launch_bounds__(kB) first_face(Cx C, Pairs P, int32_t np)
+// The kernels of a generation read its pair count from device memory and loop
+// over the pairs with the grid's stride, so that generations are launched
+// without waiting for the count (the grid follows the last count the host has
+// seen).  After an error every later kernel sees no pairs.
+__device__ __forceinline__ int32_t gen_pairs(const Cx& C, const uint32_t* np)
 {
-    const int32_t j = blockIdx.x * kB + threadIdx.x;
-    if (j >= np || !P.t[j])
-        return;
-    const int32_t f = P.c[j];
-    if (C.rg_f[f] < 0)
-        atomicMin(&C.first_f[f], j);
+    return *C.err ? 0 : (int32_t)*np;
+}
+#define VC_FOR_PAIRS(j, n)                                                    \
+    for (int32_t j = (int32_t)(blockIdx.x * kB + threadIdx.x); j < (n);       \
+         j += (int32_t)(gridDim.x * kB))
+
+// face-edge pairs compete for their face; also clears the push sums
+__global__ void __launch_bounds__(kB)
+    first_face(Cx C, Pairs P, const uint32_t* np, uint32_t* __restrict__ sup, int32_t nsup)
+{
+    VC_FOR_PAIRS(i, nsup) sup[i] = 0u;
+    const int32_t n = gen_pairs(C, np);
+    VC_FOR_PAIRS(j, n)
+    {
+        if (!P.t[j])
+            continue;
+        const int32_t f = P.c[j];
+        if (C.rg_f[f] < 0)
+            atomicMin(&C.first_f[f], j);
+    }
 }
 
 // face-edge pairs: effective iff first on their face; the effective ones and
-// the edge-vertex pairs compete for their edge; slot counts
+// the edge-vertex pairs compete for their edge
 __global__ void __launch_bounds__(kB)
-    first_edge(Cx C, Pairs P, int32_t np, uint8_t* __restrict__ eff,
-               uint32_t* __restrict__ slots)
+    first_edge(Cx C, Pairs P, const uint32_t* np, uint8_t* __restrict__ eff)
 {
-    const int32_t j = blockIdx.x * kB + threadIdx.x;
-    if (j >= np)
-        return;
-    if (P.t[j])
+    const int32_t n = gen_pairs(C, np);
+    VC_FOR_PAIRS(j, n)
     {
-        const int32_t f = P.c[j];
-        const bool e1 = C.rg_f[f] < 0 && C.first_f[f] == j;
-        eff[j] = e1 ? 1 : 0;
-        if (e1)
-            atomicMin(&C.first_e[P.o[j]], j);
-        slots[j] = (uint32_t)(C.fo[f + 1] - C.fo[f]) + 2u;
-    }
-    else
-    {
-        const int32_t e = P.c[j];
-        if (C.rg_e[e] < 0)
-            atomicMin(&C.first_e[e], j);
-        slots[j] = 1u;
+        const int32_t c = P.c[j];
+        if (P.t[j])
+        {
+            const bool e1 = C.rg_f[c] < 0 && C.first_f[c] == j;
+            eff[j] = e1 ? 1 : 0;
+            if (e1)
+                atomicMin(&C.first_e[P.o[j]], j);
+        }
+        else if (C.rg_e[c] < 0)
+            atomicMin(&C.first_e[c], j);
     }
 }
 
 __global__ void __launch_bounds__(kB)
-    decide(Cx C, Pairs P, int32_t np, uint8_t* __restrict__ eff)
+    decide(Cx C, Pairs P, const uint32_t* np, uint8_t* __restrict__ eff)
 {
-    const int32_t j = blockIdx.x * kB + threadIdx.x;
-    if (j >= np)
-        return;
-    if (P.t[j])
+    const int32_t n = gen_pairs(C, np);
+    VC_FOR_PAIRS(j, n)
     {
-        if (!eff[j])
-            return;
-        const int32_t e = P.o[j];
-        if (C.first_e[e] != j)
-            atomicMax(C.err, kErrTwice);
-        if (C.ref_e[e] != 1)
-            atomicMax(C.err, kErrLogic);
-    }
-    else
-    {
-        const int32_t e = P.c[j];
-        const bool e1 = C.rg_e[e] < 0 && C.first_e[e] == j;
-        eff[j] = e1 ? 1 : 0;
-        if (e1 && C.ref_v[P.o[j]] != 1)
-            atomicMax(C.err, kErrLogic);
+        if (P.t[j])
+        {
+            if (!eff[j])
+                continue;
+            const int32_t e = P.o[j];
+            if (C.first_e[e] != j)
+                atomicMax(C.err, kErrTwice);
+            if (C.ref_e[e] != 1)
+                atomicMax(C.err, kErrLogic);
+        }
+        else
+        {
+            const int32_t e = P.c[j];
+            const bool e1 = C.rg_e[e] < 0 && C.first_e[e] == j;
+            eff[j] = e1 ? 1 : 0;
+            if (e1 && C.ref_v[P.o[j]] != 1)
+                atomicMax(C.err, kErrLogic);
+        }
     }
 }
 
 __global__ void __launch_bounds__(kB)
-    apply(Cx C, Pairs P, int32_t np, const uint8_t* __restrict__ eff, int32_t g)
+    apply(Cx C, Pairs P, const uint32_t* np, const uint8_t* __restrict__ eff, int32_t g)
 {
-    const int32_t j = blockIdx.x * kB + threadIdx.x;
-    if (j >= np)
-        return;
-    if (P.t[j])
+    const int32_t n = gen_pairs(C, np);
+    VC_FOR_PAIRS(j, n)
     {
-        const int32_t f = P.c[j], e = P.o[j];
-        C.first_f[f] = INT_MAX;
-        C.first_e[e] = INT_MAX;
-        if (!eff[j])
-            return;
-        C.rg_f[f] = g;
-        C.rj_f[f] = j;
-        C.rg_e[e] = g;
-        C.rj_e[e] = j;
-        for (int64_t i = C.fo[f]; i < C.fo[f + 1]; ++i)
-            atomicSub(&C.ref_e[C.fe[i]], 1);
-        atomicSub(&C.ref_v[C.E[2 * e]], 1);
-        atomicSub(&C.ref_v[C.E[2 * e + 1]], 1);
-    }
-    else
-    {
-        const int32_t e = P.c[j], v = P.o[j];
-        C.first_e[e] = INT_MAX;
-        if (!eff[j])
-            return;
-        C.rg_e[e] = g;
-        C.rj_e[e] = j;
-        C.rm_v[v] = 1;
-        atomicSub(&C.ref_v[C.E[2 * e]], 1);
-        atomicSub(&C.ref_v[C.E[2 * e + 1]], 1);
+        if (P.t[j])
+        {
+            const int32_t f = P.c[j], e = P.o[j];
+            C.first_f[f] = INT_MAX;
+            C.first_e[e] = INT_MAX;
+            if (!eff[j])
+                continue;
+            C.rg_f[f] = g;
+            C.rj_f[f] = j;
+            C.rg_e[e] = g;
+            C.rj_e[e] = j;
+            for (int64_t i = C.fo[f]; i < C.fo[f + 1]; ++i)
+                atomicSub(&C.ref_e[C.fe[i]], 1);
+            atomicSub(&C.ref_v[C.E[2 * e]], 1);
+            atomicSub(&C.ref_v[C.E[2 * e + 1]], 1);
+        }
+        else
+        {
+            const int32_t e = P.c[j], v = P.o[j];
+            C.first_e[e] = INT_MAX;
+            if (!eff[j])
+                continue;
+            C.rg_e[e] = g;
+            C.rj_e[e] = j;
+            C.rm_v[v] = 1;
+            atomicSub(&C.ref_v[C.E[2 * e]], 1);
+            atomicSub(&C.ref_v[C.E[2 * e + 1]], 1);
+        }
     }
 }
 
@@ -438,128 +463,255 @@ __device__ __forceinline__ int64_t vert_event(const Cx& C, const Pairs& P,
     return mkkey(j, (C.fo[f + 1] - C.fo[f]) + (C.E[2 * e] == x ? 0 : 1));
 }
 
-// the event (j, s) of edge x: if it brings x's count to 1, push the
-// face-edge pair of the face left at that moment
-__device__ void edge_event(const Cx& C, const Pairs& P, int32_t g, int32_t x,
-                           int64_t K, float f_t, uint32_t slot,
-                           uint32_t* sflag, Pairs N)
+// The event K of element x with adjacent cells adj[lo .. hi): how many of them
+// this generation removed (n), how many before K (rank), and the first one left
+// after K.  One pass; the cells and their removal generations are read four at
+// a time, so that a list costs a quarter of its length in dependent loads.
+template <typename KeyOf>
+__device__ __forceinline__ int32_t event_scan(const int32_t* __restrict__ adj, uint32_t lo,
+                                              uint32_t hi, const int32_t* rg, int32_t g,
+                                              int64_t K, KeyOf key, int& n, int& rank)
 {
-    int n = 0, rank = 0;
-    for (uint32_t i = C.ef_off[x]; i < C.ef_off[x + 1]; ++i)
+    int32_t left = -1;
+    n = rank = 0;
+    for (uint32_t i = lo; i < hi; i += 4)
     {
-        const int32_t f = C.ef[i];
-        if (C.rg_f[f] != g)
-            continue;
-        ++n;
-        rank += mkkey(C.rj_f[f], side_pos(C, f, x)) < K ? 1 : 0;
+        int32_t c[4], r[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            c[q] = adj[min(i + q, hi - 1)];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            r[q] = rg[c[q]];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+        {
+            if (i + q >= hi)
+                continue;
+            bool there = r[q] < 0;
+            if (r[q] == g)
+            {
+                const int64_t k = key(c[q]);
+                ++n;
+                rank += k < K ? 1 : 0;
+                there = k > K;
+            }
+            if (there && left < 0)
+                left = c[q];
+        }
     }
+    return left;
+}
+
+// the event K of edge x: if it brings x's count to 1, the face left at that
+// moment, whose pair with x is pushed; else -1
+__device__ int32_t edge_event(const Cx& C, int32_t g, int32_t x, int64_t K, float f_t)
+{
+    int n, rank;
+    const int32_t f = event_scan(
+        C.ef, C.ef_off[x], C.ef_off[x + 1], C.rg_f, g, K,
+        [&](int32_t c) { return mkkey(C.rj_f[c], side_pos(C, c, x)); }, n, rank);
     const int r0 = C.ref_e[x] + n;
-    if (r0 < 2 || rank != r0 - 2)
-        return;
-    for (uint32_t i = C.ef_off[x]; i < C.ef_off[x + 1]; ++i)
-    {
-        const int32_t f = C.ef[i];
-        const int32_t rg = C.rg_f[f];
-        if (rg >= 0 && (rg != g || mkkey(C.rj_f[f], side_pos(C, f, x)) <= K))
-            continue;
-        if (C.fm[f] < f_t)
-        {
-            N.t[slot] = 1;
-            N.c[slot] = f;
-            N.o[slot] = x;
-            sflag[slot] = 1u;
-        }
-        return;
-    }
+    return r0 >= 2 && rank == r0 - 2 && f >= 0 && C.fm[f] < f_t ? f : -1;
 }
 
-__device__ void vert_event_push(const Cx& C, const Pairs& P, int32_t g,
-                                int32_t x, int64_t K, float l_t, uint32_t slot,
-                                uint32_t* sflag, Pairs N)
+// the event K of vertex x: the edge left when its count comes to 1, or -1
+__device__ int32_t vert_event_left(const Cx& C, const Pairs& P, int32_t g, int32_t x,
+                                   int64_t K, float l_t)
 {
-    int n = 0, rank = 0;
-    for (uint32_t i = C.ve_off[x]; i < C.ve_off[x + 1]; ++i)
-    {
-        const int32_t e = C.ve[i];
-        if (C.rg_e[e] != g)
-            continue;
-        ++n;
-        rank += vert_event(C, P, e, x) < K ? 1 : 0;
-    }
+    int n, rank;
+    const int32_t e = event_scan(
+        C.ve, C.ve_off[x], C.ve_off[x + 1], C.rg_e, g, K,
+        [&](int32_t c) { return vert_event(C, P, c, x); }, n, rank);
     const int r0 = C.ref_v[x] + n;
-    if (r0 < 2 || rank != r0 - 2)
-        return;
-    for (uint32_t i = C.ve_off[x]; i < C.ve_off[x + 1]; ++i)
-    {
-        const int32_t e = C.ve[i];
-        const int32_t rg = C.rg_e[e];
-        if (rg >= 0 && (rg != g || vert_event(C, P, e, x) <= K))
-            continue;
-        if (C.em[e] < l_t)
-        {
-            N.t[slot] = 0;
-            N.c[slot] = e;
-            N.o[slot] = x;
-            sflag[slot] = 1u;
-        }
-        return;
-    }
+    return r0 >= 2 && rank == r0 - 2 && e >= 0 && C.em[e] < l_t ? e : -1;
 }
 
-__global__ void __launch_bounds__(kB)
-    trigger(Cx C, Pairs P, int32_t np, const uint8_t* __restrict__ eff,
-            int32_t g, const uint32_t* __restrict__ slot_off, float f_t,
-            float l_t, uint32_t* __restrict__ sflag, Pairs N)
+// steps of an effective pair j: its sides then its edge's two ends, or the
+// edge's other end
+__device__ __forceinline__ int32_t pair_steps(const Cx& C, const Pairs& P, int32_t j)
 {
-    const int32_t j = blockIdx.x * kB + threadIdx.x;
-    if (j >= np || !eff[j])
-        return;
-    const uint32_t s0 = slot_off[j];
+    if (!P.t[j])
+        return 1;
+    const int32_t f = P.c[j];
+    return (int32_t)(C.fo[f + 1] - C.fo[f]) + 2;
+}
+
+// the push of step s of pair j; false if it pushes nothing
+__device__ bool pair_push(const Cx& C, const Pairs& P, int32_t g, int32_t j, int32_t s,
+                          int32_t steps, float f_t, float l_t, uint8_t& t, int32_t& c,
+                          int32_t& o)
+{
     if (P.t[j])
     {
         const int32_t f = P.c[j], e = P.o[j];
-        const int64_t L = C.fo[f + 1] - C.fo[f];
-        for (int64_t s = 0; s < L; ++s)
+        if (s < steps - 2)
         {
-            const int32_t x = C.fe[C.fo[f] + s];
-            if (x != e)
-                edge_event(C, P, g, x, mkkey(j, s), f_t, s0 + (uint32_t)s,
-                           sflag, N);
+            o = C.fe[C.fo[f] + s];
+            t = 1;
+            c = o != e ? edge_event(C, g, o, mkkey(j, s), f_t) : -1;
+            return c >= 0;
         }
-        for (int k = 0; k < 2; ++k)
-            vert_event_push(C, P, g, C.E[2 * e + k], mkkey(j, L + k), l_t,
-                            s0 + (uint32_t)(L + k), sflag, N);
+        o = C.E[2 * e + (s - (steps - 2))];
     }
     else
     {
-        const int32_t e = P.c[j], v = P.o[j];
-        const int32_t a = C.E[2 * e], b = C.E[2 * e + 1];
-        vert_event_push(C, P, g, a != v ? a : b, mkkey(j, 0), l_t, s0, sflag,
-                        N);
+        const int32_t e = P.c[j], v = P.o[j], a = C.E[2 * e];
+        o = a != v ? a : C.E[2 * e + 1];
+    }
+    t = 0;
+    c = vert_event_left(C, P, g, o, mkkey(j, s), l_t);
+    return c >= 0;
+}
+
+__device__ __forceinline__ uint32_t block_total(uint32_t v, uint32_t* red)
+{
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1)
+        v += __shfl_xor(v, d);
+    __syncthreads(); // red's last readers
+    if ((threadIdx.x & 63) == 0)
+        red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return red[0] + red[1] + red[2] + red[3];
+}
+
+// Pushes of a generation.  2^lsh lanes take the steps of a pair (one thread per
+// pair ran a pair's gathers one after the other: 66 us a generation on average
+// for the complex of a 96^3 volume; this count and the write below take 27 + 20
+// us and need neither slots nor their scan), a workgroup a chunk of
+// 256 >> lsh pairs.  Counts per pair, per chunk and per 256 chunks.
+__global__ void __launch_bounds__(kB)
+    push_count(Cx C, Pairs P, const uint32_t* np, const uint8_t* __restrict__ eff, int32_t g,
+               int lsh, float f_t, float l_t, uint32_t* __restrict__ cnt,
+               uint32_t* __restrict__ chunk, uint32_t* __restrict__ sup)
+{
+    __shared__ uint32_t red[4];
+    const int32_t n = gen_pairs(C, np);
+    const int lanes = 1 << lsh, ppb = kB >> lsh;
+    const int32_t nc = (n + ppb - 1) / ppb;
+    for (int32_t k = blockIdx.x; k < nc; k += gridDim.x)
+    {
+        const int32_t j = k * ppb + (int32_t)(threadIdx.x >> lsh);
+        uint32_t m = 0;
+        if (j < n && eff[j])
+        {
+            const int32_t steps = pair_steps(C, P, j);
+            for (int32_t s = threadIdx.x & (lanes - 1); s < steps; s += lanes)
+            {
+                uint8_t t;
+                int32_t c, o;
+                m += pair_push(C, P, g, j, s, steps, f_t, l_t, t, c, o) ? 1u : 0u;
+            }
+        }
+        uint32_t pm = m;
+        for (int d = lanes >> 1; d >= 1; d >>= 1)
+            pm += __shfl_xor(pm, d);
+        if (j < n && (threadIdx.x & (lanes - 1)) == 0)
+            cnt[j] = pm;
+        const uint32_t tot = block_total(m, red);
+        if (threadIdx.x == 0)
+        {
+            chunk[k] = tot;
+            if (tot)
+                atomicAdd(&sup[k >> 8], tot);
+        }
     }
 }
 
+// Writes them, evaluated again, each at the number of pushes before it, and
+// the next generation's count (to its word and, as tag << 32 | count or
+// all-ones after an error, to the host).
 __global__ void __launch_bounds__(kB)
-    compact(const uint32_t* __restrict__ pos, uint32_t ns,
-            const uint32_t* __restrict__ total, Pairs S, Pairs N)
+    push_write(Cx C, Pairs P, const uint32_t* np, const uint8_t* __restrict__ eff, int32_t g,
+               int lsh, float f_t, float l_t, const uint32_t* __restrict__ cnt,
+               const uint32_t* __restrict__ chunk, const uint32_t* __restrict__ sup, Pairs N,
+               uint32_t* np_out, unsigned long long* report, uint32_t tag)
 {
-    const int64_t i = (int64_t)blockIdx.x * kB + threadIdx.x;
-    if (i >= ns)
-        return;
-    const uint32_t next = i + 1 < ns ? pos[i + 1] : *total;
-    if (next == pos[i])
-        return;
-    const uint32_t k = pos[i];
-    N.t[k] = S.t[i];
-    N.c[k] = S.c[i];
-    N.o[k] = S.o[i];
+    __shared__ uint32_t red[4];
+    __shared__ uint32_t off[kB];
+    const int32_t n = gen_pairs(C, np);
+    const int lanes = 1 << lsh, ppb = kB >> lsh;
+    const int32_t nc = (n + ppb - 1) / ppb;
+    const int lane = threadIdx.x & 63, grp = (lane >> lsh) << lsh; // its pair's first lane
+    if (n == 0 && blockIdx.x == 0 && threadIdx.x == 0)
+    {
+        *np_out = 0;
+        __hip_atomic_store(report,
+                           (unsigned long long)tag << 32 | (*C.err ? 0xFFFFFFFFull : 0ull),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    for (int32_t k = blockIdx.x; k < nc; k += gridDim.x)
+    {
+        uint32_t before = 0;
+        if ((int32_t)threadIdx.x < (k & 255))
+            before = chunk[(k & ~255) + threadIdx.x];
+        for (int32_t q = threadIdx.x; q < k >> 8; q += kB)
+            before += sup[q];
+        const uint32_t base = block_total(before, red);
+        // pushes before each pair of the chunk
+        const int32_t j0 = k * ppb;
+        if (threadIdx.x < 64)
+        {
+            uint32_t run = base;
+            for (int q = lane; q < ppb; q += 64)
+            {
+                const uint32_t v = j0 + q < n ? cnt[j0 + q] : 0u;
+                uint32_t x = v;
+#pragma unroll
+                for (int d = 1; d < 64; d <<= 1)
+                {
+                    const uint32_t u = __shfl_up(x, d);
+                    if (lane >= d)
+                        x += u;
+                }
+                off[q] = run + x - v;
+                run += __shfl(x, 63);
+            }
+        }
+        __syncthreads();
+        const int32_t j = j0 + (int32_t)(threadIdx.x >> lsh);
+        const bool live = j < n && eff[j] && cnt[j];
+        const int32_t steps = live ? pair_steps(C, P, j) : 0;
+        uint32_t at = off[threadIdx.x >> lsh];
+        for (int32_t s = threadIdx.x & (lanes - 1);
+             __any(s < steps); s += lanes)
+        {
+            uint8_t t = 0;
+            int32_t c = 0, o = 0;
+            const bool push =
+                s < steps && pair_push(C, P, g, j, s, steps, f_t, l_t, t, c, o);
+            // this pair's lanes, from its first
+            uint64_t m = __ballot(push) >> grp;
+            if (lanes < 64)
+                m &= (1ull << lanes) - 1ull;
+            if (push)
+            {
+                const uint32_t w = at + (uint32_t)__popcll(m & ((1ull << (lane - grp)) - 1ull));
+                N.t[w] = t;
+                N.c[w] = c;
+                N.o[w] = o;
+            }
+            at += (uint32_t)__popcll(m);
+        }
+        if (k == nc - 1 && threadIdx.x == 0)
+        {
+            const uint32_t next = base + chunk[k];
+            *np_out = next;
+            __hip_atomic_store(report, (unsigned long long)tag << 32 | next, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        __syncthreads(); // off is rewritten by the next chunk
+    }
 }
 
-__global__ void __launch_bounds__(kB) fill_u32(uint32_t* a, int64_t n, uint32_t v)
+// the first generation's count (the end of the scanned flags)
+__global__ void gen_start(const uint32_t* flag_end, uint32_t* np, unsigned long long* report,
+                          uint32_t tag)
 {
-    const int64_t i = (int64_t)blockIdx.x * kB + threadIdx.x;
-    if (i < n)
-        a[i] = v;
+    *np = *flag_end;
+    __hip_atomic_store(report, (unsigned long long)tag << 32 | *flag_end, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 __global__ void __launch_bounds__(kB)
@@ -1075,12 +1227,13 @@ struct vc_cc
     int* err = nullptr;
     uint32_t* sums = nullptr;
     bool degenerate = false; // an edge with equal ends or a repeated side
+    int max_sides = 0;       // of a face
     Mem mem;
 };
 
 // the state of CellComplexThinning over one vc_cc: measures, counts, the
-// generation of every removal and the queue buffers (grown on demand and
-// kept across prune calls)
+// generation of every removal and the queue buffers (a generation's pairs are
+// at most the edges and vertices)
 struct vc_ccthin
 {
     vc_cc* cc = nullptr;
@@ -1092,12 +1245,10 @@ struct vc_ccthin
     uint8_t *rm_v = nullptr, *rm_e = nullptr, *rm_f = nullptr;
     uint32_t* qflag = nullptr;
     bool pruned = false;
-    size_t cap_p = 0, cap_s = 0;
-    Pairs P{}, N{}, SL{};
+    Pairs P{}, N{};
     uint8_t* eff = nullptr;
-    uint32_t *slot_off = nullptr, *sflag = nullptr;
+    uint32_t *cnt = nullptr, *chunk = nullptr, *sup = nullptr, *np = nullptr;
     Mem mem;
-    Mem grown;
 };
 
 namespace
@@ -1119,7 +1270,7 @@ int cc_adjacency(vc_ctx* ctx, vc_cc* c)
     get(c->mem, &c->ef_off, E + 1);
     get(c->mem, &c->ve, 2 * E);
     get(c->mem, &c->ef, (size_t)c->nfe + 1);
-    get(c->mem, &c->err, 4);
+    get(c->mem, &c->err, 80);
     get(c->mem, &c->sums, (size_t)kScanB + 1);
     get(tmp, &fillv, V);
     get(tmp, &fille, E);
@@ -1129,15 +1280,18 @@ int cc_adjacency(vc_ctx* ctx, vc_cc* c)
     VC_HIP(ctx, hipMemsetAsync(c->ef_off, 0, 4 * (E + 1), S));
     VC_HIP(ctx, hipMemsetAsync(fillv, 0, 4 * V, S));
     VC_HIP(ctx, hipMemsetAsync(fille, 0, 4 * E, S));
-    VC_HIP(ctx, hipMemsetAsync(c->err, 0, sizeof(int), S));
+    VC_HIP(ctx, hipMemsetAsync(c->err, 0, 80 * sizeof(int), S));
     if (c->ne)
         deg_v<<<nblk(c->ne), kB, 0, S>>>(c->E, c->ne, c->nv, c->ve_off, c->err);
     if (c->nf)
         deg_e<<<nblk(c->nf), kB, 0, S>>>(c->fo, c->fe, c->nf, c->ne, c->ef_off, c->err);
     VC_CHECK_LAUNCH(ctx);
-    int herr = 0;
-    if ((rc = read_err(ctx, c->err, &herr)) != VC_OK)
-        return rc;
+    int words[80] = {};
+    VC_HIP(ctx, hipMemcpyAsync(words, c->err, sizeof(words), hipMemcpyDeviceToHost, S));
+    VC_HIP(ctx, hipStreamSynchronize(S));
+    const int herr = words[0];
+    // (0: at most 6)
+    c->max_sides = *std::max_element(words + 16, words + 80);
     if (herr & kAdjRange)
         return vc_fail(ctx, VC_ERR_INVALID,
                        "cell complex: an edge end or a face side out of range");
@@ -1158,6 +1312,16 @@ int cc_adjacency(vc_ctx* ctx, vc_cc* c)
     // fillv / fille are freed on return
     VC_HIP(ctx, hipStreamSynchronize(S));
     return VC_OK;
+}
+
+// lanes per pair: a power of two that holds a face's sides and its edge's two
+// ends (8 for triangles and quads), at most a wavefront
+int pair_lanes_log2(int max_sides)
+{
+    int l = 3;
+    while (l < 6 && (1 << l) < max_sides + 2)
+        ++l;
+    return l;
 }
 
 int thin_alloc(vc_ctx* ctx, vc_ccthin* t)
@@ -1182,7 +1346,20 @@ int thin_alloc(vc_ctx* ctx, vc_ccthin* t)
     get(&t->rm_v, V);
     get(&t->rm_e, E);
     get(&t->rm_f, F);
-    get(&t->qflag, (size_t)c->ne + c->nv + 1);
+    const size_t Q = (size_t)c->ne + c->nv + 1;
+    get(&t->qflag, Q);
+    for (Pairs* p : {&t->P, &t->N})
+    {
+        get(&p->t, Q);
+        get(&p->c, Q);
+        get(&p->o, Q);
+    }
+    get(&t->eff, Q);
+    get(&t->cnt, Q);
+    const size_t chunks = Q / (size_t)(kB >> pair_lanes_log2(c->max_sides)) + 2;
+    get(&t->chunk, chunks);
+    get(&t->sup, chunks / 256 + 2);
+    get(&t->np, 2);
     if (rc != VC_OK)
         return rc;
     hipStream_t S = ctx->stream;
@@ -1191,68 +1368,31 @@ int thin_alloc(vc_ctx* ctx, vc_ccthin* t)
     return VC_OK;
 }
 
-// the pair buffers hold at least n pairs (the current ones are kept)
-int grow_pairs(vc_ctx* ctx, vc_ccthin* t, size_t n)
+// waits for the report with this tag; a stream that fails or runs dry without
+// it ends the wait
+int report_wait(vc_ctx* ctx, uint32_t tag, uint32_t* value)
 {
-    if (n <= t->cap_p)
-        return VC_OK;
-    hipStream_t S = ctx->stream;
-    const size_t c = n + n / 2 + 1024;
-    uint8_t *t1, *t2, *e1;
-    int32_t *c1, *o1, *c2, *o2;
-    uint32_t* s1;
-    int rc = VC_OK;
-    auto get = [&](auto** p, size_t k) {
-        if (rc == VC_OK)
-            rc = t->grown.get(ctx, p, k);
-    };
-    get(&t1, c);
-    get(&t2, c);
-    get(&e1, c);
-    get(&c1, c);
-    get(&o1, c);
-    get(&c2, c);
-    get(&o2, c);
-    get(&s1, c);
-    if (rc != VC_OK)
-        return rc;
-    if (t->cap_p)
+    const unsigned long long* w = ctx->h_prog + tag % VC_PROG;
+    bool idle = false;
+    for (uint32_t spin = 1;; ++spin)
     {
-        VC_HIP(ctx, hipMemcpyAsync(t1, t->P.t, t->cap_p, hipMemcpyDeviceToDevice, S));
-        VC_HIP(ctx, hipMemcpyAsync(c1, t->P.c, 4 * t->cap_p, hipMemcpyDeviceToDevice, S));
-        VC_HIP(ctx, hipMemcpyAsync(o1, t->P.o, 4 * t->cap_p, hipMemcpyDeviceToDevice, S));
+        const unsigned long long v = __atomic_load_n(w, __ATOMIC_ACQUIRE);
+        if ((uint32_t)(v >> 32) == tag)
+        {
+            *value = (uint32_t)v;
+            return VC_OK;
+        }
+        if (idle)
+            return vc_fail(ctx, VC_ERR_HIP, "collapse: a generation ran without a report");
+        __builtin_ia32_pause();
+        if (spin % 65536 == 0)
+        {
+            const hipError_t e = hipStreamQuery(ctx->stream);
+            if (e != hipSuccess && e != hipErrorNotReady)
+                return vc_fail(ctx, VC_ERR_HIP, "collapse: %s", hipGetErrorString(e));
+            idle = e == hipSuccess;
+        }
     }
-    t->P = Pairs{t1, c1, o1};
-    t->N = Pairs{t2, c2, o2};
-    t->eff = e1;
-    t->slot_off = s1;
-    t->cap_p = c;
-    return VC_OK;
-}
-
-int grow_slots(vc_ctx* ctx, vc_ccthin* t, size_t n)
-{
-    if (n <= t->cap_s)
-        return VC_OK;
-    const size_t c = n + n / 2 + 1024;
-    uint8_t* tt;
-    int32_t *cc, *oo;
-    uint32_t* fl;
-    int rc = VC_OK;
-    auto get = [&](auto** p, size_t k) {
-        if (rc == VC_OK)
-            rc = t->grown.get(ctx, p, k);
-    };
-    get(&tt, c);
-    get(&cc, c);
-    get(&oo, c);
-    get(&fl, c);
-    if (rc != VC_OK)
-        return rc;
-    t->SL = Pairs{tt, cc, oo};
-    t->sflag = fl;
-    t->cap_s = c;
-    return VC_OK;
 }
 
 // CellComplexThinning::prune(f_t, l_t) on the resident complex: every call
@@ -1311,63 +1451,62 @@ int thin_prune(vc_ctx* ctx, vc_ccthin* t, float f_t, float l_t, int64_t* gens)
     int rc = scan_any(ctx, qflag, nq + 1, c->sums);
     if (rc != VC_OK)
         return rc;
-    uint32_t np = 0;
-    VC_HIP(ctx, hipMemcpyAsync(&np, qflag + nq, 4, hipMemcpyDeviceToHost, S));
-    VC_HIP(ctx, hipStreamSynchronize(S));
-    if ((rc = grow_pairs(ctx, t, (size_t)np + 1)) != VC_OK)
-        return rc;
-    if (np)
+    if (nq)
         init_pairs<<<nblk(nq), kB, 0, S>>>(ne, nv, qflag, qflag + nq, c->ef_off,
                                             c->ef, c->ve_off, c->ve, t->P);
     VC_CHECK_LAUNCH(ctx);
 
-    int32_t g = 0;
-    while (np > 0 && rc == VC_OK)
+    // Generations are launched kAhead at a time ahead of the reports of their
+    // counts (a generation without pairs does nothing), so the device never
+    // waits for the host: with two waits and about 15 launches a generation,
+    // the complex of a 96^3 volume (43 generations) took 14.2 ms; 9.1 ms now.
+    constexpr int kAhead = 2;
+    const uint32_t tag0 = ctx->prog_epoch + 1;
+    gen_start<<<1, 1, 0, S>>>(qflag + nq, t->np, ctx->h_prog + tag0 % VC_PROG, tag0);
+    VC_CHECK_LAUNCH(ctx);
+    const int lsh = pair_lanes_log2(c->max_sides), ppb = kB >> lsh;
+    const int32_t nsup = (int32_t)((nq / ppb + 1) / 256 + 1);
+    int32_t launched = 0, g = 0;
+    int64_t last = nq; // the last count seen, which sizes the grids
+    for (;; ++g)
     {
-        const int32_t n = (int32_t)np;
-        first_face<<<nblk(n), kB, 0, S>>>(C, t->P, n);
-        first_edge<<<nblk(n), kB, 0, S>>>(C, t->P, n, t->eff, t->slot_off);
-        decide<<<nblk(n), kB, 0, S>>>(C, t->P, n, t->eff);
-        VC_CHECK_LAUNCH(ctx);
-        VC_HIP(ctx, hipMemsetAsync(t->slot_off + n, 0, 4, S));
-        if ((rc = scan_any(ctx, t->slot_off, (int64_t)n + 1, c->sums)) != VC_OK)
-            break;
-        uint32_t hs[2] = {0, 0};
-        VC_HIP(ctx, hipMemcpyAsync(&hs[0], t->slot_off + n, 4, hipMemcpyDeviceToHost, S));
-        VC_HIP(ctx, hipMemcpyAsync(&hs[1], c->err, 4, hipMemcpyDeviceToHost, S));
-        VC_HIP(ctx, hipStreamSynchronize(S));
-        if (hs[1])
+        for (; launched <= g + kAhead - 1; ++launched)
         {
-            rc = vc_fail(ctx, VC_ERR_STATE,
-                         hs[1] == kErrLogic
-                             ? "collapse: a popped pair's count is not 1 (logic err)"
-                             : "collapse: an edge removed twice in one generation");
-            break;
+            const uint32_t* np = t->np + (launched & 1);
+            uint32_t* np_out = t->np + ((launched + 1) & 1);
+            const uint32_t tag = tag0 + 1 + (uint32_t)launched;
+            const unsigned gp = (unsigned)std::min<int64_t>(nblk(last) + 1, 2048);
+            const unsigned gc = (unsigned)std::min<int64_t>(last / ppb + 1, 4096);
+            first_face<<<gp, kB, 0, S>>>(C, t->P, np, t->sup, nsup);
+            first_edge<<<gp, kB, 0, S>>>(C, t->P, np, t->eff);
+            decide<<<gp, kB, 0, S>>>(C, t->P, np, t->eff);
+            apply<<<gp, kB, 0, S>>>(C, t->P, np, t->eff, launched);
+            push_count<<<gc, kB, 0, S>>>(C, t->P, np, t->eff, launched, lsh, f_t, l_t, t->cnt,
+                                          t->chunk, t->sup);
+            push_write<<<gc, kB, 0, S>>>(C, t->P, np, t->eff, launched, lsh, f_t, l_t, t->cnt,
+                                          t->chunk, t->sup, t->N, np_out,
+                                          ctx->h_prog + tag % VC_PROG, tag);
+            ctx->prog_epoch = tag;
+            VC_CHECK_LAUNCH(ctx);
+            std::swap(t->P, t->N);
         }
-        const uint32_t ns = hs[0];
-        if ((rc = grow_slots(ctx, t, (size_t)ns + 1)) != VC_OK)
+        uint32_t np = 0; // of generation g
+        if ((rc = report_wait(ctx, tag0 + (uint32_t)g, &np)) != VC_OK)
+            return rc;
+        if (np == 0xFFFFFFFFu)
+        {
+            int herr = 0;
+            if ((rc = read_err(ctx, c->err, &herr)) != VC_OK)
+                return rc;
+            return vc_fail(ctx, VC_ERR_STATE,
+                           herr == kErrLogic
+                               ? "collapse: a popped pair's count is not 1 (logic err)"
+                               : "collapse: an edge removed twice in one generation");
+        }
+        if (np == 0)
             break;
-        apply<<<nblk(n), kB, 0, S>>>(C, t->P, n, t->eff, g);
-        fill_u32<<<nblk((int64_t)ns + 1), kB, 0, S>>>(t->sflag, (int64_t)ns + 1, 0u);
-        trigger<<<nblk(n), kB, 0, S>>>(C, t->P, n, t->eff, g, t->slot_off, f_t, l_t,
-                                         t->sflag, t->SL);
-        VC_CHECK_LAUNCH(ctx);
-        if ((rc = scan_any(ctx, t->sflag, (int64_t)ns + 1, c->sums)) != VC_OK)
-            break;
-        uint32_t nn = 0;
-        VC_HIP(ctx, hipMemcpyAsync(&nn, t->sflag + ns, 4, hipMemcpyDeviceToHost, S));
-        VC_HIP(ctx, hipStreamSynchronize(S));
-        if ((rc = grow_pairs(ctx, t, (size_t)nn + 1)) != VC_OK)
-            break;
-        if (nn)
-            compact<<<nblk(ns), kB, 0, S>>>(t->sflag, ns, t->sflag + ns, t->SL, t->N);
-        VC_CHECK_LAUNCH(ctx);
-        std::swap(t->P, t->N);
-        np = nn;
-        ++g;
+        last = np;
     }
-    if (rc != VC_OK)
-        return rc;
     const int32_t me = ne > nf ? ne : nf;
     if (me)
         results<<<nblk(me), kB, 0, S>>>(ne, nf, t->rg_e, t->rg_f, t->rm_e, t->rm_f);

@@ -276,7 +276,7 @@ int vc_ctx_create(int device, vc_ctx** out)
          hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming) != hipSuccess ||
          hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming) != hipSuccess))
         rc = VC_ERR_HIP;
-    if (rc == VC_OK && hipHostMalloc((void**)&ctx->h_prog, sizeof(*ctx->h_prog),
+    if (rc == VC_OK && hipHostMalloc((void**)&ctx->h_prog, VC_PROG * sizeof(*ctx->h_prog),
                                      hipHostMallocMapped | hipHostMallocCoherent) !=
                            hipSuccess)
     {
@@ -285,7 +285,7 @@ int vc_ctx_create(int device, vc_ctx** out)
     }
     if (rc == VC_OK)
     {
-        *ctx->h_prog = 0;
+        std::memset(ctx->h_prog, 0, VC_PROG * sizeof(*ctx->h_prog));
         rc = vc_lut_build(ctx);
     }
     if (rc == VC_OK)

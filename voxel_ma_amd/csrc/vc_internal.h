@@ -71,8 +71,10 @@ struct vc_ctx
     std::vector<hipEvent_t> ev_free;                         // reusable
     std::vector<std::pair<hipEvent_t, hipEvent_t>> ev_open;  // not yet read
     std::vector<int> ev_open_n;                              // launches per pair
-    // the word (pinned, coherent host memory) in which a tile sweep reports
-    // the sweep before it, and the level it belongs to (vc_thin.hip)
+    // words (pinned, coherent host memory) in which kernels report to a host
+    // that does not wait for the stream: tag << 32 | value.  Tags are unique
+    // in the context.  Word 0: tile sweeps (vc_thin.hip); word tag % VC_PROG:
+    // collapse generations (vc_ccthin_dev.hip)
     unsigned long long* h_prog = nullptr;
     uint32_t prog_epoch = 0;
     // vc_skeleton_noalloc: this device's scratch array (device address) and
@@ -238,6 +240,8 @@ struct vc_work
 // and the convergence is checked by copying the ring (dense passes, graphs,
 // timed sweeps)
 constexpr int VC_SEG_MIN = 4, VC_SEG_MAX = 16;
+// report words of a context (vc_ctx::h_prog)
+constexpr int VC_PROG = 8;
 // ring of per-sweep "removed anything" flags
 constexpr int VC_RING = 64;
 // stats counters: kSlots cache lines of [0] tests, [8 + k] removed at level k
