@@ -129,3 +129,37 @@ def test_edt_thick_solids(vc, oracle):
     cases["holes"] = holes
     for name, occ in cases.items():
         _check(vc, oracle, occ, "thick " + name)
+
+
+@pytest.mark.parametrize("n", [7, 8, 9, 15, 16, 63, 64, 65, 128, 135, 511, 512, 513])
+def test_edt_thick_columns_of_every_length(vc, n):
+    """Divide and conquer over columns of n rows (blocks of 8^k rows, a top level
+    of one row from 8^k to 2 8^k - 1): every tile is flagged, since the few
+    background voxels are far along z and from most voxels.  The answer is the
+    nearest of those, the lowest index among equals."""
+    import voxel_ma_amd as V
+    from conftest import say
+    rng = np.random.default_rng(n)
+    for axis in (0, 1):
+        shape = [3, 3, 330]
+        shape[axis] = n
+        for few in (1, 2, 5):
+            occ = np.ones(shape, np.uint8)
+            at = np.stack([rng.integers(0, m, few) for m in shape[:2]] +
+                          [rng.choice([0, 1, 328, 329], few)], 1)
+            if few > 2:  # equal distances across the column's middle
+                at[:2] = 0
+                at[1, axis] = n - 1
+            occ[tuple(at.T)] = 0
+            at = np.argwhere(occ == 0)  # in index order
+            g = np.indices(shape)
+            d = np.stack([sum((g[a] - p[a]) ** 2 for a in range(3)) for p in at])
+            k = d.argmin(0)  # the first of equals
+            say("thick column", shape, few)
+            vol = vc.upload(occ)
+            for _ in range(2):  # the flags are cleared and set again
+                vol.edt()
+                assert np.array_equal(vol.get(V.BUF_EDT), d.min(0))
+                assert np.array_equal(vol.get(V.BUF_FT),
+                                      np.ravel_multi_index(at.T, shape)[k])
+            vol.release()

@@ -35,16 +35,23 @@ constexpr int kInf = 0x7FFFFFFF;
 // distance of the voxel's own staged candidate (its cost bounds the best),
 // which the previous pass knows: pass z flags the y-pass tiles holding a
 // voxel more than kDeepY from the background along z (or with none in its
-// row), pass y the x-pass tiles holding a voxel whose (y, z) cost exceeds
-// kDeepX^2 (or has none).  A flagged tile is computed by divide and conquer
-// (column_argmins), whose work does not grow with the distance, and clears
-// its flag; the others run the outward search.  Either way the result is the
-// leftmost minimiser, so a stale flag costs time, never correctness.  On the
-// 512^3 blurred-noise volume no tile is flagged (its longest z run of inside
-// voxels has a half-length below 128; at a y threshold of 64, 13 % of the
-// y-pass tiles were, and the EDT took 1.44 instead of 1.26 ms); in a ball of
-// radius 250 most are (EDT 10.2 -> 4.1 ms).
-constexpr int kDeepY = 128, kDeepX = 48;
+// row), or more than kDeepYs in one of every kDeepRows rows; pass y the x-pass
+// tiles holding a voxel whose (y, z) cost exceeds kDeepX^2 (or has none).  A
+// flagged tile is computed by divide and conquer (column_argmins), whose work
+// does not grow with the distance, and clears its flag; the others run the
+// outward search.  Either way the result is the leftmost minimiser, so a stale
+// flag costs time, never correctness.
+//
+// The lines: divide and conquer costs about as much as searches of 40-50
+// distances throughout a tile.  One deep voxel does not make a tile slow, many
+// rows with them do, and the sampled rows tell the two apart: with kDeepY = 64
+// for every voxel, 13 % of the y-pass tiles of the 512^3 blurred-noise volume
+// were flagged and its EDT took 15 % longer; with 128 alone the tiles of a
+// 512^3 ball of radius 250 that lie 64-128 deep were not (y pass 2.08 ms; 1.32
+// with the samples, the noise volume's EDT 1.25 and 1.23 ms).  Sampled at 32,
+// 48, 96: noise 1.44-1.62, 1.30-1.43, 1.23 ms, ball 2.53, 2.54, 2.90 ms against
+// 1.26 and 2.68 (all before the single-row top level below).
+constexpr int kDeepY = 128, kDeepX = 48, kDeepYs = 64, kDeepRows = 64;
 
 // rows along z: vc_ez_lanes(nz) lanes per row and 8 voxels per lane and
 // access, whatever nz is (one load, a background byte by SWAR zero-byte
@@ -140,7 +147,7 @@ __global__ void __launch_bounds__(kBlock)
                         }
                     }
                 uint32_t packed[4];
-                bool deep = false;
+                int far = 0; // most steps to the background, rows without one apart
 #pragma unroll
                 for (int j = 0; j < 8; ++j)
                 {
@@ -155,7 +162,7 @@ __global__ void __launch_bounds__(kBlock)
                         const int L = below ? z0 + 31 - __clz(below) : Lb;
                         const int R = above ? z0 + __ffs(above) - 1 : Rb;
                         res = L < 0 ? R : (R < 0 ? L : (z - L <= R - z ? L : R));
-                        deep = deep || res < 0 || abs(z - res) > kDeepY;
+                        far = max(far, res < 0 ? kDeepY + 1 : abs(z - res));
                     }
                     if (j & 1)
                         packed[j >> 1] |= (uint32_t)(uint16_t)res << 16;
@@ -164,7 +171,8 @@ __global__ void __launch_bounds__(kBlock)
                 }
                 // (a flag too many, past the row's end or in a narrower tile,
                 // costs time only)
-                if (deep)
+                if (far > kDeepYs &&
+                    (far > kDeepY || (row % (uint32_t)d.ny) % kDeepRows == kDeepRows / 2))
                     for (int z = z0; z < min(z0 + 8, nz); z += d.tzy)
                         d.fy[(int64_t)(row / (uint32_t)d.ny) * ((nz + d.tzy - 1) / d.tzy) +
                              z / d.tzy] = 1;
@@ -193,11 +201,12 @@ constexpr int kNoBg = 1 << 30;
 
 // Leftmost minimum over an aligned group of G lanes (G a power of two, at
 // most 64): the smallest cost, then the smallest index; index -1 = none.
-__device__ __forceinline__ void group_min(int& c, int& q, int G)
+__device__ __forceinline__ void group_min(uint32_t& c, int& q, int G)
 {
     for (int d = 1; d < G; d <<= 1)
     {
-        const int oc = __shfl_xor(c, d), oq = __shfl_xor(q, d);
+        const uint32_t oc = __shfl_xor(c, d);
+        const int oq = __shfl_xor(q, d);
         if (oq >= 0 && (q < 0 || oc < c || (oc == c && oq < q)))
         {
             c = oc;
@@ -209,78 +218,112 @@ __device__ __forceinline__ void group_min(int& c, int& q, int G)
 // Leftmost argmin A(y) of cost(y, q) = f(q) + (y - q)^2 over q in [0, n),
 // for every y in [0, n) of the tile's columns c < ncol, by divide and
 // conquer: cost is a Monge array ((y' - y)(q' - q) >= 0 orders the cross
-// terms), so A is non-decreasing in y and A(mid) of a segment lies between
-// the A of the segment's two bounding rows.  Rows are the nodes of the
-// perfect binary tree over [0, 2^L - 1): level l holds 2^l nodes, node j has
-// mid ((2j+1) << (L-1-l)) - 1 and bounding rows (j << (L-l)) - 1 and
-// ((j+1) << (L-l)) - 1, mids of earlier levels (or outside [0, n)).  Each
-// level spreads its (column, node) tasks over the workgroup, G lanes per
-// task while tasks are fewer than lanes; about n log2 n cost evaluations per
-// column.  A column without a finite cost gets -1 everywhere.
-//   cost(c, y, q): the cost, >= lim when q has no background;
+// terms), so A is non-decreasing in y and rows between two rows whose A is
+// known search only between those.  A level of step s = 8^k takes the blocks of
+// 8 s rows: the block's 7 rows (b 8 s + (i + 1) s - 1) search together, each
+// candidate read once for all seven, between the A of the rows before and at the
+// block's end (from the levels above; the whole column where there is none).
+// One task per (column, block), G lanes per task while tasks are fewer than
+// lanes.  A column without a finite cost gets -1 everywhere.
+//
+// Seven rows per candidate: 5 instructions a cost instead of about 12 (the read
+// and the loop are shared), and a 512-row column takes 4 levels with a barrier
+// and their dependent reads instead of 10, for up to 3.5 times the costs: with the
+// flags above, the EDT of a 512^3 ball of radius 250 takes 2.46 ms instead of 3.90
+// (x pass 1.50 -> 1.00 ms).  Searching the widest ranges with a whole wavefront,
+// one after the other, was slower at every threshold tried (8 to 96).
+//   load(c, q): f(q), >= lim (and below 2^32 - n^2) when q has no background;
 //   put(c, y, q, cost): the result of row y (q = -1: none), to global memory;
 //   get(c, y): A(y) of a row put at an earlier level (-1: none), read back
 //   after the level's barrier (global writes of a workgroup are visible to
 //   the workgroup after __syncthreads).
 // Every lane of the workgroup must call it (barriers, shuffles).
-template <class Cost, class Put, class Get>
-__device__ void column_argmins(int n, int ncol, int TZ, int lim, Cost cost,
+// One level of step 1 << sh, with R rows a block (7, or the top's only one).
+template <int R, class Load, class Put, class Get>
+__device__ __forceinline__ void argmin_level(int sh, int n, int ncol, int TZ, uint32_t lim,
+                                             Load load, Put put, Get get)
+{
+    const int nthr = (int)blockDim.x;
+    const int ntask = TZ * ((n + (8 << sh) - 1) >> (sh + 3));
+    int gl = 0;
+    while (gl < 6 && (ntask << (gl + 1)) <= nthr)
+        ++gl;
+    const int G = 1 << gl, ngroups = nthr >> gl;
+    const int sub = (int)threadIdx.x & (G - 1);
+    const int trips = (ntask + ngroups - 1) / ngroups;
+    for (int it = 0; it < trips; ++it)
+    {
+        const int task = it * ngroups + ((int)threadIdx.x >> gl);
+        const int c = task % TZ, b = task / TZ;
+        const int yb = b << (sh + 3), y0 = yb + (1 << sh) - 1;
+        const bool active = task < ntask && c < ncol && y0 < n;
+        uint32_t bc[R];
+        int bq[R];
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+        {
+            bc[i] = lim;
+            bq[i] = -1;
+        }
+        if (active)
+        {
+            const int yr = yb + (8 << sh) - 1;
+            int qlo = 0, qhi = n - 1;
+            bool none = false;
+            if (yb > 0)
+            {
+                const int a = get(c, yb - 1);
+                none = a < 0;
+                qlo = a;
+            }
+            if (yr < n)
+            {
+                const int a = get(c, yr);
+                none = none || a < 0;
+                qhi = a;
+            }
+            if (!none)
+                for (int q = qlo + sub; q <= qhi; q += G)
+                {
+                    const uint32_t f = load(c, q);
+                    int d = y0 - q;
+#pragma unroll
+                    for (int i = 0; i < R; ++i)
+                    {
+                        const uint32_t v = f + (uint32_t)__mul24(d, d);
+                        const bool t = v < bc[i];
+                        bc[i] = t ? v : bc[i];
+                        bq[i] = t ? q : bq[i];
+                        d += 1 << sh;
+                    }
+                }
+        }
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+            group_min(bc[i], bq[i], G);
+        if (active && sub == 0)
+#pragma unroll
+            for (int i = 0; i < R; ++i)
+                if (y0 + (i << sh) < n)
+                    put(c, y0 + (i << sh), bq[i], bc[i]);
+    }
+    __syncthreads(); // this level's rows are read by the next
+}
+
+template <class Load, class Put, class Get>
+__device__ void column_argmins(int n, int ncol, int TZ, uint32_t lim, Load load,
                                Put put, Get get)
 {
-    int L = 1;
-    while ((1 << L) - 1 < n)
-        ++L;
-    const int nthr = (int)blockDim.x;
-    for (int l = 0; l < L; ++l)
+    int sh = 0;
+    while ((8 << sh) <= n)
+        sh += 3;
+    if (n >> sh == 1) // a length of 8^k .. 2 8^k - 1: one row at the top
     {
-        const int ntask = TZ << l;
-        int gl = 0;
-        while (gl < 6 && (ntask << (gl + 1)) <= nthr)
-            ++gl;
-        const int G = 1 << gl, ngroups = nthr >> gl;
-        const int sub = (int)threadIdx.x & (G - 1);
-        const int trips = (ntask + ngroups - 1) / ngroups;
-        for (int it = 0; it < trips; ++it)
-        {
-            const int task = it * ngroups + ((int)threadIdx.x >> gl);
-            const int c = task % TZ, j = task / TZ;
-            const int mid = ((2 * j + 1) << (L - 1 - l)) - 1;
-            const bool active = task < ntask && c < ncol && mid < n;
-            int bc = lim, bq = -1;
-            if (active)
-            {
-                const int yl = (j << (L - l)) - 1, yr = ((j + 1) << (L - l)) - 1;
-                int qlo = 0, qhi = n - 1;
-                bool none = false;
-                if (yl >= 0)
-                {
-                    const int a = get(c, yl);
-                    none = a < 0;
-                    qlo = a;
-                }
-                if (yr < n)
-                {
-                    const int a = get(c, yr);
-                    none = none || a < 0;
-                    qhi = a;
-                }
-                if (!none)
-                    for (int q = qlo + sub; q <= qhi; q += G)
-                    {
-                        const int v = cost(c, mid, q);
-                        if (v < bc)
-                        {
-                            bc = v;
-                            bq = q;
-                        }
-                    }
-            }
-            group_min(bc, bq, G);
-            if (active && sub == 0)
-                put(c, mid, bq, bc);
-        }
-        __syncthreads(); // this level's rows are read by the next
+        argmin_level<1>(sh, n, ncol, TZ, lim, load, put, get);
+        sh -= 3;
     }
+    for (; sh >= 0; sh -= 3)
+        argmin_level<7>(sh, n, ncol, TZ, lim, load, put, get);
 }
 
 
@@ -356,31 +399,31 @@ __global__ void __launch_bounds__(kBlock) edt_pass_y(vc_work W)
             if (kM)
                 column_argmins(
                     ny, ncol, TZ, kNoBg,
-                    [&](int c, int y, int q) -> int {
+                    [&](int c, int q) -> uint32_t {
                         const int e = colz[q * SY + c];
-                        return __mul24(e, e) + (y - q) * (y - q);
+                        return (uint32_t)__mul24(e, e);
                     },
-                    [&](int c, int y, int q, int v) {
+                    [&](int c, int y, int q, uint32_t v) {
                         ftc[(int64_t)y * nz + c] =
                             q < 0 ? VC_NONE
                                   : ((uint32_t)q << 16) |
                                         (uint32_t)(uint16_t)(z0 + c - colz[q * SY + c]);
-                        flag_x(y, z0 + c, q < 0, v);
+                        flag_x(y, z0 + c, q < 0, (int)v);
                     },
                     get);
             else
                 column_argmins(
                     ny, ncol, TZ, kInf,
-                    [&](int c, int y, int q) -> int {
+                    [&](int c, int q) -> uint32_t {
                         const int e = colz[q * SY + c];
-                        return e < 0 ? kInf
-                                     : (z0 + c - e) * (z0 + c - e) + (y - q) * (y - q);
+                        return e < 0 ? (uint32_t)kInf
+                                     : (uint32_t)((z0 + c - e) * (z0 + c - e));
                     },
-                    [&](int c, int y, int q, int v) {
+                    [&](int c, int y, int q, uint32_t v) {
                         ftc[(int64_t)y * nz + c] =
                             q < 0 ? VC_NONE
                                   : ((uint32_t)q << 16) | (uint32_t)(uint16_t)colz[q * SY + c];
-                        flag_x(y, z0 + c, q < 0, v);
+                        flag_x(y, z0 + c, q < 0, (int)v);
                     },
                     get);
             if (threadIdx.x == 0)
@@ -577,10 +620,10 @@ __global__ void __launch_bounds__(kBlock) edt_pass_x(vc_work W)
             uint32_t* ftc = ft + (int64_t)y * nz + z0;
             column_argmins(
                 nx, ncol, TZ, kInf,
-                [&](int c, int xx, int q) -> int {
-                    return dot_cost(colyz[q * TZ + c], (xx - q) * (xx - q));
+                [&](int c, int q) -> uint32_t {
+                    return (uint32_t)dot_cost(colyz[q * TZ + c], 0);
                 },
-                [&](int c, int xx, int q, int v) {
+                [&](int c, int xx, int q, uint32_t v) {
                     const int64_t o = (int64_t)xx * sx + (int64_t)y * nz + z0 + c;
                     if (q < 0)
                     {
