@@ -70,3 +70,28 @@ def test_reused_blocks(oracle, threads):
     for t in ts:
         t.join()
     assert not wrong
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (3, 5, 7), (4, 4, 16), (17, 19, 23), (64, 64, 65),
+                                   (160, 330, 330)])
+def test_results_into_caller_memory(vc, shape):
+    """vc_get_device against vc_get for every buffer, small (copied by a kernel)
+    and large, and into memory at odd offsets of the caller's."""
+    rng = np.random.default_rng(5)
+    occ = (rng.random(shape) < 0.7).astype(np.uint8)
+    vol = vc.upload(occ)
+    vol.edt().measure().thin_levels([1.0, 2.0], stats=False)
+    N = occ.size
+    for which in (V.BUF_OCC, V.BUF_EDT, V.BUF_FT, V.BUF_LAM2, V.BUF_LABEL, V.BUF_LEVEL):
+        ref = vol.get(which)
+        step = ref.itemsize
+        for off in (0, step, 3 * step):
+            buf = V.DeviceBuffer.from_array(np.full(N * step + 8 * step, 0xA5, np.uint8))
+            say("into caller memory", shape, which, off)
+            vol.get_device(which, buf.ptr + off, N * step)
+            vc.synchronize()
+            out = buf.download(np.uint8, N * step + 8 * step)
+            buf.free()
+            assert np.array_equal(out[off:off + N * step], ref.reshape(-1).view(np.uint8))
+            assert (out[:off] == 0xA5).all() and (out[off + N * step:] == 0xA5).all()
+    vol.release()

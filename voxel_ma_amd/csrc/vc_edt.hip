@@ -855,22 +855,27 @@ __global__ void __launch_bounds__(64 * kMeasWaves) measure_lam2(vc_work W)
     }
 }
 
+// packed features as linear indices (below 2^31), four per thread and access
+// (one per thread took 303 us for 512^3, 170 us now: 6.3 TB/s)
 __global__ void __launch_bounds__(kBlock)
     ft_linear(const uint32_t* __restrict__ ft, int32_t* __restrict__ out,
-              int ny, int nz, int64_t N, vc_pack pk)
+              uint32_t ny, uint32_t nz, uint32_t N, vc_pack pk)
 {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N)
-        return;
-    const uint32_t f = ft[i];
-    if (f == VC_NONE)
+    auto lin = [&](uint32_t f) -> int32_t {
+        int x, y, z;
+        vc_unpack_xyz(pk, f, x, y, z);
+        return f == VC_NONE ? -1
+                            : (int32_t)(((uint32_t)x * ny + (uint32_t)y) * nz + (uint32_t)z);
+    };
+    const uint32_t i = 4u * (blockIdx.x * kBlock + threadIdx.x);
+    if (i + 4u <= N)
     {
-        out[i] = -1;
-        return;
+        const uint4 f = *reinterpret_cast<const uint4*>(ft + i);
+        vc_stu(out + i, make_int4(lin(f.x), lin(f.y), lin(f.z), lin(f.w)));
     }
-    int x, y, z;
-    vc_unpack_xyz(pk, f, x, y, z);
-    out[i] = (int32_t)(((int64_t)x * ny + y) * nz + z);
+    else
+        for (uint32_t j = i; j < N; ++j)
+            out[j] = lin(ft[j]);
 }
 
 } // namespace
@@ -971,9 +976,9 @@ int vc_measure_sched(vc_ctx* ctx, vc_sched* s)
 
 int vc_ft_to_linear(vc_ctx* ctx, vc_vol* v, int32_t* dst)
 {
-    unsigned blocks = (unsigned)((v->N + kBlock - 1) / kBlock);
-    ft_linear<<<blocks, kBlock, 0, ctx->stream>>>(v->ft, dst, v->ny, v->nz,
-                                                  v->N, v->pk);
+    const unsigned blocks = (unsigned)((v->N + 4 * kBlock - 1) / (4 * kBlock));
+    ft_linear<<<blocks, kBlock, 0, ctx->stream>>>(v->ft, dst, (uint32_t)v->ny, (uint32_t)v->nz,
+                                                  (uint32_t)v->N, v->pk);
     VC_CHECK_LAUNCH(ctx);
     return VC_OK;
 }
