@@ -116,6 +116,30 @@ def test_batch_every_schedule_same_result(vc, ragged, sched):
         m.release()
 
 
+@pytest.mark.parametrize("over", [0, 1])
+def test_tile_sweep_few_and_many_tiles(vc, oracle, over):
+    """Batches of exactly two tiles per CU and of more: the tile sweep has a form
+    for either side.  Tiles of every cut (8 per volume, most of them partial)."""
+    cus = 256
+    rng = np.random.default_rng(23)
+    shapes = [(33, 34, 65), (47, 64, 128), (64, 33, 67)]  # 2 x 2 x 2 tiles
+    vols = [(rng.random(s) < p).astype(np.uint8) for s, p in zip(shapes, (0.9, 0.97, 0.8))]
+    levels = np.array([_levels_for(o) for o in vols], np.float32)
+    ref = [_oracle_all(oracle, o, list(map(float, lv))) for o, lv in zip(vols, levels)]
+    pick = [i % 3 for i in range(2 * cus // 8 + over)]
+    say("tiles", 8 * len(pick), "on", cus, "CUs")
+    members = [vc.upload(vols[i]) for i in pick]
+    b = V.Batch(vc, members)
+    st = b.run(levels[pick])
+    for m, i in zip(members, pick):
+        assert np.array_equal(m.get(V.BUF_LABEL), ref[i][3]), (shapes[i], over)
+    for k in range(levels.shape[1]):
+        assert st.removed[k] == sum(ref[i][4].removed[k] for i in pick)
+    b.release()
+    for m in members:
+        m.release()
+
+
 def test_batch_graph_replays(vc, ragged):
     """A captured segment is replayed many times, with eager work (another
     volume's thinning, host syncs) between calls; every replay must equal the

@@ -259,6 +259,7 @@ struct vc_sched
     uint32_t total[VK_COUNT] = {};
     size_t lds[VK_COUNT] = {};
     int64_t voxels = 0, words = 0;
+    bool few_tiles = false; // tile sweeps with at most two workgroups per CU
     vc_schedule sc{};
     // per-volume level thresholds, n x VC_MAX_LEVELS each
     uint64_t* d_T = nullptr;

@@ -239,6 +239,7 @@ int vc_sched_apply(vc_ctx* ctx, vc_sched* s, const vc_schedule& sc)
         VC_HIP(ctx, hipMemcpy(s->d_items[k], tab.data(), 8 * tab.size(),
                               hipMemcpyHostToDevice));
     }
+    s->few_tiles = s->total[VK_TT] <= 2u * (uint32_t)std::max(ctx->cu_count, 1);
     return upload_desc(ctx, s);
 }
 

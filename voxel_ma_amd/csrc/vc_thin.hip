@@ -908,22 +908,20 @@ __device__ __forceinline__ uint32_t halo_nbrs(int x, int y, int z)
     return ((xs & 1u) ? yz : 0u) | ((xs & 2u) ? yz << 9 : 0u) |
            ((xs & 4u) ? yz << 18 : 0u);
 }
-#ifndef VC_TILE_BLOCK
-#define VC_TILE_BLOCK 512
-#endif
-constexpr int kTBlock = VC_TILE_BLOCK; // threads of a tile-sweep workgroup
-#ifndef VC_TILE_WAVES
-#define VC_TILE_WAVES 8
-#endif
-// waves per SIMD the tile sweep is compiled for (4 workgroups of 512 per CU,
-// which its 37 KB of LDS allows: 64 VGPRs)
-constexpr int kTWaves = VC_TILE_WAVES;
+constexpr int kTBlock = 512; // threads of a tile-sweep workgroup
+// Waves per SIMD the tile sweep is compiled for.  With many tiles, four
+// workgroups per CU, which its 37 KB of LDS allows: 64 VGPRs.  With at most two
+// tiles per CU all are resident either way, and a sweep lasts as long as its
+// slowest visit: two workgroups per CU (92 VGPRs) let a visit keep every load of
+// its region in flight (kFew).  Skeletons at either side of that line, many / few:
+// 256^3 balls (256 tiles) 2.12 / 2.02 ms, 301 x 222 x 437 noise (490) 2.63 / 2.54,
+// 512^3 noise (2048) 6.44 / 7.32, 64 solids in a batch (over 512) 4.60 / 5.00.
+constexpr int kTWaves = 8, kTWavesFew = 4;
 constexpr int kTQ = 1024;              // candidate queue entries per round
-// rows of one parity evaluated per pass: at most 23 x 19 (pass 0)
-constexpr int kTRowsPerThread = (23 * 19 + kTBlock - 1) / kTBlock;
+// rows of one parity evaluated per pass: at most 23 x 19 (pass 0), one per thread;
 // a row holds at most 34 candidates of one z parity (68-bit window), and the
 // scan's ballot prefix takes per-thread counts below 64
-static_assert(kTRowsPerThread * 34 < 64, "tile_scan counts fit 6 bits");
+static_assert(23 * 19 <= kTBlock, "a row per thread");
 __device__ __forceinline__ int fy_of(int p) { return (7 - p) >> 1; }
 
 // window of word (o, w): bits 62..63 of word w-1, word w, bits 0..1 of w+1
@@ -1082,8 +1080,8 @@ __device__ __forceinline__ void report_sweep(unsigned long long* prog, uint32_t 
 // kTQ / kTBlock queue entries: neighbourhood code from the LDS rows, table
 // lookup, and on a hit an LDS atomic clears the bit.  Same-subfield voxels
 // are not 26-adjacent, so a code never reads a bit that this pass clears.
-template <bool kB>
-__global__ void __launch_bounds__(kTBlock, kTWaves)
+template <bool kB, bool kFew>
+__global__ void __launch_bounds__(kTBlock, kFew ? kTWavesFew : kTWaves)
     thin_tile_sweep(vc_work W, const uint32_t* __restrict__ lut, int j,
                     int k_arg, int nvol, const uint32_t* __restrict__ ctl,
                     uint32_t* gany, uint32_t* vany,
@@ -1155,20 +1153,54 @@ __global__ void __launch_bounds__(kTBlock, kTWaves)
         const uint64_t* Pin = (sweep & 1) ? d.alive2 : d.alive;
         uint64_t* Pout = (sweep & 1) ? d.alive : d.alive2;
         const int X0 = tx * kTT - kHX, Y0 = ty * kTT - kHY; // region origin
-        for (int r = threadIdx.x; r < kTRows; r += kTBlock)
+        // The windows of U of the thread's rows at a time, all their loads in
+        // flight together from clamped addresses: of one row for many tiles
+        // (512^3 noise 6.64 -> 6.44 ms against loads behind their bounds; of two
+        // 6.43, but a batch of 64 solids 4.62 against 4.60), of all for few
+        constexpr int U = kFew ? (kTRows + kTBlock - 1) / kTBlock : 1;
+#pragma unroll 1
+        for (int r0 = threadIdx.x; r0 < kTRows; r0 += U * kTBlock)
         {
-            const int x = X0 + r / kRY, y = Y0 + r % kRY;
-            uint64_t alo = 0, elo = 0;
-            uint32_t ahi = 0, ehi = 0;
-            if ((unsigned)x < (unsigned)d.nx && (unsigned)y < (unsigned)d.ny)
+            uint64_t v[U][6];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
             {
+                const int r = min(r0 + u * kTBlock, kTRows - 1);
+                const int x = min(max(X0 + r / kRY, 0), d.nx - 1);
+                const int y = min(max(Y0 + r % kRY, 0), d.ny - 1);
                 const int64_t o = ((int64_t)x * d.ny + y) * nwz + w;
-                load_win(Pin, o, w, nwz, alo, ahi);
-                load_win(d.elig, o, w, nwz, elo, ehi);
+                const int64_t op = o - (w > 0), on = o + (w + 1 < nwz);
+                v[u][0] = Pin[o];
+                v[u][1] = Pin[op];
+                v[u][2] = Pin[on];
+                v[u][3] = d.elig[o];
+                v[u][4] = d.elig[op];
+                v[u][5] = d.elig[on];
             }
-            SAL[r] = alo;
-            SElo[r] = elo;
-            SHB[r] = (uint8_t)(ahi | (ehi << 4));
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+            {
+                const int r = r0 + u * kTBlock;
+                const int x = X0 + r / kRY, y = Y0 + r % kRY;
+                const bool in = (unsigned)x < (unsigned)d.nx && (unsigned)y < (unsigned)d.ny;
+                uint64_t lo[2];
+                uint32_t hi[2];
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+                {
+                    const uint64_t c = v[u][3 * q];
+                    const uint64_t pv = w > 0 ? v[u][3 * q + 1] : 0ull;
+                    const uint64_t nv = w + 1 < nwz ? v[u][3 * q + 2] : 0ull;
+                    lo[q] = in ? (pv >> 62) | (c << 2) : 0ull;
+                    hi[q] = in ? (uint32_t)(c >> 62) | ((uint32_t)(nv & 3ull) << 2) : 0u;
+                }
+                if (r < kTRows)
+                {
+                    SAL[r] = lo[0];
+                    SElo[r] = lo[1];
+                    SHB[r] = (uint8_t)(hi[0] | (hi[1] << 4));
+                }
+            }
         }
         __syncthreads();
         uint32_t nrem = 0, ntest = 0, nbr = 0;
@@ -1184,27 +1216,23 @@ __global__ void __launch_bounds__(kTBlock, kTWaves)
             const int ylo = kHY - Fy, yhi = kHY + kTT + Fy;
             const int rx0 = xlo + ((xlo & 1) != sx), ry0 = ylo + ((ylo & 1) != sy);
             const int nrx = (xhi - rx0 + 1) >> 1, nry = (yhi - ry0 + 1) >> 1;
+            // q / nry for q < 512 as q * ceil(2^16 / nry) >> 16, nry = 19 - p / 2
+            // (with the division 64 solids 0.5 %, 512^3 0.4 %, 64^3 2 % slower)
+            const uint32_t inv = (uint32_t)(0x10010F100E390D7Aull >> (16 * (p >> 1))) & 0xFFFFu;
             // window bit parity = z parity (64w - 2 is even); bits
             // [kHZ - Fz, kHZ + 64 + Fz): low word from bit 1 or 2 up, high
             // bits 64..65 or 64..66
             const uint64_t zs64 = sz ? 0xAAAAAAAAAAAAAAAAull : 0x5555555555555555ull;
             const uint64_t zlo = zs64 & (~0ull << (kHZ - Fz));
             const uint32_t zhi = (uint32_t)zs64 & ((1u << (kHZ + Fz)) - 1u);
-            uint64_t clo[kTRowsPerThread];
-            uint32_t chi[kTRowsPerThread];
-            int rr[kTRowsPerThread];
-            uint32_t cnt = 0;
-#pragma unroll
-            for (int t = 0; t < kTRowsPerThread; ++t)
+            uint64_t clo = 0;
+            uint32_t chi = 0, cnt = 0;
+            int r = 0;
+            if (const int q = threadIdx.x; q < nrx * nry)
             {
-                clo[t] = 0;
-                chi[t] = 0;
-                rr[t] = 0;
-                const int q = threadIdx.x + t * kTBlock;
-                if (q >= nrx * nry)
-                    continue;
-                const int rx = rx0 + 2 * (q / nry), ry = ry0 + 2 * (q % nry);
-                const int r = rx * kRY + ry;
+                const int qx = (int)(((uint32_t)q * inv) >> 16), qy = q - qx * nry;
+                const int rx = rx0 + 2 * qx, ry = ry0 + 2 * qy;
+                r = rx * kRY + ry;
                 const uint32_t hb = SHB[r];
                 const TRow C{SAL[r], hb & 0xFu, 0u};
                 uint64_t cl = C.lo & SElo[r] & zlo;
@@ -1222,34 +1250,29 @@ __global__ void __launch_bounds__(kTBlock, kTWaves)
                     const uint32_t hup = C.hi >> 1;
                     ch &= ~(a.hi & bb.hi & c.hi & e.hi & hdn & hup);
                 }
-                clo[t] = cl;
-                chi[t] = ch;
-                rr[t] = r;
-                cnt += (uint32_t)(__popcll(cl) + __popc(ch));
+                clo = cl;
+                chi = ch;
+                cnt = (uint32_t)(__popcll(cl) + __popc(ch));
             }
             uint32_t total;
             uint32_t idx = tile_scan(cnt, red + (p & 1) * (kTBlock / 64), &total);
             ntest += total;
             for (uint32_t c0 = 0; c0 < total; c0 += kTQ)
             {
-#pragma unroll
-                for (int t = 0; t < kTRowsPerThread; ++t)
+                const uint32_t base = (uint32_t)r << 7;
+                while (clo && idx < c0 + kTQ)
                 {
-                    const uint32_t base = (uint32_t)rr[t] << 7;
-                    while (clo[t] && idx < c0 + kTQ)
-                    {
-                        const int i = __ffsll((unsigned long long)clo[t]) - 1;
-                        clo[t] &= clo[t] - 1;
-                        tq[idx - c0] = base | (uint32_t)i;
-                        ++idx;
-                    }
-                    while (chi[t] && idx < c0 + kTQ)
-                    {
-                        const int i = __ffs(chi[t]) - 1;
-                        chi[t] &= chi[t] - 1;
-                        tq[idx - c0] = base | (uint32_t)(64 + i);
-                        ++idx;
-                    }
+                    const int i = __ffsll((unsigned long long)clo) - 1;
+                    clo &= clo - 1;
+                    tq[idx - c0] = base | (uint32_t)i;
+                    ++idx;
+                }
+                while (chi && idx < c0 + kTQ)
+                {
+                    const int i = __ffs(chi) - 1;
+                    chi &= chi - 1;
+                    tq[idx - c0] = base | (uint32_t)(64 + i);
+                    ++idx;
                 }
                 __syncthreads();
                 const uint32_t n = min((uint32_t)kTQ, total - c0);
@@ -1394,8 +1417,12 @@ void launch_tile_sweep(hipStream_t S, unsigned g, const vc_work& W,
                        const uint32_t* ctl, vc_sched* s,
                        unsigned long long* prog = nullptr, uint32_t epoch = 0)
 {
-    thin_tile_sweep<kB><<<g, kTBlock, 0, S>>>(W, lut, j, k, n, ctl, s->d_gany,
-                                             s->d_vany, s->d_ctr, prog, epoch);
+    if (s->few_tiles)
+        thin_tile_sweep<kB, true><<<g, kTBlock, 0, S>>>(W, lut, j, k, n, ctl, s->d_gany,
+                                                           s->d_vany, s->d_ctr, prog, epoch);
+    else
+        thin_tile_sweep<kB, false><<<g, kTBlock, 0, S>>>(W, lut, j, k, n, ctl, s->d_gany,
+                                                          s->d_vany, s->d_ctr, prog, epoch);
 }
 
 // sweep timing: an event from the context's pool (nullptr when none can be
