@@ -172,3 +172,18 @@ def test_finalize_device_matches_host(vc):
         d = V.cc_finalize(nv, e_in, fs, ctx=vc)
         for a, b in zip(h, d):
             assert np.array_equal(a, b), i
+
+
+@pytest.mark.parametrize("sides", [3, 4, 5, 7, 8, 9, 17])
+@pytest.mark.parametrize("nv", [20, 4000])
+def test_finalize_device_lanes_per_face(vc, sides, nv):
+    """A face's sides go to four lanes: fewer, as many and more sides than lanes,
+    many faces on the same few pairs and nearly every pair its own, faces fewer
+    than the given edges and no given edges."""
+    rng = np.random.default_rng(sides * nv)
+    faces = [list(rng.permutation(nv)[:int(rng.integers(3, sides + 1))]) for _ in range(700)]
+    for m in (0, 5, 3000):
+        e = [tuple(rng.permutation(nv)[:2]) for _ in range(m)]
+        say("finalize lanes", sides, nv, m)
+        for a, b in zip(V.cc_finalize(nv, e, faces), V.cc_finalize(nv, e, faces, ctx=vc)):
+            assert np.array_equal(a, b)

@@ -142,6 +142,26 @@ def test_resident_diagram_matches_host_steps(vc):
         vol.release()
 
 
+@pytest.mark.parametrize("n", [2, 3, 31, 32, 33, 48])
+def test_valid_box_of_every_size(vc, n):
+    """The tag's count and box: fewer vertices than a workgroup, and more than the
+    capped grid has threads (32768)."""
+    rng = np.random.default_rng(n)
+    occ = (rng.random((n, n + 1, n)) < 0.7).astype(np.uint8)
+    occ[0, 0, 0] = 0
+    vol = vc.upload(occ)
+    vol.edt()
+    d = V.VoroDiagram(vol).tag(vol)
+    g, info = d.get(), d.info()
+    say("box", n, len(g["vts"]), "vertices")
+    ok = g["valid"] == 1
+    assert info["n_valid"] == int(ok.sum())
+    if ok.any():
+        assert np.array_equal(info["bb_min"], g["vts"][ok].min(0))
+        assert np.array_equal(info["bb_max"], g["vts"][ok].max(0))
+    vol.release()
+
+
 def test_resident_diagram_empty_and_errors(vc):
     """No inside voxel: an empty diagram through every step; a diagram
     before vc_edt is refused."""

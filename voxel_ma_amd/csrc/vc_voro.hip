@@ -383,33 +383,43 @@ __device__ __forceinline__ uint64_t mix64(uint64_t k)
     return k;
 }
 
-// insert key with value v (the table keeps the smallest value per key)
-__device__ void hash_min(uint64_t* keys, unsigned long long* vals, uint64_t mask,
-                         uint64_t key, unsigned long long v)
+// a key and the smallest value inserted with it, in one cache line
+struct Slot
+{
+    unsigned long long key, val;
+};
+
+// Insert key with value v (the table keeps the smallest value per key).  A slot's key never changes once set and its value only falls, so a plain look
+// first can only err on the side of an atomic too many.  Most pairs come more
+// than once (a diagram's edge has three faces or more), and the atomics' rate is
+// what bounds the insertions: fz_keys on the diagram of 96^3 noise 231 us with two
+// atomics per side on two arrays, 145 with the look at the key, 127 with both looks
+// in one slot (fz_first 68 -> 54, fz_emit 54 -> 40, xi_keep 57 -> 43: one line each).
+__device__ void hash_min(Slot* tab, uint64_t mask, uint64_t key, unsigned long long v)
 {
     uint64_t h = mix64(key) & mask;
     for (;;)
     {
-        const uint64_t prev = atomicCAS(
-            reinterpret_cast<unsigned long long*>(&keys[h]),
-            (unsigned long long)kEmptyKey, (unsigned long long)key);
+        uint64_t prev = __hip_atomic_load(&tab[h].key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (prev == kEmptyKey)
+            prev = atomicCAS(&tab[h].key, (unsigned long long)kEmptyKey,
+                             (unsigned long long)key);
         if (prev == kEmptyKey || prev == key)
         {
-            atomicMin(&vals[h], v);
+            if (__hip_atomic_load(&tab[h].val, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > v)
+                atomicMin(&tab[h].val, v);
             return;
         }
         h = (h + 1) & mask;
     }
 }
 
-__device__ unsigned long long hash_get(const uint64_t* keys,
-                                       const unsigned long long* vals,
-                                       uint64_t mask, uint64_t key)
+__device__ unsigned long long hash_get(const Slot* tab, uint64_t mask, uint64_t key)
 {
     uint64_t h = mix64(key) & mask;
-    while (keys[h] != key)
+    while (tab[h].key != key)
         h = (h + 1) & mask;
-    return vals[h];
+    return tab[h].val;
 }
 
 __global__ void __launch_bounds__(kBlock)
@@ -441,7 +451,7 @@ __global__ void __launch_bounds__(kBlock)
                const uint32_t* __restrict__ vpos, const uint32_t* __restrict__ epos,
                const float* __restrict__ lam_e, int32_t* __restrict__ vts_idx,
                int32_t* __restrict__ e_out, float* __restrict__ em,
-               uint64_t* keys, unsigned long long* vals, uint64_t mask)
+               Slot* tab, uint64_t mask)
 {
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (i < nv && valid[i])
@@ -453,9 +463,15 @@ __global__ void __launch_bounds__(kBlock)
         e_out[2 * k] = (int32_t)vpos[a];
         e_out[2 * k + 1] = (int32_t)vpos[b];
         em[k] = lam_e[i];
-        hash_min(keys, vals, mask, pair_key(a, b), 0ull);
+        hash_min(tab, mask, pair_key(a, b), 0ull);
     }
 }
+
+// Lanes per face in the kernels that insert a face's sides: a thread that inserts
+// them one after the other is a chain of waits for memory far away, the lanes of a
+// group take them side by side.  Diagram of 96^3 noise, one / four lanes: fz_keys
+// 127 / 112 us, xi_tris 121 / 87.
+constexpr int kFaceLanes = 4;
 
 // triangles of the valid faces (zig-zag: triangle t of an n-gon is
 // (p[i], p[j], p[j+1]) for even t and (p[i], p[j], p[i-1]) for odd t, with
@@ -466,18 +482,18 @@ __global__ void __launch_bounds__(kBlock)
             const int32_t* __restrict__ fv, const uint32_t* __restrict__ toff,
             const uint32_t* __restrict__ vpos, const float* __restrict__ lam_f,
             int32_t* __restrict__ tris, int32_t* __restrict__ from_fi,
-            float* __restrict__ fm, uint64_t* __restrict__ ckey, uint64_t* keys,
-            unsigned long long* vals, uint64_t mask)
+            float* __restrict__ fm, uint64_t* __restrict__ ckey, Slot* tab, uint64_t mask)
 {
-    const int64_t f = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    const int64_t f = i / kFaceLanes;
     if (f >= nf || toff[f + 1] == toff[f])
         return;
     const int32_t* p = fv + fo[f];
     const int n = (int)(fo[f + 1] - fo[f]);
-    for (int t = 0; t < n - 2; ++t)
+    for (int t = (int)(i % kFaceLanes); t < n - 2; t += kFaceLanes)
     {
-        const int i = n - 1 - t / 2, j = (t + 1) / 2;
-        const int32_t v[3] = {p[i], p[j], (t & 1) ? p[i - 1] : p[j + 1]};
+        const int u = n - 1 - t / 2, j = (t + 1) / 2;
+        const int32_t v[3] = {p[u], p[j], (t & 1) ? p[u - 1] : p[j + 1]};
         const int64_t T = (int64_t)toff[f] + t;
         for (int s = 0; s < 3; ++s)
         {
@@ -491,7 +507,7 @@ __global__ void __launch_bounds__(kBlock)
             }
             const uint64_t k = pair_key(a, b);
             ckey[3 * T + s] = k;
-            hash_min(keys, vals, mask, k, (unsigned long long)(3 * T + s) + 1ull);
+            hash_min(tab, mask, k, (unsigned long long)(3 * T + s) + 1ull);
         }
         from_fi[T] = (int32_t)f;
         fm[T] = lam_f[f];
@@ -499,13 +515,12 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 __global__ void __launch_bounds__(kBlock)
-    xi_keep(int64_t nc, const uint64_t* __restrict__ ckey, const uint64_t* keys,
-            const unsigned long long* vals, uint64_t mask,
+    xi_keep(int64_t nc, const uint64_t* __restrict__ ckey, const Slot* tab, uint64_t mask,
             uint32_t* __restrict__ keep)
 {
     const int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (c < nc)
-        keep[c] = hash_get(keys, vals, mask, ckey[c]) == (unsigned long long)c + 1ull
+        keep[c] = hash_get(tab, mask, ckey[c]) == (unsigned long long)c + 1ull
                       ? 1u
                       : 0u;
 }
@@ -534,22 +549,21 @@ __global__ void __launch_bounds__(kBlock)
 __global__ void __launch_bounds__(kBlock)
     fz_keys(int32_t ne, const int32_t* __restrict__ E, int32_t nf,
             const int64_t* __restrict__ fo, const int32_t* __restrict__ fv,
-            uint64_t* __restrict__ ckey, uint64_t* keys,
-            unsigned long long* vals, uint64_t mask)
+            uint64_t* __restrict__ ckey, Slot* tab, uint64_t mask)
 {
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (i < ne)
     {
         const uint64_t k = pair_key(E[2 * i], E[2 * i + 1]);
         ckey[i] = k;
-        hash_min(keys, vals, mask, k, (unsigned long long)i);
+        hash_min(tab, mask, k, (unsigned long long)i);
     }
-    if (i < nf)
+    if (const int64_t f = i / kFaceLanes; f < nf)
     {
-        const int64_t n = fo[i + 1] - fo[i];
-        for (int64_t j = 0; j < n; ++j)
+        const int64_t f0 = fo[f], n = fo[f + 1] - f0;
+        for (int64_t j = i % kFaceLanes; j < n; j += kFaceLanes)
         {
-            int32_t a = fv[fo[i] + j], b = fv[fo[i] + (j + 1) % n];
+            int32_t a = fv[f0 + j], b = fv[f0 + (j + 1 < n ? j + 1 : 0)];
             if (a > b)
             {
                 const int32_t t = a;
@@ -557,28 +571,26 @@ __global__ void __launch_bounds__(kBlock)
                 b = t;
             }
             const uint64_t k = pair_key(a, b);
-            const int64_t c = ne + fo[i] + j;
+            const int64_t c = ne + f0 + j;
             ckey[c] = k;
-            hash_min(keys, vals, mask, k, (unsigned long long)c);
+            hash_min(tab, mask, k, (unsigned long long)c);
         }
     }
 }
 
 __global__ void __launch_bounds__(kBlock)
-    fz_first(int64_t nc, const uint64_t* __restrict__ ckey, const uint64_t* keys,
-             const unsigned long long* vals, uint64_t mask,
+    fz_first(int64_t nc, const uint64_t* __restrict__ ckey, const Slot* tab, uint64_t mask,
              uint32_t* __restrict__ first)
 {
     const int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (c < nc)
-        first[c] = hash_get(keys, vals, mask, ckey[c]) == (unsigned long long)c ? 1u
+        first[c] = hash_get(tab, mask, ckey[c]) == (unsigned long long)c ? 1u
                                                                                 : 0u;
 }
 
 __global__ void __launch_bounds__(kBlock)
     fz_emit(int64_t nc, int32_t ne, const uint64_t* __restrict__ ckey,
-            const uint32_t* __restrict__ pos, const uint64_t* keys,
-            const unsigned long long* vals, uint64_t mask,
+            const uint32_t* __restrict__ pos, const Slot* tab, uint64_t mask,
             int32_t* __restrict__ e_out, int32_t* __restrict__ fe)
 {
     const int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x;
@@ -591,7 +603,7 @@ __global__ void __launch_bounds__(kBlock)
         e_out[2 * (int64_t)pos[c] + 1] = (int32_t)(k & 0xFFFFFFFFull);
     }
     if (c >= ne)
-        fe[c - ne] = (int32_t)pos[hash_get(keys, vals, mask, k)];
+        fe[c - ne] = (int32_t)pos[hash_get(tab, mask, k)];
 }
 
 __global__ void __launch_bounds__(kBlock) fill_u64(uint64_t* a, int64_t n, uint64_t v)
@@ -696,30 +708,28 @@ int vc_cc_finalize_dev(vc_ctx* ctx, int32_t ne_in, const int32_t* dE, int32_t nf
     uint64_t H = 1024;
     while (H < 2 * (uint64_t)NC + 1)
         H <<= 1;
-    uint64_t *keys, *ckey;
-    unsigned long long* vals;
+    Slot* tab;
+    uint64_t* ckey;
     uint32_t* pos;
     int rc = VC_OK;
     auto get = [&](auto** p, size_t n) {
         if (rc == VC_OK)
             rc = sc.get(ctx, p, n);
     };
-    get(&keys, (size_t)H);
-    get(&vals, (size_t)H);
+    get(&tab, (size_t)H);
     get(&ckey, (size_t)NC + 1);
     get(&pos, (size_t)NC + 1);
     if (rc != VC_OK)
         return rc;
-    fill_u64<<<blocks_for((int64_t)H), kBlock, 0, S>>>(keys, (int64_t)H, kEmptyKey);
-    fill_u64<<<blocks_for((int64_t)H), kBlock, 0, S>>>(
-        reinterpret_cast<uint64_t*>(vals), (int64_t)H, ~0ull);
+    static_assert(kEmptyKey == ~0ull, "one fill clears keys and values");
+    fill_u64<<<blocks_for(2 * (int64_t)H), kBlock, 0, S>>>(reinterpret_cast<uint64_t*>(tab),
+                                                           2 * (int64_t)H, ~0ull);
     VC_HIP(ctx, hipMemsetAsync(pos, 0, 4 * ((size_t)NC + 1), S));
-    const int64_t mx = std::max<int64_t>(ne_in, nf);
+    const int64_t mx = std::max<int64_t>(ne_in, (int64_t)nf * kFaceLanes);
     if (mx)
-        fz_keys<<<blocks_for(mx), kBlock, 0, S>>>(ne_in, dE, nf, dfo, dfv, ckey, keys,
-                                                  vals, H - 1);
+        fz_keys<<<blocks_for(mx), kBlock, 0, S>>>(ne_in, dE, nf, dfo, dfv, ckey, tab, H - 1);
     if (NC)
-        fz_first<<<blocks_for(NC), kBlock, 0, S>>>(NC, ckey, keys, vals, H - 1, pos);
+        fz_first<<<blocks_for(NC), kBlock, 0, S>>>(NC, ckey, tab, H - 1, pos);
     VC_CHECK_LAUNCH(ctx);
     if ((rc = vc_scan_u32(ctx, pos, NC + 1)) != VC_OK)
         return rc;
@@ -728,7 +738,7 @@ int vc_cc_finalize_dev(vc_ctx* ctx, int32_t ne_in, const int32_t* dE, int32_t nf
     VC_HIP(ctx, hipStreamSynchronize(S));
     *ne_out = (int32_t)ne;
     if (NC)
-        fz_emit<<<blocks_for(NC), kBlock, 0, S>>>(NC, ne_in, ckey, pos, keys, vals,
+        fz_emit<<<blocks_for(NC), kBlock, 0, S>>>(NC, ne_in, ckey, pos, tab,
                                                   H - 1, deo, dfe);
     VC_CHECK_LAUNCH(ctx);
     // the temporaries are freed on return: wait for the kernels reading them
@@ -1304,8 +1314,7 @@ int vc_voro_extract_dev(vc_ctx* ctx, int32_t nv, int32_t ne, int32_t nf,
     uint64_t H = 1024;
     while (H < 2 * (uint64_t)(NE + NC) + 1)
         H <<= 1;
-    uint64_t* keys;
-    unsigned long long* vals;
+    Slot* tab;
     uint64_t* ckey;
     uint32_t* keep;
     own(&out->vi, (size_t)NV + 1);
@@ -1314,8 +1323,7 @@ int vc_voro_extract_dev(vc_ctx* ctx, int32_t nv, int32_t ne, int32_t nf,
     own(&out->tr, 3 * (size_t)NT + 3);
     own(&out->ff, (size_t)NT + 1);
     own(&out->fm, (size_t)NT + 1);
-    get(&keys, (size_t)H);
-    get(&vals, (size_t)H);
+    get(&tab, (size_t)H);
     get(&ckey, (size_t)NC + 1);
     get(&keep, (size_t)NC + 1);
     if (rc != VC_OK)
@@ -1323,24 +1331,23 @@ int vc_voro_extract_dev(vc_ctx* ctx, int32_t nv, int32_t ne, int32_t nf,
         vc_voro_xi_free(out);
         return rc;
     }
-    fill_u64<<<blocks_for((int64_t)H), kBlock, 0, S>>>(keys, (int64_t)H, kEmptyKey);
-    fill_u64<<<blocks_for((int64_t)H), kBlock, 0, S>>>(
-        reinterpret_cast<uint64_t*>(vals), (int64_t)H, ~0ull);
+    static_assert(kEmptyKey == ~0ull, "one fill clears keys and values");
+    fill_u64<<<blocks_for(2 * (int64_t)H), kBlock, 0, S>>>(reinterpret_cast<uint64_t*>(tab),
+                                                           2 * (int64_t)H, ~0ull);
     const int64_t mve = std::max<int64_t>(nv, ne);
     if (mve)
         xi_emit_ve<<<blocks_for(mve), kBlock, 0, S>>>(nv, ne, dE, dval, vpos, epos, dle,
-                                                      out->vi, out->eo, out->em, keys,
-                                                      vals, H - 1);
+                                                      out->vi, out->eo, out->em, tab, H - 1);
     if (nf)
-        xi_tris<<<blocks_for(nf), kBlock, 0, S>>>(nf, dfo, dfv, toff, vpos, dlf, out->tr,
-                                                  out->ff, out->fm, ckey, keys, vals,
+        xi_tris<<<blocks_for((int64_t)nf * kFaceLanes), kBlock, 0, S>>>(nf, dfo, dfv, toff, vpos, dlf, out->tr,
+                                                  out->ff, out->fm, ckey, tab,
                                                   H - 1);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess)
         e = hipMemsetAsync(keep, 0, 4 * ((size_t)NC + 1), S);
     if (e == hipSuccess && NC)
     {
-        xi_keep<<<blocks_for(NC), kBlock, 0, S>>>(NC, ckey, keys, vals, H - 1, keep);
+        xi_keep<<<blocks_for(NC), kBlock, 0, S>>>(NC, ckey, tab, H - 1, keep);
         e = hipGetLastError();
     }
     if (e != hipSuccess)
