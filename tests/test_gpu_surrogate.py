@@ -288,6 +288,38 @@ def test_gated_measure_drives_exact_thinning(vc, oracle, tau):
     net.release()
 
 
+@pytest.mark.parametrize("shape", [(2, 3, 2), (3, 5, 1), (13, 11, 23), (16, 12, 30)])
+def test_gate_on_every_remainder(vc, oracle, shape):
+    """The gate takes 16 and 4 voxels per access: volumes of 12, 15, 3289 and 5760
+    voxels, the last voxels inside, half of the voxels accepted."""
+    rng = np.random.default_rng(sum(shape))
+    occ = (rng.random(shape) < 0.75).astype(np.uint8)
+    occ[-1, -1] = 1
+    occ[0, 0] = 0
+    vol = vc.upload(occ)
+    vol.edt()
+    net = V.Surrogate(vc, seed=8)
+    net.set_params(_theta(8))
+    lam, rel = net.infer(vol)
+    inside = occ > 0
+    tau = float(np.median(rel[inside]))
+    st = net.measure(vol, max_rel_err=tau)
+    say("gate", shape, tau, st.as_dict())
+    acc = rel <= np.float32(tau)
+    assert st.inside == int(inside.sum()) and st.accepted == int(acc[inside].sum())
+    assert st.accepted + st.fallback == st.inside and st.fallback > 0
+    vol.thin_levels([0.0])
+    lam2 = vol.get(V.BUF_LAM2)
+    meas = np.where(acc, np.maximum(lam, np.float32(0)), np.sqrt(lam2.astype(np.float32)))
+    # one level at each of the measures that occur: a voxel is a level-0 voxel
+    # where its measure is below, so the levels show every value
+    for t in np.unique(meas[inside])[:: max(1, inside.sum() // 40)]:
+        vol.thin_levels([float(t)])
+        assert np.array_equal(vol.get(V.BUF_LEVEL)[inside] == 0, meas[inside] < t), t
+    vol.release()
+    net.release()
+
+
 def test_trained_network_gain(vc):
     """What training buys, on held-out volumes the network never saw: the
     committed weights (voxel_ma_amd/data/unet.bin, trained by

@@ -95,7 +95,7 @@ __global__ void __launch_bounds__(kB)
               int32_t nv, unsigned long long* cnt, uint32_t* box)
 {
     // The seven words take one atomic after the other (about 10 ns each): a capped
-    // grid strides over the vertices and each workgroup adds once.  0.6 M vertices:
+    // grid strides over the vertices and each workgroup adds once.  96^3 noise:
     // one add per wavefront of a full grid 295 us, of 256 workgroups 74, this under 40
     __shared__ uint32_t sh[kB / 64][7];
     uint32_t c = 0;
