@@ -417,7 +417,7 @@ def edt_ball_row(ctx, n, reps=3):
             "ms": round(ms, 3), "value": round(n ** 3 / ms / 1e3, 1), "unit": "Mvoxels/s",
             "achieved_gbs": round(gbs, 1), "frac": round(gbs / 8000.0, 4),
             "note": "column passes search outward until the squared distance passes the "
-                    "best cost, so their work grows with the distance to the surface"}
+                    "best cost; deep tiles, nearly all here, divide and conquer instead"}
 
 
 def rows_leg(ctx, occ_host, label_host, reps=3):

@@ -6,10 +6,10 @@
 // four pairs (lane group g = lane / 16 holds one), so any channel count that
 // is a multiple of 8 tiles K exactly; the input is staged in LDS per output
 // brick (conv_fwd_lds).  The input-gradient pass is the same kernel with the
-// taps flipped and the channel roles swapped; the weight gradient stages 64-voxel
-// blocks of the layer input and output gradient in LDS and reduces over
-// voxels on MFMA into per-chunk partials, summed by a second kernel (fixed
-// order: the gradients are deterministic).
+// taps flipped and the channel roles swapped; the weight gradient stages 4 x 4 x 32
+// bricks of the output gradient and of the layer input with its halo in LDS and
+// reduces over voxels on MFMA into per-chunk partials, summed by a second kernel
+// (fixed order: the gradients are deterministic).
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
