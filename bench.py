@@ -79,8 +79,9 @@ def measured_traffic(kernel, n):
         return None
     with open(path) as f:
         t = json.load(f).get("traffic_bytes_per_dispatch", {})
-    v = t.get(kernel)
-    return None if v is None else round(v)
+    # the summary names instances: thin_tile_sweep<false, false>
+    v = [b for k, b in t.items() if k.split("<")[0] == kernel]
+    return round(v[0]) if v else None
 
 
 def _host_cpu():
