@@ -153,6 +153,13 @@ __global__ void __launch_bounds__(kBlock)
 
 unsigned blocks_for(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
 
+// for kernels whose work-items may reach 2^32, which no launch can hold (several
+// items per element): 2^31 at most, striding over the rest
+unsigned stride_blocks(int64_t n)
+{
+    return (unsigned)std::min<int64_t>((n + kBlock - 1) / kBlock, (int64_t(1) << 31) / kBlock);
+}
+
 // device copies that are freed on every exit path
 struct Scratch
 {
@@ -389,7 +396,8 @@ struct Slot
     unsigned long long key, val;
 };
 
-// Insert key with value v (the table keeps the smallest value per key).  A slot's key never changes once set and its value only falls, so a plain look
+// Insert key with value v (the table keeps the smallest value per key).  A
+// slot's key never changes once set and its value only falls, so a plain look
 // first can only err on the side of an atomic too many.  Most pairs come more
 // than once (a diagram's edge has three faces or more), and the atomics' rate is
 // what bounds the insertions: fz_keys on the diagram of 96^3 noise 231 us with two
@@ -484,33 +492,36 @@ __global__ void __launch_bounds__(kBlock)
             int32_t* __restrict__ tris, int32_t* __restrict__ from_fi,
             float* __restrict__ fm, uint64_t* __restrict__ ckey, Slot* tab, uint64_t mask)
 {
-    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    const int64_t f = i / kFaceLanes;
-    if (f >= nf || toff[f + 1] == toff[f])
-        return;
-    const int32_t* p = fv + fo[f];
-    const int n = (int)(fo[f + 1] - fo[f]);
-    for (int t = (int)(i % kFaceLanes); t < n - 2; t += kFaceLanes)
+    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i / kFaceLanes < nf;
+         i += (int64_t)gridDim.x * kBlock)
     {
-        const int u = n - 1 - t / 2, j = (t + 1) / 2;
-        const int32_t v[3] = {p[u], p[j], (t & 1) ? p[u - 1] : p[j + 1]};
-        const int64_t T = (int64_t)toff[f] + t;
-        for (int s = 0; s < 3; ++s)
+        const int64_t f = i / kFaceLanes;
+        if (toff[f + 1] == toff[f])
+            continue;
+        const int32_t* p = fv + fo[f];
+        const int n = (int)(fo[f + 1] - fo[f]);
+        for (int t = (int)(i % kFaceLanes); t < n - 2; t += kFaceLanes)
         {
-            tris[3 * T + s] = (int32_t)vpos[v[s]];
-            int32_t a = v[s], b = v[(s + 1) % 3];
-            if (a > b)
+            const int u = n - 1 - t / 2, j = (t + 1) / 2;
+            const int32_t v[3] = {p[u], p[j], (t & 1) ? p[u - 1] : p[j + 1]};
+            const int64_t T = (int64_t)toff[f] + t;
+            for (int s = 0; s < 3; ++s)
             {
-                const int32_t x = a;
-                a = b;
-                b = x;
+                tris[3 * T + s] = (int32_t)vpos[v[s]];
+                int32_t a = v[s], b = v[(s + 1) % 3];
+                if (a > b)
+                {
+                    const int32_t x = a;
+                    a = b;
+                    b = x;
+                }
+                const uint64_t k = pair_key(a, b);
+                ckey[3 * T + s] = k;
+                hash_min(tab, mask, k, (unsigned long long)(3 * T + s) + 1ull);
             }
-            const uint64_t k = pair_key(a, b);
-            ckey[3 * T + s] = k;
-            hash_min(tab, mask, k, (unsigned long long)(3 * T + s) + 1ull);
+            from_fi[T] = (int32_t)f;
+            fm[T] = lam_f[f];
         }
-        from_fi[T] = (int32_t)f;
-        fm[T] = lam_f[f];
     }
 }
 
@@ -551,29 +562,32 @@ __global__ void __launch_bounds__(kBlock)
             const int64_t* __restrict__ fo, const int32_t* __restrict__ fv,
             uint64_t* __restrict__ ckey, Slot* tab, uint64_t mask)
 {
-    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i < ne)
+    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+         i < ne || i / kFaceLanes < nf; i += (int64_t)gridDim.x * kBlock)
     {
-        const uint64_t k = pair_key(E[2 * i], E[2 * i + 1]);
-        ckey[i] = k;
-        hash_min(tab, mask, k, (unsigned long long)i);
-    }
-    if (const int64_t f = i / kFaceLanes; f < nf)
-    {
-        const int64_t f0 = fo[f], n = fo[f + 1] - f0;
-        for (int64_t j = i % kFaceLanes; j < n; j += kFaceLanes)
+        if (i < ne)
         {
-            int32_t a = fv[f0 + j], b = fv[f0 + (j + 1 < n ? j + 1 : 0)];
-            if (a > b)
+            const uint64_t k = pair_key(E[2 * i], E[2 * i + 1]);
+            ckey[i] = k;
+            hash_min(tab, mask, k, (unsigned long long)i);
+        }
+        if (const int64_t f = i / kFaceLanes; f < nf)
+        {
+            const int64_t f0 = fo[f], n = fo[f + 1] - f0;
+            for (int64_t j = i % kFaceLanes; j < n; j += kFaceLanes)
             {
-                const int32_t t = a;
-                a = b;
-                b = t;
+                int32_t a = fv[f0 + j], b = fv[f0 + (j + 1 < n ? j + 1 : 0)];
+                if (a > b)
+                {
+                    const int32_t t = a;
+                    a = b;
+                    b = t;
+                }
+                const uint64_t k = pair_key(a, b);
+                const int64_t c = ne + f0 + j;
+                ckey[c] = k;
+                hash_min(tab, mask, k, (unsigned long long)c);
             }
-            const uint64_t k = pair_key(a, b);
-            const int64_t c = ne + f0 + j;
-            ckey[c] = k;
-            hash_min(tab, mask, k, (unsigned long long)c);
         }
     }
 }
@@ -608,8 +622,8 @@ __global__ void __launch_bounds__(kBlock)
 
 __global__ void __launch_bounds__(kBlock) fill_u64(uint64_t* a, int64_t n, uint64_t v)
 {
-    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i < n)
+    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n;
+         i += (int64_t)gridDim.x * kBlock)
         a[i] = v;
 }
 
@@ -722,12 +736,12 @@ int vc_cc_finalize_dev(vc_ctx* ctx, int32_t ne_in, const int32_t* dE, int32_t nf
     if (rc != VC_OK)
         return rc;
     static_assert(kEmptyKey == ~0ull, "one fill clears keys and values");
-    fill_u64<<<blocks_for(2 * (int64_t)H), kBlock, 0, S>>>(reinterpret_cast<uint64_t*>(tab),
-                                                           2 * (int64_t)H, ~0ull);
+    fill_u64<<<stride_blocks(2 * (int64_t)H), kBlock, 0, S>>>(reinterpret_cast<uint64_t*>(tab),
+                                                              2 * (int64_t)H, ~0ull);
     VC_HIP(ctx, hipMemsetAsync(pos, 0, 4 * ((size_t)NC + 1), S));
     const int64_t mx = std::max<int64_t>(ne_in, (int64_t)nf * kFaceLanes);
     if (mx)
-        fz_keys<<<blocks_for(mx), kBlock, 0, S>>>(ne_in, dE, nf, dfo, dfv, ckey, tab, H - 1);
+        fz_keys<<<stride_blocks(mx), kBlock, 0, S>>>(ne_in, dE, nf, dfo, dfv, ckey, tab, H - 1);
     if (NC)
         fz_first<<<blocks_for(NC), kBlock, 0, S>>>(NC, ckey, tab, H - 1, pos);
     VC_CHECK_LAUNCH(ctx);
@@ -1332,16 +1346,15 @@ int vc_voro_extract_dev(vc_ctx* ctx, int32_t nv, int32_t ne, int32_t nf,
         return rc;
     }
     static_assert(kEmptyKey == ~0ull, "one fill clears keys and values");
-    fill_u64<<<blocks_for(2 * (int64_t)H), kBlock, 0, S>>>(reinterpret_cast<uint64_t*>(tab),
-                                                           2 * (int64_t)H, ~0ull);
+    fill_u64<<<stride_blocks(2 * (int64_t)H), kBlock, 0, S>>>(reinterpret_cast<uint64_t*>(tab),
+                                                              2 * (int64_t)H, ~0ull);
     const int64_t mve = std::max<int64_t>(nv, ne);
     if (mve)
         xi_emit_ve<<<blocks_for(mve), kBlock, 0, S>>>(nv, ne, dE, dval, vpos, epos, dle,
                                                       out->vi, out->eo, out->em, tab, H - 1);
     if (nf)
-        xi_tris<<<blocks_for((int64_t)nf * kFaceLanes), kBlock, 0, S>>>(nf, dfo, dfv, toff, vpos, dlf, out->tr,
-                                                  out->ff, out->fm, ckey, tab,
-                                                  H - 1);
+        xi_tris<<<stride_blocks((int64_t)nf * kFaceLanes), kBlock, 0, S>>>(
+            nf, dfo, dfv, toff, vpos, dlf, out->tr, out->ff, out->fm, ckey, tab, H - 1);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess)
         e = hipMemsetAsync(keep, 0, 4 * ((size_t)NC + 1), S);
