@@ -80,3 +80,30 @@ def test_launches_below_the_dispatch_limit(fake, case):
     assert F.fake_launches() > 0
     assert F.fake_items() < 1 << 32, (F.fake_items(), F.fake_biggest())
     """ % case)
+
+
+def test_allocations_go_on_while_another_context_frees(fake):
+    """hipFree waits for its device: a context whose blocks are too large to be
+    kept (4.6 GB here) frees them on a busy device, and another context's
+    allocations from its own kept blocks do not wait for it."""
+    fake("""
+    shape = (1024, 1024, 1100)
+    other = V.Context(0)
+    warm = lambda: other.upload(np.ones((20, 20, 20), np.uint8)).release()
+    warm()
+    big = vc.from_device(4096, shape).edt()
+    F.fake_hold(1)
+    a = threading.Thread(target=big.release)
+    b = threading.Thread(target=warm)
+    a.start()
+    while not F.fake_held():
+        time.sleep(0.01)
+    n = F.fake_allocs()
+    b.start()
+    b.join(10)
+    waited = b.is_alive()
+    F.fake_hold(0)
+    a.join()
+    b.join()
+    assert not waited and F.fake_allocs() == n
+    """)

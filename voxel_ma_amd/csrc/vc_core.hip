@@ -3,6 +3,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <list>
 #include <mutex>
 #include <new>
 #include <set>
@@ -29,7 +30,7 @@ int vc_fail(vc_ctx* ctx, int code, const char* fmt, ...)
 // the complex of a 96^3 volume makes about 300 of them, a volume made and
 // released per call about 25.  So what a context frees is kept, up to kDevCap
 // and kHostCap bytes (the oldest blocks go first), and given back when the
-// context is destroyed or when any allocation would fail: the 96^3 complex
+// context is destroyed or when an allocation made here would fail: the 96^3 complex
 // 36.7 -> 14.2 ms, a 96 x 81 x 107 volume's skeleton from host to host bytes 1.26
 // -> 0.96 ms, the boundary mesh of a new 256^3 volume 2.81 -> 2.53 ms.
 namespace
@@ -37,14 +38,12 @@ namespace
 constexpr size_t kDevCap = size_t(8) << 30, kDevBlock = size_t(2) << 30;
 constexpr size_t kHostCap = size_t(64) << 20, kHostBlock = size_t(16) << 20;
 
-struct live_block
-{
-    vc_ctx* ctx; // null: its context is gone, or the block is not kept
-    size_t bytes;
-};
+// The tables below, held for a look-up or a list operation only: the runtime
+// allocates and frees outside it, since hipFree waits for its device and would
+// stop the allocations of every other context meanwhile.
 std::mutex g_mem_mu;
-std::unordered_map<void*, live_block> g_live[2]; // handed out: device, host
-std::set<vc_ctx*> g_ctxs;                         // contexts that keep blocks
+std::unordered_map<void*, vc_block*> g_blocks[2]; // device, pinned host
+std::set<vc_ctx*> g_ctxs;                          // contexts that keep blocks
 
 vc_cache& cache_of(vc_ctx* ctx, int host)
 {
@@ -61,32 +60,65 @@ void raw_free(int host, void* p)
     else
         (void)hipFree(p);
 }
-// frees the oldest kept blocks until at most `keep` bytes are left
-void trim(vc_cache& c, int host, size_t keep)
+// sizes are rounded up to eighths of a power of two, so that the buffers of
+// similar volumes reuse each other's blocks; cls is the index of the size
+size_t size_class(size_t bytes, int& cls)
+{
+    size_t step = 256;
+    int s = 0;
+    for (; step * 16 < bytes; ++s)
+        step <<= 1;
+    const size_t k = (bytes + step - 1) / step; // 1..16, from 9 on for s > 0
+    cls = s == 0 ? (int)k - 1 : 8 + 8 * s + (int)k - 9;
+    return k * step;
+}
+// a kept block leaves its cache (under the lock)
+void take(vc_cache& c, vc_block* b)
+{
+    int cls;
+    size_class(b->bytes, cls);
+    b->node.splice(b->node.begin(), c.order, b->at);
+    b->fit_node.splice(b->fit_node.begin(), c.fit[cls], b->fit_at);
+    c.bytes -= b->bytes;
+    b->kept = false;
+}
+// takes the oldest kept blocks out until at most `keep` bytes are left; the
+// caller frees them after it let the lock go
+void trim(vc_cache& c, int host, size_t keep, std::list<vc_block*>& out)
 {
     while (c.bytes > keep)
     {
-        const vc_cache::block b = c.order.front();
-        auto r = c.by_size.equal_range(b.bytes);
-        for (auto it = r.first; it != r.second; ++it)
-            if (it->second == c.order.begin())
-            {
-                c.by_size.erase(it);
-                break;
-            }
-        c.order.pop_front();
-        c.bytes -= b.bytes;
-        raw_free(host, b.p);
+        vc_block* b = c.order.front();
+        take(c, b);
+        g_blocks[host].erase(b->p);
+        out.splice(out.end(), b->node);
     }
 }
-// sizes are rounded up to eighths of a power of two, so that the buffers of
-// similar volumes reuse each other's blocks
-size_t size_class(size_t bytes)
+void free_all(int host, std::list<vc_block*>& out)
 {
-    size_t step = 256;
-    while (step * 16 < bytes)
-        step <<= 1;
-    return (bytes + step - 1) / step * step;
+    for (vc_block* b : out)
+    {
+        raw_free(host, b->p);
+        delete b;
+    }
+    out.clear();
+}
+// a record with its list nodes; null when the host has no memory
+vc_block* new_block()
+{
+    vc_block* b = nullptr;
+    try
+    {
+        b = new vc_block();
+        b->node.push_back(b);
+        b->fit_node.push_back(b);
+    }
+    catch (const std::bad_alloc&)
+    {
+        delete b;
+        b = nullptr;
+    }
+    return b;
 }
 
 int mem_alloc(vc_ctx* ctx, int host, void** p, size_t bytes)
@@ -95,45 +127,71 @@ int mem_alloc(vc_ctx* ctx, int host, void** p, size_t bytes)
     if (bytes == 0)
         bytes = 256;
     const bool kept = bytes <= (host ? kHostBlock : kDevBlock);
-    const size_t want = kept ? size_class(bytes) : bytes;
-    std::lock_guard<std::mutex> lock(g_mem_mu);
+    size_t want = bytes;
     if (kept)
     {
+        int cls;
+        want = size_class(bytes, cls);
+        std::lock_guard<std::mutex> lock(g_mem_mu);
         vc_cache& c = cache_of(ctx, host);
-        auto it = c.by_size.lower_bound(want);
-        if (it != c.by_size.end() && it->first <= want + want / 4)
+        for (; cls < VC_SIZE_CLASSES; ++cls)
         {
-            *p = it->second->p;
-            g_live[host][*p] = live_block{ctx, it->first};
-            c.bytes -= it->first;
-            c.order.erase(it->second);
-            c.by_size.erase(it);
+            if (c.fit[cls].empty())
+                continue;
+            vc_block* b = c.fit[cls].front();
+            if (b->bytes > want + want / 4)
+                break;
+            take(c, b);
+            *p = b->p;
             return VC_OK;
         }
-        g_ctxs.insert(ctx);
     }
-    hipError_t e = raw_alloc(host, p, want);
+    vc_block* b = new_block();
+    if (!b)
+        return vc_fail(ctx, VC_ERR_NOMEM, "no host memory for an allocation's record");
+    b->bytes = want;
+    b->home = kept ? &cache_of(ctx, host) : nullptr;
+    hipError_t e = raw_alloc(host, &b->p, want);
     if (e != hipSuccess)
     {
         // memory that is only kept goes back first
         (void)hipGetLastError();
-        for (vc_ctx* c : g_ctxs)
+        std::list<vc_block*> out[2];
         {
-            trim(c->cache_dev, 0, 0);
-            trim(c->cache_host, 1, 0);
+            std::lock_guard<std::mutex> lock(g_mem_mu);
+            for (vc_ctx* c : g_ctxs)
+            {
+                trim(c->cache_dev, 0, 0, out[0]);
+                trim(c->cache_host, 1, 0, out[1]);
+            }
         }
-        e = raw_alloc(host, p, bytes);
+        free_all(0, out[0]);
+        free_all(1, out[1]);
+        b->bytes = bytes;
+        b->home = nullptr;
+        e = raw_alloc(host, &b->p, bytes);
         if (e != hipSuccess)
         {
-            *p = nullptr;
+            delete b;
             (void)hipGetLastError();
             return vc_fail(ctx, VC_ERR_NOMEM, "%s(%zu bytes) failed: %s",
                            host ? "hipHostMalloc" : "hipMalloc", bytes, hipGetErrorString(e));
         }
-        g_live[host][*p] = live_block{nullptr, bytes};
-        return VC_OK;
     }
-    g_live[host][*p] = live_block{kept ? ctx : nullptr, want};
+    try
+    {
+        std::lock_guard<std::mutex> lock(g_mem_mu);
+        if (b->home)
+            g_ctxs.insert(ctx);
+        g_blocks[host].emplace(b->p, b);
+    }
+    catch (const std::bad_alloc&)
+    {
+        raw_free(host, b->p);
+        delete b;
+        return vc_fail(ctx, VC_ERR_NOMEM, "no host memory for an allocation's record");
+    }
+    *p = b->p;
     return VC_OK;
 }
 
@@ -141,22 +199,33 @@ void mem_free(int host, void* p)
 {
     if (!p)
         return;
-    std::lock_guard<std::mutex> lock(g_mem_mu);
-    auto it = g_live[host].find(p);
-    if (it == g_live[host].end())
-        return;
-    const live_block b = it->second;
-    g_live[host].erase(it);
-    if (!b.ctx)
+    std::list<vc_block*> out;
     {
-        raw_free(host, p);
-        return;
+        std::lock_guard<std::mutex> lock(g_mem_mu);
+        auto it = g_blocks[host].find(p);
+        if (it == g_blocks[host].end() || it->second->kept)
+            return;
+        vc_block* b = it->second;
+        if (!b->home)
+        {
+            g_blocks[host].erase(it);
+            out.splice(out.end(), b->node);
+        }
+        else
+        {
+            vc_cache& c = *b->home;
+            int cls;
+            size_class(b->bytes, cls);
+            b->at = b->node.begin();
+            b->fit_at = b->fit_node.begin();
+            c.order.splice(c.order.end(), b->node);
+            c.fit[cls].splice(c.fit[cls].end(), b->fit_node);
+            c.bytes += b->bytes;
+            b->kept = true;
+            trim(c, host, host ? kHostCap : kDevCap, out);
+        }
     }
-    vc_cache& c = cache_of(b.ctx, host);
-    c.order.push_back(vc_cache::block{p, b.bytes});
-    c.by_size.emplace(b.bytes, std::prev(c.order.end()));
-    c.bytes += b.bytes;
-    trim(c, host, host ? kHostCap : kDevCap);
+    free_all(host, out);
 }
 } // namespace
 
@@ -167,14 +236,19 @@ void vc_host_free(void* p) { mem_free(1, p); }
 
 void vc_cache_release(vc_ctx* ctx)
 {
-    std::lock_guard<std::mutex> lock(g_mem_mu);
-    trim(ctx->cache_dev, 0, 0);
-    trim(ctx->cache_host, 1, 0);
-    g_ctxs.erase(ctx);
-    for (int host = 0; host < 2; ++host)
-        for (auto& l : g_live[host])
-            if (l.second.ctx == ctx)
-                l.second.ctx = nullptr;
+    std::list<vc_block*> out[2];
+    {
+        std::lock_guard<std::mutex> lock(g_mem_mu);
+        trim(ctx->cache_dev, 0, 0, out[0]);
+        trim(ctx->cache_host, 1, 0, out[1]);
+        g_ctxs.erase(ctx);
+        for (int host = 0; host < 2; ++host)
+            for (auto& b : g_blocks[host])
+                if (b.second->home == &cache_of(ctx, host))
+                    b.second->home = nullptr;
+    }
+    free_all(0, out[0]);
+    free_all(1, out[1]);
 }
 
 int vc_ws_get(vc_ctx* ctx, int slot, size_t bytes, void** p)

@@ -34,18 +34,24 @@ enum vc_ws_slot
     VC_WS_SLOTS
 };
 
-// A context's freed memory, kept for its next allocations (vc_alloc,
-// vc_host_alloc): blocks in the order they were freed, oldest first, and by
-// size.  Guarded by one lock over all contexts.
+// Memory of a context (vc_alloc, vc_host_alloc), and what it freed and keeps for
+// its next allocations: the kept blocks in the order they were freed, oldest
+// first, and by size class.  A block's list nodes come with it, so that freeing
+// allocates nothing.  Guarded by one lock over all contexts (vc_core.hip).
+struct vc_cache;
+struct vc_block
+{
+    void* p = nullptr;
+    size_t bytes = 0;
+    vc_cache* home = nullptr; // null: its context is gone, or it is never kept
+    bool kept = false;
+    std::list<vc_block*> node, fit_node; // empty while the block is kept
+    std::list<vc_block*>::iterator at, fit_at;
+};
+constexpr int VC_SIZE_CLASSES = 176; // up to 2 GiB
 struct vc_cache
 {
-    struct block
-    {
-        void* p;
-        size_t bytes;
-    };
-    std::list<block> order;
-    std::multimap<size_t, std::list<block>::iterator> by_size;
+    std::list<vc_block*> order, fit[VC_SIZE_CLASSES];
     size_t bytes = 0;
 };
 
