@@ -84,6 +84,16 @@ int vc_last_error(const vc_ctx* ctx, char* buf, size_t n);
 /* the hipStream_t every entry point of this context is enqueued on */
 int vc_ctx_stream(vc_ctx* ctx, void** hip_stream);
 int vc_ctx_synchronize(vc_ctx* ctx);
+/* Memory that a context's calls free (a released volume's buffers among it)
+ * stays with the context for its next allocations: at most 8 GiB of device and
+ * 64 MiB of pinned host memory, the oldest blocks beyond that and blocks above
+ * 2 GiB and 16 MiB go back at once.  It is given back when the context is
+ * destroyed, when an allocation of this library fails (every context's then,
+ * before the allocation is tried again), and by this call: that of ctx, or of
+ * every context of the process when ctx is NULL.  Programs whose other
+ * allocators share the GPU call it when those run out.  Waits for the device if
+ * there is something to give back. */
+int vc_ctx_trim(vc_ctx* ctx);
 /* copy of the device simple-point table: 2^21 uint32 words, bit b of word w
  * is the simple flag of neighbourhood code (w << 5) | b (waits) */
 int vc_simple_table_host(vc_ctx* ctx, uint32_t* words_out);

@@ -107,3 +107,76 @@ def test_allocations_go_on_while_another_context_frees(fake):
     b.join()
     assert not waited and F.fake_allocs() == n
     """)
+
+
+def test_kept_memory_is_bounded_and_given_back(fake):
+    """What released volumes leave behind: at most 8 GiB, the oldest blocks gone
+    first, none above 2 GiB, all of it back on vc_ctx_trim (one context's or every
+    context's), when an allocation would fail (the library's own or a
+    DeviceBuffer's), and at the context's end; counted by the runtime."""
+    fake("""
+    GB = 1 << 30
+    other = V.Context(0)
+    vc.trim(); other.trim()
+    base = F.fake_used(0)
+
+    def run(c, shape):
+        v = c.from_device(4096, shape).edt()
+        v.release()
+    # 900 MB of occupancy: 3.6 GB buffers go back at once, the small ones stay
+    run(vc, (1000, 1000, 900))
+    kept = F.fake_used(0) - base
+    assert 0.9 * GB < kept + GB // 8 and kept < 5 * GB, kept
+    vc.trim()
+    assert F.fake_used(0) == base
+    # 240 MB volumes of growing size classes (960 MB buffers): the cap holds
+    for n in range(240, 470, 16):
+        run(vc, (1000, 1000, n))
+        assert F.fake_used(0) - base <= 8 * GB, n
+    assert F.fake_used(0) - base > 6 * GB
+    # the newest volume's blocks are still there: nothing is allocated for it
+    a = F.fake_allocs()
+    run(vc, (1000, 1000, n))
+    assert F.fake_allocs() == a
+    # one context's memory, then every context's
+    run(other, (100, 100, 100))
+    mine = F.fake_used(0)
+    vc.trim()
+    assert base < F.fake_used(0) < mine and F.fake_used(0) - base < GB
+    run(vc, (300, 300, 300))
+    L.vc_ctx_trim(None)
+    assert F.fake_used(0) == base
+    # an allocation that would fail takes back what every context keeps
+    run(vc, (500, 500, 500)); run(other, (500, 500, 500))
+    assert F.fake_used(0) - base > 2 * GB
+    F.fake_limit(base + 2 * GB)
+    v = vc.from_device(4096, (400, 400, 400)).edt()
+    F.fake_limit((1 << 63) - 1)
+    v.release()
+    run(other, (500, 500, 500))
+    F.hipMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t]
+    F.hipFree.argtypes = [ctypes.c_void_p]
+    V._hip = type("Runtime", (), {"h": F})()
+    F.fake_limit(base + 2 * GB)
+    b = V.DeviceBuffer(2 * GB - 4096)
+    assert F.fake_used(0) == base + b.nbytes
+    try:
+        vc.from_device(4096, (500, 500, 500))
+        raise SystemExit("allocated beyond the limit")
+    except V.VcError as e:
+        assert e.code == V.VC_ERR_NOMEM
+    b.free()
+    F.fake_limit((1 << 63) - 1)
+    # pinned memory, and the end of a context with and without live volumes
+    third = V.Context(0)
+    at = F.fake_used(0), F.fake_used(1)
+    live = third.from_device(4096, (64, 64, 64)).edt()
+    run(third, (64, 64, 64))
+    assert F.fake_used(0) > at[0] and F.fake_used(1) > at[1]
+    run(third, (64, 64, 64))
+    live.release()
+    third.close()
+    other.close()
+    vc.close()
+    assert F.fake_used(0) == 0 and F.fake_used(1) == 0, (F.fake_used(0), F.fake_used(1))
+    """)

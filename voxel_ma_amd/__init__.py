@@ -31,7 +31,7 @@ _BUF_DTYPE = {BUF_OCC: np.uint8, BUF_EDT: np.int32, BUF_FT: np.int32,
 # every symbol declared in include/vc_api.h
 EXPORTS = [
     "vc_ctx_create", "vc_ctx_destroy", "vc_last_error", "vc_ctx_stream",
-    "vc_ctx_synchronize", "vc_simple_table_host", "vc_thin_timing",
+    "vc_ctx_synchronize", "vc_ctx_trim", "vc_simple_table_host", "vc_thin_timing",
     "vc_thin_timing_read", "vc_volume_upload",
     "vc_volume_from_device", "vc_volume_release", "vc_volume_dims", "vc_edt",
     "vc_measure", "vc_set_measure_f32", "vc_thin_levels", "vc_boundary_extract",
@@ -163,6 +163,7 @@ def library():
         "vc_last_error": [P, ctypes.c_char_p, ctypes.c_size_t],
         "vc_ctx_stream": [P, PP],
         "vc_ctx_synchronize": [P],
+        "vc_ctx_trim": [P],
         "vc_simple_table_host": [P, P],
         "vc_thin_timing": [P, I],
         "vc_thin_timing_read": [P, ctypes.POINTER(ctypes.c_int64),
@@ -313,6 +314,10 @@ class DeviceBuffer:
         self.nbytes = int(nbytes)
         p = ctypes.c_void_p()
         rc = hip().hipMalloc(ctypes.byref(p), max(self.nbytes, 1))
+        if rc != 0:  # memory that contexts only keep goes back first
+            library().vc_ctx_trim(None)
+            hip().hipGetLastError()
+            rc = hip().hipMalloc(ctypes.byref(p), max(self.nbytes, 1))
         if rc != 0:
             raise VcError(VC_ERR_NOMEM, "hipMalloc(%d) failed (%d)" % (self.nbytes, rc))
         self.ptr = p.value
@@ -380,6 +385,11 @@ class Context:
 
     def synchronize(self):
         self.check(self._lib.vc_ctx_synchronize(self.handle))
+
+    def trim(self):
+        """Give back the memory that this context's calls freed and that it keeps
+        for its next allocations (vc_ctx_trim)."""
+        self.check(self._lib.vc_ctx_trim(self.handle))
 
     def thin_timing(self, enable):
         """Bracket every tile-sweep launch of this context with HIP events

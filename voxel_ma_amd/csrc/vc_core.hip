@@ -30,7 +30,8 @@ int vc_fail(vc_ctx* ctx, int code, const char* fmt, ...)
 // the complex of a 96^3 volume makes about 300 of them, a volume made and
 // released per call about 25.  So what a context frees is kept, up to kDevCap
 // and kHostCap bytes (the oldest blocks go first), and given back when the
-// context is destroyed or when an allocation made here would fail: the 96^3 complex
+// context is destroyed, by vc_ctx_trim, or when vc_alloc or vc_host_alloc would
+// fail (direct runtime calls and other allocators call vc_ctx_trim): the 96^3 complex
 // 36.7 -> 14.2 ms, a 96 x 81 x 107 volume's skeleton from host to host bytes 1.26
 // -> 0.96 ms, the boundary mesh of a new 256^3 volume 2.81 -> 2.53 ms.
 namespace
@@ -156,17 +157,7 @@ int mem_alloc(vc_ctx* ctx, int host, void** p, size_t bytes)
     {
         // memory that is only kept goes back first
         (void)hipGetLastError();
-        std::list<vc_block*> out[2];
-        {
-            std::lock_guard<std::mutex> lock(g_mem_mu);
-            for (vc_ctx* c : g_ctxs)
-            {
-                trim(c->cache_dev, 0, 0, out[0]);
-                trim(c->cache_host, 1, 0, out[1]);
-            }
-        }
-        free_all(0, out[0]);
-        free_all(1, out[1]);
+        vc_ctx_trim(nullptr);
         b->bytes = bytes;
         b->home = nullptr;
         e = raw_alloc(host, &b->p, bytes);
@@ -432,6 +423,23 @@ int vc_ctx_synchronize(vc_ctx* ctx)
     if (!ctx)
         return VC_ERR_INVALID;
     VC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return VC_OK;
+}
+
+int vc_ctx_trim(vc_ctx* ctx)
+{
+    std::list<vc_block*> out[2];
+    {
+        std::lock_guard<std::mutex> lock(g_mem_mu);
+        for (vc_ctx* c : g_ctxs)
+            if (!ctx || c == ctx)
+            {
+                trim(c->cache_dev, 0, 0, out[0]);
+                trim(c->cache_host, 1, 0, out[1]);
+            }
+    }
+    free_all(0, out[0]);
+    free_all(1, out[1]);
     return VC_OK;
 }
 

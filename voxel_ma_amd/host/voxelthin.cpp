@@ -45,7 +45,15 @@ void VoxelThinning::assignMeasure(const std::vector<float>& m)
     // stage through the device: vc_set_measure_f32 takes device memory
     vc_ctx* c = vcdev::context();
     float* d = nullptr;
-    if (hipMalloc(&d, N * sizeof(float)) != hipSuccess)
+    hipError_t e = hipMalloc(&d, N * sizeof(float));
+    if (e != hipSuccess)
+    {
+        // memory that contexts only keep goes back first
+        (void)hipGetLastError();
+        vc_ctx_trim(nullptr);
+        e = hipMalloc(&d, N * sizeof(float));
+    }
+    if (e != hipSuccess)
         throw std::runtime_error("hipMalloc for the measure failed");
     int rc = hipMemcpy(d, m.data(), N * sizeof(float), hipMemcpyHostToDevice) ==
                      hipSuccess
