@@ -180,3 +180,16 @@ def test_kept_memory_is_bounded_and_given_back(fake):
     vc.close()
     assert F.fake_used(0) == 0 and F.fake_used(1) == 0, (F.fake_used(0), F.fake_used(1))
     """)
+
+
+def test_noalloc_call_drains_after_an_error(fake):
+    """vc_skeleton_noalloc's scratch array is the device's: a call that fails (no
+    sweep reports here, since no kernel runs) returns with nothing in flight, as
+    one that succeeds does."""
+    fake("""
+    lv = np.array([1.0, 2.0], np.float32)
+    rc = L.vc_skeleton_noalloc(vc.handle, ctypes.c_void_p(4096), 20, 30, 40, P(lv), 2,
+                               ctypes.c_void_p(8192), None)
+    assert rc == V.VC_ERR_HIP and "report" in vc.last_error(), (rc, vc.last_error())
+    assert F.fake_launches() > 3 and F.fake_unwaited() == 0
+    """)

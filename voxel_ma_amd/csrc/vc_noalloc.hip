@@ -282,8 +282,10 @@ extern "C" int vc_skeleton_noalloc(vc_ctx* ctx, const uint8_t* d_occ, int nx,
     if (rc == VC_OK)
         rc = vc_thin_sched(ctx, s, levels, n_levels, stats);
     // the caller's label array is complete for every stream and the host, and
-    // the scratch array idle, when the call returns
-    if (rc == VC_OK)
-        VC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    // the scratch array, which every context of the device shares, idle when the
+    // call returns, also after an error
+    const hipError_t e = hipStreamSynchronize(ctx->stream);
+    if (rc == VC_OK && e != hipSuccess)
+        rc = vc_fail(ctx, VC_ERR_HIP, "vc_skeleton_noalloc: %s", hipGetErrorString(e));
     return rc;
 }
