@@ -193,3 +193,41 @@ def test_noalloc_call_drains_after_an_error(fake):
     assert rc == V.VC_ERR_HIP and "report" in vc.last_error(), (rc, vc.last_error())
     assert F.fake_launches() > 3 and F.fake_unwaited() == 0
     """)
+
+
+def test_null_stream_copies_wait_for_the_context_stream(fake):
+    """The context's stream does not order itself with the null stream, so a copy on
+    the null stream comes after a wait for every kernel before it."""
+    fake("""
+    def ok(what):
+        assert F.fake_racing() == b"", (what, F.fake_racing())
+    occ = np.ones((40, 33, 70), np.uint8)
+    vol = vc.upload(occ)
+    vol.edt().measure()
+    vol.boundary()
+    ok("volume")
+    for _ in range(2):
+        V.Batch(vc, [vol, vc.upload(occ)]).edt().measure()
+    ok("batch")
+    nv, ne, nf = 8, 5, 2
+    vts, edges = np.zeros((nv, 3), np.float32), np.zeros((ne, 2), np.int32)
+    fo, fv = np.array([0, 4, 8], np.int64), np.zeros(8, np.int32)
+    veo, ve = np.zeros(nv + 1, np.int64), np.zeros(1, np.int32)
+    val = np.ones(nv, np.uint8)
+    i32 = lambda n: P(np.zeros(n, np.int32))
+    n1, n2, on = ctypes.c_int(), ctypes.c_int64(), ctypes.c_int()
+    out = [np.zeros(32, np.int64) for _ in range(8)]
+    rc = L.vc_voro_merge_close_device(
+        vc.handle, nv, ne, nf, P(vts), P(edges), P(fo), P(fv), P(veo), P(ve), P(val),
+        ctypes.c_float(0.1), 0, P(out[0]), P(out[1]), ctypes.byref(n1), P(out[2]), P(out[3]),
+        P(out[4]), P(out[5]), ctypes.c_int64(16), ctypes.byref(n2), P(out[6]), ctypes.byref(on))
+    assert rc == V.VC_OK and on.value == 1
+    ok("merge")
+    net = V.Surrogate(vc, seed=1)
+    net.set_params(net.params())
+    net.infer(vol)
+    net.set_params(net.params())
+    ok("surrogate")
+    d = V.VoroDiagram(vol)
+    ok("diagram")
+    """)

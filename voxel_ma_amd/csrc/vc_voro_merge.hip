@@ -328,11 +328,14 @@ int vc_voro_merge_dev(vc_ctx* ctx, int32_t nv, int32_t ne, int32_t nf, const flo
         gather_keys<<<nblk((int64_t)NK), kB, 0, S>>>((int64_t)NK, key, kflag, kin);
     hip(hipGetLastError());
     uint32_t cnt[3] = {0, 0, 0}; // new vertices, kept faces, keys
-    hip(hipMemcpy(&cnt[0], vflag + nv, 4, hipMemcpyDeviceToHost));
-    hip(hipMemcpy(&cnt[1], out->fpos + nf, 4, hipMemcpyDeviceToHost));
-    hip(hipMemcpy(&cnt[2], kflag + NK, 4, hipMemcpyDeviceToHost));
+    // on the stream: face_write, which writes nfo, is not waited for above
+    hip(hipMemcpyAsync(&cnt[0], vflag + nv, 4, hipMemcpyDeviceToHost, S));
+    hip(hipMemcpyAsync(&cnt[1], out->fpos + nf, 4, hipMemcpyDeviceToHost, S));
+    hip(hipMemcpyAsync(&cnt[2], kflag + NK, 4, hipMemcpyDeviceToHost, S));
+    hip(hipStreamSynchronize(S));
     int64_t nfv_new = 0;
-    hip(hipMemcpy(&nfv_new, out->nfo + cnt[1], 8, hipMemcpyDeviceToHost));
+    hip(hipMemcpyAsync(&nfv_new, out->nfo + cnt[1], 8, hipMemcpyDeviceToHost, S));
+    hip(hipStreamSynchronize(S));
     if (e != hipSuccess)
         return fail(vc_fail(ctx, VC_ERR_HIP, "merge: %s", hipGetErrorString(e)));
     const int64_t nk = cnt[2];
