@@ -259,7 +259,7 @@ struct vc_sched
     int n = 0;
     std::vector<vc_vol*> vols;
     std::vector<vc_vdesc> h_desc;
-    vc_vdesc* d_desc = nullptr;
+    vc_vdesc* d_desc = nullptr;  // views of a batch (one volume: vc_work::one)
     vc_vdesc* h_stage = nullptr; // pinned staging of h_desc
     uint64_t* d_items[VK_COUNT] = {};
     uint32_t total[VK_COUNT] = {};

@@ -2,9 +2,8 @@
 // volume held in caller device memory, with no device allocation.
 //
 // Every intermediate of the path (squared EDT, feature transform, lambda^2,
-// level bytes, the thinning bit planes, revisit flags, tile neighbour masks,
-// the per-volume view and the thinning control words) lives in one
-// file-scope device array, `scratch`, of VC_NOALLOC_SCRATCH_BYTES.  Each GPU
+// level bytes, the thinning bit planes, revisit flags, tile neighbour masks
+// and the thinning control words) lives in one file-scope device array, `scratch`, of VC_NOALLOC_SCRATCH_BYTES.  Each GPU
 // the library runs on holds its own copy at its own address until the
 // process ends; the address is taken once per device with
 // hipGetSymbolAddress at context creation and passed to the kernels as an
@@ -15,9 +14,9 @@
 // reading it (the level set-up clears the control words and rings and
 // writes the planes, the tile-sweep entry writes the neighbour masks, the
 // statistics counters are cleared at the start of the thinning), and the
-// level thresholds and the view are uploaded on every call.  Calls that
-// overlap on one device (two host threads, two contexts of one device)
-// race on the array.
+// level thresholds are uploaded on every call (the kernels take the volume's
+// view as an argument).  Calls that overlap on one device (two host threads, two
+// contexts of one device) race on the array.
 //
 // The host side of the call reuses a volume record and a one-volume schedule
 // built, with their pinned staging buffers, by vc_ctx_create; the call
@@ -52,7 +51,7 @@ int bits_for(int n)
 struct Layout
 {
     size_t edt, ft, lam2, lvl, alive, elig, dflag, alive2, tchg, eflag;
-    size_t desc, T, L, ctl, gany, vany, ctr, end;
+    size_t T, L, ctl, gany, vany, ctr, end;
 };
 
 Layout layout(int nx, int ny, int nz)
@@ -77,7 +76,6 @@ Layout layout(int nx, int ny, int nz)
     take(l.alive2, 8 * words);
     take(l.tchg, 2 * 4 * tiles);
     take(l.eflag, (size_t)nz * ((size_t)nx + ny));
-    take(l.desc, sizeof(vc_vdesc));
     take(l.T, 8 * (size_t)VC_MAX_LEVELS);
     take(l.L, 4 * (size_t)VC_MAX_LEVELS);
     take(l.ctl, 4 * 64);
@@ -130,9 +128,7 @@ int vc_noalloc_setup(vc_ctx* ctx)
     s->lv_cache.reserve(VC_MAX_LEVELS);
     ctx->na_vol = v;
     ctx->na_sched = s;
-    if (hipHostMalloc((void**)&s->h_stage, sizeof(vc_vdesc),
-                      hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc(&s->h_lv, 12 * (size_t)VC_MAX_LEVELS,
+    if (hipHostMalloc(&s->h_lv, 12 * (size_t)VC_MAX_LEVELS,
                       hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void**)&s->h_ring, 4 * VC_RING, hipHostMallocDefault) !=
             hipSuccess ||
@@ -151,8 +147,6 @@ void vc_noalloc_teardown(vc_ctx* ctx)
     vc_sched* s = ctx->na_sched;
     if (s)
     {
-        if (s->h_stage)
-            (void)hipHostFree(s->h_stage);
         if (s->h_lv)
             (void)hipHostFree(s->h_lv);
         if (s->h_ring)
@@ -257,19 +251,17 @@ extern "C" int vc_skeleton_noalloc(vc_ctx* ctx, const uint8_t* d_occ, int nx,
     d.nty = (ny + 31) / 32;
     s->voxels = N;
     s->words = (int64_t)words;
-    s->d_desc = reinterpret_cast<vc_vdesc*>(base + L.desc);
     s->d_T = reinterpret_cast<uint64_t*>(base + L.T);
     s->d_L = reinterpret_cast<float*>(base + L.L);
     s->d_ctl = reinterpret_cast<uint32_t*>(base + L.ctl);
     s->d_gany = reinterpret_cast<uint32_t*>(base + L.gany);
     s->d_vany = reinterpret_cast<uint32_t*>(base + L.vany);
     s->d_ctr = reinterpret_cast<unsigned long long*>(base + L.ctr);
-    // thresholds and view are uploaded on every call: another context of
-    // this device may have used the array since
+    // the thresholds are uploaded on every call: another context of this
+    // device may have used the array since
     s->lv_cache.clear();
     s->lv_n = 0;
-    // one volume: no work tables, so this allocates nothing; it uploads the
-    // view into the scratch array
+    // one volume: no work tables, so this allocates and uploads nothing
     rc = vc_sched_apply(ctx, s, vc_schedule_default());
     // the EDT's thick-tile flags start cleared (the array may hold another
     // call's data there; a stale flag would cost time only)

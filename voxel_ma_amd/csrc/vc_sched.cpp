@@ -289,7 +289,7 @@ int vc_sched_build(vc_ctx* ctx, vc_vol* const* vols, int n,
         s->voxels += v->N;
         s->words += (int64_t)words;
     }
-    if (rc == VC_OK)
+    if (rc == VC_OK && n > 1)
         rc = vc_alloc(ctx, (void**)&s->d_desc, sizeof(vc_vdesc) * n);
     if (rc == VC_OK)
         rc = vc_alloc(ctx, (void**)&s->d_T, 8 * (size_t)n * VC_MAX_LEVELS);
@@ -304,7 +304,7 @@ int vc_sched_build(vc_ctx* ctx, vc_vol* const* vols, int n,
     if (rc == VC_OK)
         rc = vc_alloc(ctx, (void**)&s->d_ctr,
                       8 * (size_t)VC_CTR_SLOTS * VC_CTR_WORDS);
-    if (rc == VC_OK)
+    if (rc == VC_OK && n > 1)
         rc = vc_host_alloc(ctx, (void**)&s->h_stage, sizeof(vc_vdesc) * n);
     if (rc == VC_OK)
         rc = vc_host_alloc(ctx, &s->h_lv, 12 * (size_t)n * VC_MAX_LEVELS);

@@ -924,18 +924,6 @@ constexpr int kTQ = 1024;              // candidate queue entries per round
 static_assert(23 * 19 <= kTBlock, "a row per thread");
 __device__ __forceinline__ int fy_of(int p) { return (7 - p) >> 1; }
 
-// window of word (o, w): bits 62..63 of word w-1, word w, bits 0..1 of w+1
-__device__ __forceinline__ void load_win(const uint64_t* __restrict__ P,
-                                         int64_t o, int w, int nwz,
-                                         uint64_t& lo, uint32_t& hi)
-{
-    const uint64_t c = P[o];
-    const uint64_t p = w > 0 ? P[o - 1] : 0ull;
-    const uint64_t n = w + 1 < nwz ? P[o + 1] : 0ull;
-    lo = (p >> 62) | (c << 2);
-    hi = (uint32_t)(c >> 62) | ((uint32_t)(n & 3ull) << 2);
-}
-
 // a region row: window bits 0..63 and 64..67 (in LDS the low words and the
 // high nibbles live in separate arrays, which keeps the tile sweep at 37 KB)
 struct TRow
