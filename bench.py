@@ -72,16 +72,16 @@ TRAFFIC_SOURCE = ("profiles/traffic.json: rocprofv3 --pmc FETCH_SIZE and WRITE_S
 
 
 def measured_traffic(kernel, n):
-    """HBM bytes per dispatch of `kernel` from the committed rocprofv3
-    FETCH_SIZE / WRITE_SIZE summary (512^3 workload only), else None."""
+    """HBM bytes per dispatch of `kernel` (with its template arguments, as the
+    summary names it) from the committed rocprofv3 FETCH_SIZE / WRITE_SIZE
+    summary (512^3 workload only), else None."""
     path = os.path.join(ROOT, "profiles", "traffic.json")
     if n != 512 or not os.path.exists(path):
         return None
     with open(path) as f:
         t = json.load(f).get("traffic_bytes_per_dispatch", {})
-    # the summary names instances: thin_tile_sweep<false, false>
-    v = [b for k, b in t.items() if k.split("<")[0] == kernel]
-    return round(v[0]) if v else None
+    v = t.get(kernel)
+    return None if v is None else round(v)
 
 
 def _host_cpu():
@@ -898,7 +898,7 @@ def main():
         "roofline": {"bound": "hbm", "kernel": "thin_tile_sweep (8 subfield passes)",
                      "achieved": round(thin_gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(thin_gbs / HBM_PEAK_GBS, 4),
-                     "traffic": measured_traffic("thin_tile_sweep", n),
+                     "traffic": measured_traffic("thin_tile_sweep<false, false>", n),
                      "traffic_source": TRAFFIC_SOURCE,
                      "bytes_per_voxel_pass": round(THIN_BYTES_PER_VOXEL_PASS, 4),
                      "voxel_passes_per_step": int(stats.voxel_passes),
@@ -914,8 +914,9 @@ def main():
                          "peak": HBM_PEAK_GBS, "unit": "GB/s",
                          "frac": round(edt_gbs / HBM_PEAK_GBS, 4), "bytes_per_voxel": 21,
                          "traffic": sum(filter(None, (measured_traffic(k, n) for k in
-                                                      ("edt_pass_z", "edt_pass_y",
-                                                       "edt_pass_x")))) or None,
+                                                      ("edt_pass_z<false>",
+                                                       "edt_pass_y<false, true>",
+                                                       "edt_pass_x<false>")))) or None,
                          "traffic_source": TRAFFIC_SOURCE},
     }
     if not (a.no_surrogate or a.profile_steps):

@@ -154,7 +154,8 @@ int vc_thin_levels(vc_ctx* ctx, vc_vol* vol, const float* levels,
  * vc_batch_run issues on this context is bracketed by two HIP events on the
  * context stream (with use_graph, one pair per graph segment, which then also
  * holds the segment's entry and bookkeeping kernels); the elapsed times are
- * read at the host wait that ends each segment.  Enabling or disabling
+ * read when the call has waited for the launches, which it does while timing is
+ * enabled.  Enabling or disabling
  * resets the totals.  vc_thin_timing_read returns the launches timed and
  * their summed duration in milliseconds. */
 int vc_thin_timing(vc_ctx* ctx, int enable);

@@ -38,9 +38,9 @@ typedef struct vc_schedule {
                             checks: 0 = adaptive (4, 8, 12, then 16),
                             -1 = adaptive doubling (4, 8, then 16), or
                             1-32.  With 0 or -1, tile sweeps that run from
-                            a level's start outside a graph and untimed
-                            are launched ahead of their own reports and
-                            have no such checks                           */
+                            a level's start outside a graph are
+                            launched ahead of their own reports and have
+                            no such checks                                */
     int use_graph;       /* 1: each segment of sweeps is a captured
                             hipGraph replayed on the context stream       */
     int tail_sweep;      /* sweeps with index >= tail_sweep within a level

@@ -130,6 +130,34 @@ def test_thin_watched_levels(vc, oracle, case):
         vol.release()
 
 
+@pytest.mark.parametrize("nz", [40, 65, 90, 115, 140])
+def test_timed_sweeps_are_those_that_run(vc, nz):
+    """With timing on, a level runs as without: launched ahead of the sweeps' own
+    reports, with at most three sweeps past the last report (a bar loses two voxels
+    per end and sweep; segments between checks would launch up to 15 too many)."""
+    import voxel_ma_amd as V
+    occ = np.zeros((5, 6, nz), np.uint8)
+    occ[2, 3, 3:-3] = 1
+    vol = vc.upload(occ)
+    vol.edt().measure()
+    ref = vol.thin_levels([1e6])
+    lab = vol.get(V.BUF_LABEL)
+    say("timed sweeps", nz)
+    vc.thin_timing(True)
+    st = vol.thin_levels([1e6])
+    launches, ms = vc.thin_timing_read()
+    vol.thin_levels([1e6], stats=False)  # timed calls wait also without statistics
+    again, _ = vc.thin_timing_read()
+    vc.thin_timing(False)
+    sweeps = st.passes // 8
+    assert st.passes == ref.passes and st.tests == ref.tests
+    assert np.array_equal(vol.get(V.BUF_LABEL), lab)
+    assert st.launches == launches + 1 and ms > 0.0  # and the level's set-up
+    assert sweeps < launches <= sweeps + 3, (sweeps, launches)
+    assert launches + sweeps < again <= launches + sweeps + 3
+    vol.release()
+
+
 @pytest.mark.parametrize("nz", [1, 2, 7, 8, 9, 15, 63, 64, 65, 71, 128, 131, 255, 257, 519])
 def test_row_lengths(vc, oracle, nz):
     """Rows of every alignment: the row pass of the EDT and the level set-ups

@@ -243,8 +243,7 @@ struct vc_work
 };
 
 // sweeps per segment when vc_schedule.sweeps_per_sync is 0 or -1 (adaptive)
-// and the convergence is checked by copying the ring (dense passes, graphs,
-// timed sweeps)
+// and the convergence is checked by copying the ring (dense passes, graphs)
 constexpr int VC_SEG_MIN = 4, VC_SEG_MAX = 16;
 // report words of a context (vc_ctx::h_prog)
 constexpr int VC_PROG = 8;

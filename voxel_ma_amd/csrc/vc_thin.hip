@@ -1629,6 +1629,10 @@ int run_level_watched(vc_ctx* ctx, vc_sched* s, int k, int64_t guard, int64_t* c
             if (launched > guard)
                 return vc_fail(ctx, VC_ERR_GUARD, "thinning did not converge in %lld sweeps",
                                (long long)launched);
+            hipEvent_t ev[2];
+            int rc = ev_begin(ctx, ev);
+            if (rc != VC_OK)
+                return rc;
             if (s->n > 1)
                 launch_tile_sweep<true>(ctx->stream, g, W, ctx->d_lut, (int)launched, k, s->n,
                                         nullptr, s, ctx->h_prog, epoch);
@@ -1636,6 +1640,8 @@ int run_level_watched(vc_ctx* ctx, vc_sched* s, int k, int64_t guard, int64_t* c
                 launch_tile_sweep<false>(ctx->stream, g, W, ctx->d_lut, (int)launched, k, s->n,
                                          nullptr, s, ctx->h_prog, epoch);
             VC_CHECK_LAUNCH(ctx);
+            if ((rc = ev_end(ctx, ev, 1)) != VC_OK)
+                return rc;
         }
         // until a new report; the stream is asked now and then, so that a
         // failed launch ends the wait (its status) and so does an idle stream
@@ -1790,7 +1796,7 @@ int vc_thin_sched(vc_ctx* ctx, vc_sched* s, const float* levels, int nlev,
         }
         // tile sweeps from a level's start, launched one by one
         if (sc.tile_sweep == 0 && s->total[VK_TT] != 0 && !sc.use_graph &&
-            sc.sweeps_per_sync <= 0 && !ctx->time_sweeps)
+            sc.sweeps_per_sync <= 0)
         {
             int64_t conv = 0;
             rc = run_level_watched(ctx, s, k, guard, &conv, &launches);
@@ -1853,6 +1859,13 @@ int vc_thin_sched(vc_ctx* ctx, vc_sched* s, const float* levels, int nlev,
             else if (sc.sweeps_per_sync < 0)
                 K = K * 2 < VC_SEG_MAX ? K * 2 : VC_SEG_MAX;
         }
+    }
+    // watched levels waited for no stream
+    if (!ctx->ev_open.empty())
+    {
+        VC_HIP(ctx, hipStreamSynchronize(S));
+        if ((rc = ev_collect(ctx)) != VC_OK)
+            return rc;
     }
     if (st)
     {
