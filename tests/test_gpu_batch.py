@@ -3,6 +3,8 @@ a batch gets exactly the oracle's EDT, FT, levels and labels (the same as
 the single-volume path), under every schedule, with captured graph segments
 replayed repeatedly; the device solids generator equals its host
 restatement byte for byte."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -120,7 +122,9 @@ def test_batch_every_schedule_same_result(vc, ragged, sched):
 def test_tile_sweep_few_and_many_tiles(vc, oracle, over):
     """Batches of exactly two tiles per CU and of more: the tile sweep has a form
     for either side.  Tiles of every cut (8 per volume, most of them partial)."""
-    cus = 256
+    n = ctypes.c_int()  # hipDeviceAttributeMultiprocessorCount
+    assert V.hip().hipDeviceGetAttribute(ctypes.byref(n), 63, 0) == 0
+    cus = n.value
     rng = np.random.default_rng(23)
     shapes = [(33, 34, 65), (47, 64, 128), (64, 33, 67)]  # 2 x 2 x 2 tiles
     vols = [(rng.random(s) < p).astype(np.uint8) for s, p in zip(shapes, (0.9, 0.97, 0.8))]
