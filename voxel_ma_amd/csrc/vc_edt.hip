@@ -45,8 +45,9 @@ constexpr int kInf = 0x7FFFFFFF;
 // The lines: divide and conquer costs about as much as searches of 40-50
 // distances throughout a tile.  One deep voxel does not make a tile slow, many
 // rows with them do, and the sampled rows tell the two apart: with kDeepY = 64
-// for every voxel, 13 % of the y-pass tiles of the 512^3 blurred-noise volume
-// were flagged and its EDT took 15 % longer; with 128 alone the tiles of a
+// for every voxel, 9 % of the y-pass tiles of the 512^3 blurred-noise volume
+// are flagged (the sampled rows flag 0.8 %, 128 none) and its EDT took 15 %
+// longer; with 128 alone the tiles of a
 // 512^3 ball of radius 250 that lie 64-128 deep were not (y pass 2.08 ms; 1.32
 // with the samples, the noise volume's EDT 1.25 and 1.23 ms).  Sampled at 32,
 // 48, 96: noise 1.44-1.62, 1.30-1.43, 1.23 ms, ball 2.53, 2.54, 2.90 ms against

@@ -3,11 +3,12 @@
 //
 // Every intermediate of the path (squared EDT, feature transform, lambda^2,
 // level bytes, the thinning bit planes, revisit flags, tile neighbour masks
-// and the thinning control words) lives in one file-scope device array, `scratch`, of VC_NOALLOC_SCRATCH_BYTES.  Each GPU
-// the library runs on holds its own copy at its own address until the
-// process ends; the address is taken once per device with
-// hipGetSymbolAddress at context creation and passed to the kernels as an
-// ordinary pointer (the array's name is only a host-side stand-in).
+// and the thinning control words) lives in one file-scope device array,
+// `scratch`, of VC_NOALLOC_SCRATCH_BYTES.  Each GPU the library runs on holds
+// its own copy at its own address until the process ends; the address is taken
+// once per device with hipGetSymbolAddress at context creation and passed to
+// the kernels as an ordinary pointer (the array's name is only a host-side
+// stand-in).
 //
 // Every call on a device shares that device's array and the array keeps the
 // last call's contents: the kernels initialise every word they read before

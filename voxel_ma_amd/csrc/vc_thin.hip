@@ -145,8 +145,8 @@ __device__ __forceinline__ int64_t widx(const Plane& P, int x, int y, int w)
 // mask bits shifted down, so every row length runs on vector accesses: byte
 // accesses for the lengths that are no multiple of 8, and a wavefront per row,
 // took 131 us for 301 x 222 x 437 voxels and 831 us for 64 volumes of edge
-// 32-192 (84 M voxels), 58 and 169 us now (512^3: 240 us either way).  Bound: memory (occupancy, the measure of inside
-// voxels, levels and labels).
+// 32-192 (84 M voxels), 58 and 169 us now (512^3: 240 us either way).  Bound:
+// memory (occupancy, the measure of inside voxels, levels and labels).
 template <bool kB>
 __global__ void __launch_bounds__(kBlock)
     thin_level_init(vc_work W, const uint64_t* __restrict__ Tq,
@@ -1206,7 +1206,7 @@ __global__ void __launch_bounds__(kTBlock, kFew ? kTWavesFew : kTWaves)
             const int nrx = (xhi - rx0 + 1) >> 1, nry = (yhi - ry0 + 1) >> 1;
             // q / nry for q < 512 as q * ceil(2^16 / nry) >> 16, nry = 19 - p / 2
             // (with the division 64 solids 0.5 %, 512^3 0.4 %, 64^3 2 % slower)
-            const uint32_t inv = (uint32_t)(0x10010F100E390D7Aull >> (16 * (p >> 1))) & 0xFFFFu;
+            const uint32_t inv = (uint32_t)(0x10000F100E390D7Aull >> (16 * (p >> 1))) & 0xFFFFu;
             // window bit parity = z parity (64w - 2 is even); bits
             // [kHZ - Fz, kHZ + 64 + Fz): low word from bit 1 or 2 up, high
             // bits 64..65 or 64..66
@@ -1610,8 +1610,9 @@ int run_segment(vc_ctx* ctx, vc_sched* s, int K, int64_t first, int k,
 // watches the word in which each sweep reports the one before it.  A sweep
 // launched past convergence visits nothing.  Segments of 4, 8, 12, 16 sweeps
 // with a copied ring between them left the GPU idle for 25-30 us per check
-// and launched up to 15 sweeps too many (3-6 us each): 64^3 in one call 573 ->
-// 483 us, 256^3 balls 2.35 -> 2.18 ms, 512^3 noise 6.89 -> 6.68 ms per pass.
+// and launched up to 15 sweeps too many (3-6 us each): 64^3 in one call 727 ->
+// 655 us, 256^3 balls 2.42 -> 2.27 ms, 512^3 noise 6.86 -> 6.60 ms per pass, 64
+// solids in a batch 5.67 -> 5.46 ms (one box, the trees before and after).
 // Ahead: 2, 3 and 4 in flight measured the same within 1 %, 6 up to 4 % slower
 // (a level ends with that many sweeps too many).
 constexpr int kAhead = 3;

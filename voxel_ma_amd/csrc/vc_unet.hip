@@ -1550,7 +1550,8 @@ __global__ void __launch_bounds__(kBlock)
     // wavefront and counter serialised millions of atomics on 3 addresses)
     __shared__ unsigned long long sh[2][kBlock / 64];
     // bound by the bytes read: 16 voxels per thread and access, the errors of a
-    // 16 without an inside voxel left out (512^3 noise: a voxel per thread and trip 310 us, this 185)
+    // 16 without an inside voxel left out (512^3 noise: a voxel per thread and
+    // trip 310 us, this 185)
     unsigned long long acc = 0, fb = 0;
     const int64_t n16 = N / 16, t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     for (int64_t i = t0; i < n16; i += (int64_t)gridDim.x * blockDim.x)
@@ -1624,7 +1625,8 @@ __global__ void __launch_bounds__(kBlock)
              float tau, int64_t N, float* __restrict__ meas)
 {
     // bound by the bytes moved: four voxels per thread and access, and of the two
-    // measures only what one of the four takes (512^3 noise: a voxel per thread 577 us, this 243)
+    // measures only what one of the four takes (512^3 noise: a voxel per thread
+    // 577 us, this 243)
     const int64_t i = 4 * ((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
     if (i >= N)
         return;
