@@ -1612,7 +1612,7 @@ int run_segment(vc_ctx* ctx, vc_sched* s, int K, int64_t first, int k,
 // with a copied ring between them left the GPU idle for 25-30 us per check
 // and launched up to 15 sweeps too many (3-6 us each): 64^3 in one call 727 ->
 // 655 us, 256^3 balls 2.42 -> 2.27 ms, 512^3 noise 6.86 -> 6.60 ms per pass, 64
-// solids in a batch 5.67 -> 5.46 ms (one box, the trees before and after).
+// solids in a batch 5.67 -> 5.46 ms (one card, the code before and after).
 // Ahead: 2, 3 and 4 in flight measured the same within 1 %, 6 up to 4 % slower
 // (a level ends with that many sweeps too many).
 constexpr int kAhead = 3;
